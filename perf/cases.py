@@ -341,3 +341,40 @@ def tolerance(case):
         # with float32 arithmetic: up to 4.5e-3 (the weight gradients)
         return {"rel": 1.5e-2}
     return "exact"
+
+
+def _stored_values(w, precision):
+    """What a bf16 weight reads back as after it was stored with `precision` mantissa bits (half-up
+    rounding of the magnitude, the carry running into the exponent)."""
+    if precision == 7:
+        return w
+    bits = w.view(torch.int16).to(torch.int32) & 0xFFFF
+    mag = ((bits & 0x7FFF) + (1 << (6 - precision))) & 0x7FFF & ~((1 << (7 - precision)) - 1)
+    bits = (bits & 0x8000) | mag
+    return torch.where(bits >= 0x8000, bits - 0x10000, bits).to(torch.int16).view(torch.bfloat16)
+
+
+def exact(case, seed):
+    """The outputs of `run` on the inputs of `prepare(case, seed)` in float64; None for the kinds
+    whose outputs are stored values and bytes."""
+    kind = case["kind"]
+    if kind not in ("block", "train"):
+        return None
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    model = (_Gated if kind == "block" else _Gpt2)(case, gen)
+    for m in model.modules():
+        if isinstance(m, torch.nn.Linear):
+            m.weight.data = _stored_values(m.weight.data, case["precision"])
+    model = model.double()
+    if kind == "block":
+        x = [_rows(case["tokens"], case["width"], gen).double() for _ in range(3)]
+        with torch.no_grad():
+            return model(*x)
+    x = _rows(case["tokens"], case["width"], gen).double().requires_grad_(True)
+    gy = (_rows(case["tokens"], case["width"], gen) * 1e-3).double()
+    y = model(x)
+    y.backward(gy)
+    weights = [model.qkv.weight, model.proj.weight, model.fc.weight, model.fc2.weight]
+    dense = [p.grad for p in model.parameters() if not any(p is w for w in weights)]
+    # the compressed weights' gradients come in the order of the backward pass
+    return [y.detach(), x.grad, *dense, *[w.grad for w in reversed(weights)]]
