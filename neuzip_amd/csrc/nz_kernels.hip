@@ -17,6 +17,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "nz_format.h"
 
 #ifndef NZ_HIST_COPIES
@@ -25,6 +27,8 @@
 #define NZ_HIST_STRIDE 257u
 #define NZ_RING_WORDS 1024u  // per-wave LDS ring of renormalisation words
 #define NZ_RING_DWORDS (NZ_RING_WORDS / 2)
+#define NZ_ONE_WORDS 512u    // the same with an 8-byte entry per word (NzWaveDecOne)
+#define NZ_ONE_BLOCK 256u    // words that ring is refilled by: the most four steps of a wavefront consume
 
 // ----------------------------------------------------------------------------
 // element-wise split / merge arithmetic
@@ -1491,7 +1495,7 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 // falls below 2^16 a 16-bit word taken at (words consumed so far by the wave +
 // rank of the lane among the lanes that need one).
 
-#define NZ_RING_ALLOC_DWORDS NZ_RING_DWORDS
+#define NZ_RING_ALLOC_DWORDS(one) ((one) ? 2 * NZ_ONE_WORDS : NZ_RING_DWORDS)
 // What the table parse leaves for the slot-table fill (runs, windows, flags)
 // lies in the last slots of the table itself; those are filled last, from
 // registers.
@@ -1499,7 +1503,10 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 #define NZ_TMETA_SLOT ((uint32_t)(NZ_M - 416))  /* first slot under it; a multiple of 32 */
 static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 32 == 0, "parse results fit under the tail");
 // dynamic LDS of a decode workgroup whose chunks have up to `spc` segments
-#define NZ_DEC_LDS_BYTES(spc) ((size_t)(2 * NZ_M + (spc) * NZ_RING_ALLOC_DWORDS) * 4)
+#define NZ_DEC_LDS_BYTES(spc, one) ((size_t)(2 * NZ_M + (spc) * NZ_RING_ALLOC_DWORDS(one)) * 4)
+// Launches of at most this many workgroups, one per compute unit and so at most
+// two wavefronts per SIMD, decode with NzWaveDecOne (whose figures stand there).
+#define NZ_ONE_READ_WORKGROUPS 256u
 
 // S+1 packed bytes of one 8-element group, as a little-endian integer
 template <int S>
@@ -1882,6 +1889,165 @@ struct NzWaveDec {
       base += (uint32_t)__popcll(m);
     }
   }
+  __device__ __forceinline__ void finish() {}  // the state is complete after every step
+};
+
+// Decoder state of one wavefront, for launches with few wavefronts per SIMD.
+//
+// What then bounds a step is its chain of dependent operations, not its instruction
+// count.  In the plain form the chain holds two LDS round trips: the
+// renormalisation word (its place depends on the ballot of the fresh states),
+// then the slot entry that the state with the word shifted in selects.  But a
+// state that takes a word w becomes x << 16 | w, so its slot is w & 4095, which
+// the word alone decides, and
+//   f * ((x << 16 | w) >> 12) + bias = f * (x << 4) + (f * (w >> 12) + bias).
+// The ring therefore holds, per word, the slot entry that the word selects with
+// f * (w >> 12) already added to the bias (it is below 16 f: 16 bits), and a
+// step is ONE read: from the ring at the lane's rank where the state fell below
+// 2^16, from the slot table otherwise, then one multiply-add.  A wavefront
+// makes the entries of 256 words at a time, four per lane, with independent
+// reads; a weight's exponents take one word per six symbols or so, so that is
+// one prepared entry for six chains of half the length.
+struct NzWaveDecOne {
+  const uint2* lut;
+  uint32_t* ring32;       // 512 entries: a window of the words
+  const uint8_t* words;   // start of the record (uniform); word indices count from here
+  uint32_t lim;           // largest byte offset from `words` that may be loaded: container end - 16 (uniform)
+  uint32_t lut_lds, ring_lds;  // LDS byte addresses (the same in all lanes, kept in vector registers)
+  uint32_t nwords;        // 16-bit units the record holds, table and states included
+  uint32_t lane;
+  uint32_t x;             // this lane's rANS state, before the word it may still have to take
+  uint32_t top;           // the state's upper bits, x << 4 with a word to take, x >> 12 without
+  uint32_t widx;          // index of that word
+  uint2 e;                // entry of the next step
+  uint32_t base;          // words consumed by the wave (the same in all lanes, kept in a vector register)
+  uint32_t filled;        // words entered into the ring (multiple of 4; uniform)
+  uint2 r;                // 4 words per lane fetched after the previous refill
+
+  // 16 (8) bytes of the word stream at dword index d.  Addresses are clamped to
+  // the container's closing padding, so every load is unconditional and in
+  // bounds; words past the record are never consumed by a valid stream.
+  __device__ __forceinline__ uint4 fetch(uint32_t d) const {
+    const uint32_t off = 4u * d < lim ? 4u * d : lim;
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(words + off);
+    return make_uint4(q[0], q[1], q[2], q[3]);
+  }
+  __device__ __forceinline__ uint2 fetch2(uint32_t d) const {
+    const uint32_t off = 4u * d < lim ? 4u * d : lim;
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(words + off);
+    return make_uint2(q[0], q[1]);
+  }
+
+  // record at comp + pos of a container of comp_bytes (pos + 16 <= comp_bytes)
+  __device__ __forceinline__ void attach(const uint8_t* comp, uint64_t comp_bytes, uint64_t pos, uint32_t* ring) {
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    ring32 = ring;
+    ring_lds = (uint32_t)(uintptr_t)((lds_u32*)ring);
+    lut_lds = (uint32_t)(uintptr_t)((lds_u32*)reinterpret_cast<const uint32_t*>(lut));
+    words = comp + pos;
+    const uint64_t room = comp_bytes - NZ_TAIL_PAD - pos;
+    lim = room < 0xFFFFFFF0ull ? (uint32_t)room : 0xFFFFFFF0u;
+  }
+
+  // Stage the first 512 dwords of the record (table of a chunk's first record,
+  // coder states, first words) where the ring will be.
+  __device__ __forceinline__ void stage() {
+    uint4 v[2];
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) v[q] = fetch(256 * q + 4 * lane);
+#pragma unroll
+    for (uint32_t q = 0; q < 2; ++q) *reinterpret_cast<uint4*>(ring32 + 256 * q + 4 * lane) = v[q];
+  }
+
+  // the entries of words first + 4 * lane ... + 3 (first a multiple of 4) into the ring
+  __device__ __forceinline__ void enter(uint32_t first, const uint2 v) {
+    const uint32_t w[4] = {v.x & 0xFFFFu, v.x >> 16, v.y & 0xFFFFu, v.y >> 16};
+    uint2 t[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t[k] = lut[w[k] & (NZ_M - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t[k].y += __umul24(t[k].x, w[k] >> NZ_PROB_BITS);
+    uint4* at = reinterpret_cast<uint4*>(ring32 + 2 * ((first + 4 * lane) & (NZ_ONE_WORDS - 1)));
+    at[0] = make_uint4(t[0].x, t[0].y, t[1].x, t[1].y);
+    at[1] = make_uint4(t[2].x, t[2].y, t[3].x, t[3].y);
+  }
+  __device__ __forceinline__ void lds_order() const {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  // Start decoding from state x0; the words begin `first_word` 16-bit units
+  // into the record (at most 348, so the first 512 from a multiple of 4 are staged).
+  __device__ __forceinline__ void start(uint32_t x0, uint32_t first_word) {
+    const uint32_t from = __builtin_amdgcn_readfirstlane(first_word) & ~3u;
+    filled = from + NZ_ONE_WORDS;
+    r = fetch2(filled / 2 + 2 * lane);  // the 256 words behind the ring's
+    const uint2 a = *reinterpret_cast<const uint2*>(ring32 + from / 2 + 2 * lane);
+    const uint2 b = *reinterpret_cast<const uint2*>(ring32 + from / 2 + NZ_ONE_BLOCK / 2 + 2 * lane);
+    lds_order();
+    enter(from, a);
+    enter(from + NZ_ONE_BLOCK, b);
+    lds_order();
+    x = x0;
+    top = x0 >> NZ_PROB_BITS;
+    widx = first_word;
+    e = lut[x0 & (NZ_M - 1)];
+    base = first_word;
+    // keep the per-lane constants in vector registers of their own
+    asm volatile("" : "+v"(lut_lds), "+v"(ring_lds), "+v"(base));
+  }
+
+  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7].
+  //
+  // Ring upkeep, before every four steps: they consume at most 4 * 64 = 256
+  // words.  The 256 words behind the ring's window wait in registers (`r`,
+  // fetched right after the previous refill); when no more than 256 are left
+  // ahead of `base` their entries are made and written, and the next 256 are
+  // fetched.  So at least 256 words are ahead of every four steps, the window
+  // [base, filled) never exceeds the ring's 512, and for exponent data a fetch
+  // has some three groups to arrive.
+  //
+  // [base - 64, base) may just have been read when a refill writes over it: LDS
+  // operations of a wavefront run in order, and the fences keep them so.
+  __device__ __forceinline__ void group(uint32_t (&ew)[8]) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) const u32x2 lds_cu64;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if ((j & 3) == 0) {
+        const uint32_t used = __builtin_amdgcn_readfirstlane(base);
+        if (filled - used <= NZ_ONE_BLOCK) {
+          lds_order();  // entries of words already taken are written over
+          enter(filled, r);
+          filled += NZ_ONE_BLOCK;
+          lds_order();
+          r = fetch2(filled / 2 + 2 * lane);
+        }
+      }
+      x = __umul24(e.x, top) + e.y;
+      ew[j] = e.x;
+      const bool need = x < NZ_L;
+      const uint64_t m = __ballot(need);
+      widx = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
+      uint32_t rw = widx & (NZ_ONE_WORDS - 1), sl = x & (NZ_M - 1);
+      asm volatile("" : "+v"(rw), "+v"(sl));  // mask, then one shift-add (not shift, mask, add)
+      const uint32_t at_ring = (rw << 3) + ring_lds, at_lut = (sl << 3) + lut_lds;
+      const uint32_t at = need ? at_ring : at_lut;
+      const u32x2 v = *(lds_cu64*)(uintptr_t)at;
+      e = make_uint2(v.x, v.y);
+      top = need ? x << 4 : x >> NZ_PROB_BITS;
+      base += (uint32_t)__popcll(m);
+    }
+  }
+
+  // The state after the last step, with the word it took: the ring does not
+  // hold the words themselves, so that one comes from the record again.
+  __device__ __forceinline__ void finish() {
+    if (x < NZ_L) {
+      const uint32_t off = 2u * widx < lim ? 2u * widx : lim;
+      x = (x << 16) | *reinterpret_cast<const uint16_t*>(words + off);
+    }
+  }
 };
 
 // One workgroup decodes chunk `c` of one tensor; wavefront k of the workgroup
@@ -1893,7 +2059,7 @@ struct NzWaveDec {
 // ragged and no group straddles two rows).
 // With NORM every merged value is multiplied by its group's factor (`nm`)
 // before it is stored or used.
-template <int S, int GEMV, bool NORM, bool STREAM>
+template <int S, int GEMV, bool NORM, bool STREAM, bool ONE>
 __device__ __forceinline__ void nz_decode_chunk(
     const uint8_t* __restrict__ comp, const uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
@@ -1962,9 +2128,9 @@ __device__ __forceinline__ void nz_decode_chunk(
   const uint32_t whole = seg_n / NZ_GROUP_SYMS < body ? seg_n / NZ_GROUP_SYMS : body;
   const uint32_t lane_off = lane * (S + 1);
   const uint32_t last_off = whole ? (whole - 1) * NZ_LANES * (S + 1) + lane_off : 0u;
-  NzWaveDec w;
+  std::conditional_t<ONE, NzWaveDecOne, NzWaveDec> w;
   w.lut = lut;
-  w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + wk * NZ_RING_ALLOC_DWORDS);
+  w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + wk * NZ_RING_ALLOC_DWORDS(ONE));
   w.nwords = rec_all / 2;
   w.lane = lane;
   w.filled = 0;
@@ -2274,6 +2440,7 @@ __device__ __forceinline__ void nz_decode_chunk(
 
   // every lane must be back at the encoder's start state (2^16 | carried bits)
   // and the wave must not have read past its record
+  w.finish();
   const bool bad = (carry ? (w.x >> 16) != 1u : w.x != NZ_L) || (w.base > w.nwords);
   if (__ballot(bad) != 0 && lane == 0) atomicOr(d_status, 4u);
 
@@ -2300,11 +2467,11 @@ __device__ __forceinline__ void nz_decode_chunk(
     if (walk.pending) walk.flush(lane);
 }
 
-template <int S, bool NORM, bool STREAM>
+template <int S, bool NORM, bool STREAM, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_kernel(
     const uint8_t* __restrict__ comp, uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm) {
-  nz_decode_chunk<S, 0, NORM, STREAM>(comp, comp_bytes, packed, out, g, d_status, blockIdx.x, NzGemv{}, nm);
+  nz_decode_chunk<S, 0, NORM, STREAM, ONE>(comp, comp_bytes, packed, out, g, d_status, blockIdx.x, NzGemv{}, nm);
 }
 
 // Several tensors in one launch: the grid is the concatenation of their
@@ -2333,7 +2500,7 @@ struct NzBatch {
   NzBatchItem item[NZ_BATCH_MAX];
 };
 
-template <int S, bool NORM, bool STREAM>
+template <int S, bool NORM, bool STREAM, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
   uint32_t t = 0, first = 0;
@@ -2342,13 +2509,13 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_ke
     ++t;
   }
   const NzBatchItem& it = b.item[t];
-  nz_decode_chunk<S, 0, NORM, STREAM>(it.comp, it.comp_bytes, it.packed, it.out, it.g, d_status,
+  nz_decode_chunk<S, 0, NORM, STREAM, ONE>(it.comp, it.comp_bytes, it.packed, it.out, it.g, d_status,
                                           blockIdx.x - first, NzGemv{}, NzNorm{it.norm, b.log2n});
 }
 
 // The same walk over several matrices that multiply one activation row, or up
 // to MR of them (each decoded weight is then used MR times before it is dropped).
-template <int S, bool NORM, int MR>
+template <int S, bool NORM, int MR, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
   uint32_t t = 0, first = 0;
@@ -2358,7 +2525,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_ker
   }
   const NzBatchItem& it = b.item[t];
   const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features, b.x_rows};
-  nz_decode_chunk<S, MR, NORM, false>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
+  nz_decode_chunk<S, MR, NORM, false, ONE>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
                                         blockIdx.x - first, gv, NzNorm{it.norm, b.log2n});
 }
 
@@ -2369,7 +2536,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_ker
 // kernel then lifts the row out of its slots.  An index outside the table sets
 // status bit 8 and yields a row of zeros.
 // ----------------------------------------------------------------------------
-template <int S, bool NORM>
+template <int S, bool NORM, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_rows_kernel(
     const uint8_t* __restrict__ comp, uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ scratch, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm,
@@ -2387,7 +2554,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_rows_ker
   // that the chunk's first element lands at the start of this workgroup's slot
   uint16_t* out = scratch + ((int64_t)blockIdx.x - (int64_t)c) * (int64_t)g.chunk_syms;
   // (the slots are read back by the copy kernel right away: ordinary stores)
-  nz_decode_chunk<S, 0, NORM, false>(comp, comp_bytes, packed, out, g, d_status, c, NzGemv{}, nm);
+  nz_decode_chunk<S, 0, NORM, false, ONE>(comp, comp_bytes, packed, out, g, d_status, c, NzGemv{}, nm);
 }
 
 #ifndef NZ_TEMPLATES_ONLY

@@ -36,17 +36,20 @@ void nz_launch_encode(const NzEncBatch& b, int cls, dim3 grid, dim3 block, uint3
 template <int S>
 void nz_launch_decode(const NzGeom& g, const void* comp, uint64_t comp_bytes, const void* packed, void* out,
                       uint32_t* d_status, const NzNorm& nm, uint32_t stream_out, hipStream_t st) {
-  const size_t lds = NZ_DEC_LDS_BYTES(g.spc);
+  const bool one = !stream_out && g.n_chunks <= NZ_ONE_READ_WORKGROUPS;
+  const size_t lds = NZ_DEC_LDS_BYTES(g.spc, one);
   const dim3 gd((uint32_t)g.n_chunks), bd(64 * g.spc);
-#define NZ_DEC_LAUNCH(NORM, STREAM)                                                                            \
-  hipLaunchKernelGGL((nz_decode_kernel<S, NORM, STREAM>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes, \
+#define NZ_DEC_LAUNCH(NORM, STREAM, ONE)                                                                       \
+  hipLaunchKernelGGL((nz_decode_kernel<S, NORM, STREAM, ONE>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes, \
                      (const uint8_t*)packed, (uint16_t*)out, g, d_status, nm)
   if (nm.bytes) {
-    if (stream_out) NZ_DEC_LAUNCH(true, true);
-    else NZ_DEC_LAUNCH(true, false);
+    if (stream_out) NZ_DEC_LAUNCH(true, true, false);
+    else if (one) NZ_DEC_LAUNCH(true, false, true);
+    else NZ_DEC_LAUNCH(true, false, false);
   } else {
-    if (stream_out) NZ_DEC_LAUNCH(false, true);
-    else NZ_DEC_LAUNCH(false, false);
+    if (stream_out) NZ_DEC_LAUNCH(false, true, false);
+    else if (one) NZ_DEC_LAUNCH(false, false, true);
+    else NZ_DEC_LAUNCH(false, false, false);
   }
 #undef NZ_DEC_LAUNCH
 }
@@ -54,45 +57,60 @@ void nz_launch_decode(const NzGeom& g, const void* comp, uint64_t comp_bytes, co
 template <int S>
 void nz_launch_decode_batch(const NzBatch& b, uint32_t grid, uint32_t max_spc, bool stream_out, uint32_t* d_status,
                             hipStream_t st) {
-  const size_t lds = NZ_DEC_LDS_BYTES(max_spc);
+  const bool one = !stream_out && grid <= NZ_ONE_READ_WORKGROUPS;
+  const size_t lds = NZ_DEC_LDS_BYTES(max_spc, one);
   const dim3 gd(grid), bd(64 * max_spc);
-#define NZ_BATCH_LAUNCH(NORM, STREAM) \
-  hipLaunchKernelGGL((nz_decode_batch_kernel<S, NORM, STREAM>), gd, bd, lds, st, b, d_status)
+#define NZ_BATCH_LAUNCH(NORM, STREAM, ONE) \
+  hipLaunchKernelGGL((nz_decode_batch_kernel<S, NORM, STREAM, ONE>), gd, bd, lds, st, b, d_status)
   if (b.item[0].norm) {
-    if (stream_out) NZ_BATCH_LAUNCH(true, true);
-    else NZ_BATCH_LAUNCH(true, false);
+    if (stream_out) NZ_BATCH_LAUNCH(true, true, false);
+    else if (one) NZ_BATCH_LAUNCH(true, false, true);
+    else NZ_BATCH_LAUNCH(true, false, false);
   } else {
-    if (stream_out) NZ_BATCH_LAUNCH(false, true);
-    else NZ_BATCH_LAUNCH(false, false);
+    if (stream_out) NZ_BATCH_LAUNCH(false, true, false);
+    else if (one) NZ_BATCH_LAUNCH(false, false, true);
+    else NZ_BATCH_LAUNCH(false, false, false);
   }
 #undef NZ_BATCH_LAUNCH
 }
 
-template <int S>
-void nz_launch_gemv(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
-  const size_t lds = NZ_DEC_LDS_BYTES(max_spc);
+template <int S, bool ONE>
+void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
+  const size_t lds = NZ_DEC_LDS_BYTES(max_spc, ONE);
   const dim3 gd(grid), bd(64 * max_spc);
   // one activation row, or kernels that hold 2, 4 or 8 of them per lane (tensors with
   // normalizers: one row only, the caller has checked)
-  if (b.item[0].norm) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, true, 1>), gd, bd, lds, st, b, d_status);
-  else if (b.x_rows <= 1) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 1>), gd, bd, lds, st, b, d_status);
-  else if (b.x_rows <= 2) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 2>), gd, bd, lds, st, b, d_status);
-  else if (b.x_rows <= 4) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 4>), gd, bd, lds, st, b, d_status);
-  else hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 8>), gd, bd, lds, st, b, d_status);
+  if (b.item[0].norm) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, true, 1, ONE>), gd, bd, lds, st, b, d_status);
+  else if (b.x_rows <= 1) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 1, ONE>), gd, bd, lds, st, b, d_status);
+  else if (b.x_rows <= 2) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 2, ONE>), gd, bd, lds, st, b, d_status);
+  else if (b.x_rows <= 4) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 4, ONE>), gd, bd, lds, st, b, d_status);
+  else hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 8, ONE>), gd, bd, lds, st, b, d_status);
+}
+
+template <int S>
+void nz_launch_gemv(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
+  if (grid <= NZ_ONE_READ_WORKGROUPS) nz_launch_gemv_form<S, true>(b, grid, max_spc, d_status, st);
+  else nz_launch_gemv_form<S, false>(b, grid, max_spc, d_status, st);
 }
 
 template <int S>
 void nz_launch_rows(const NzGeom& g, const void* comp, uint64_t comp_bytes, const void* packed, uint16_t* scratch,
                     uint32_t* d_status, const NzNorm& nm, const long long* idx, uint32_t count, uint32_t row_len,
                     uint32_t cpr, hipStream_t st) {
-  const size_t lds = NZ_DEC_LDS_BYTES(g.spc);
+  const bool one = count * cpr <= NZ_ONE_READ_WORKGROUPS;
+  const size_t lds = NZ_DEC_LDS_BYTES(g.spc, one);
   const dim3 gd(count * cpr), bd(64 * g.spc);
-  if (nm.bytes)
-    hipLaunchKernelGGL((nz_decode_rows_kernel<S, true>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes,
-                       (const uint8_t*)packed, scratch, g, d_status, nm, idx, row_len, cpr);
-  else
-    hipLaunchKernelGGL((nz_decode_rows_kernel<S, false>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes,
-                       (const uint8_t*)packed, scratch, g, d_status, nm, idx, row_len, cpr);
+#define NZ_ROWS_LAUNCH(NORM, ONE)                                                                               \
+  hipLaunchKernelGGL((nz_decode_rows_kernel<S, NORM, ONE>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes, \
+                     (const uint8_t*)packed, scratch, g, d_status, nm, idx, row_len, cpr)
+  if (nm.bytes) {
+    if (one) NZ_ROWS_LAUNCH(true, true);
+    else NZ_ROWS_LAUNCH(true, false);
+  } else {
+    if (one) NZ_ROWS_LAUNCH(false, true);
+    else NZ_ROWS_LAUNCH(false, false);
+  }
+#undef NZ_ROWS_LAUNCH
 }
 
 // NZ_PART (optional) cuts the unit into parts that a build can compile side by side:
