@@ -15,6 +15,20 @@
 #include "../../include/neuzip_hip.h"
 #include "nz_launch.h"
 
+#define NZ_MAX_DEVICES 64
+
+uint32_t nz_compute_units() {
+  static std::atomic<uint32_t> known[NZ_MAX_DEVICES];  // 0: not looked up yet
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= NZ_MAX_DEVICES) return 0;
+  uint32_t n = known[dev].load(std::memory_order_relaxed);
+  if (n == 0 && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0) {
+    n = (uint32_t)cus;
+    known[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 namespace {
 
 thread_local std::string g_err;
@@ -371,7 +385,6 @@ int encode_stateless(const void* dev_bf16, uint64_t n, int precision, uint32_t c
 // In host code `nz_static_scratch` is only a handle for hipGetSymbolAddress;
 // the device address of each GPU's copy is looked up once and kept.
 static __device__ __align__(256) uint8_t nz_static_scratch[NZ_STATIC_SCRATCH_BYTES];
-#define NZ_MAX_DEVICES 64
 std::mutex g_static_mu;
 uint8_t* g_static_ptr[NZ_MAX_DEVICES];
 

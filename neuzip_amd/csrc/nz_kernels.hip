@@ -1504,9 +1504,27 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 32 == 0, "parse results fit under the tail");
 // dynamic LDS of a decode workgroup whose chunks have up to `spc` segments
 #define NZ_DEC_LDS_BYTES(spc, one) ((size_t)(2 * NZ_M + (spc) * NZ_RING_ALLOC_DWORDS(one)) * 4)
-// Launches of at most this many workgroups, one per compute unit and so at most
-// two wavefronts per SIMD, decode with NzWaveDecOne (whose figures stand there).
-#define NZ_ONE_READ_WORKGROUPS 256u
+// Launches of at most one workgroup per compute unit decode with NzWaveDecOne,
+// unless their output is written with streaming stores.  The line lies where the
+// figures cross for the default chunk (eight wavefronts, 256 symbols per lane;
+// MI355X, 256 compute units; two-read against one-read step, microseconds):
+//   read     8 workgroups 29.7 / 25.2, 128 33.6 / 29.7, 256 34.6 / 31.7,
+//            257 40.7 / 40.7, 320 41.2 / 41.2, 512 42.9 / 44.4, 768 62.6 / 67.1
+//   product  1 row   256 workgroups 34.0 / 29.4, 320 42.0 / 41.6, 448 42.2 / 41.9, 896 72.6 / 77.5
+//            8 rows  256 workgroups 42.0 / 39.2, 320 64.5 / 63.2, 448 65.9 / 64.3, 896 121.0 / 118.7
+//   gather   1 row 32.5 / 27.8, 256 rows 40.5 / 38.1, 320 rows 48.2 / 47.8, 512 rows 52.4 / 53.3
+// It counts workgroups and not wavefronts: chunks of four wavefronts (65536 / 256)
+// still gain above it (320 workgroups 34.6 / 30.8, 512 35.5 / 32.4, 768 39.4 / 38.3)
+// and lose at 1024 (45.2 / 61.1), and so do eight-row products (above) and reads
+// with normalizers (320 workgroups, precision 3, groups of 64: 50.3 / 47.2); all
+// of those keep the two-read step.  Below the line it costs where a wavefront
+// takes many words (6 bits per exponent, 256 workgroups: 36.3 / 36.9; 8 workgroups:
+// 29.8 / 27.1) and where four streams launch 256 workgroups each at the same time
+// (342 / 370 for sixteen reads: two workgroups to a compute unit and not three;
+// two such streams 206 / 204, eight of 128 workgroups 486 / 459).
+NZ_HD static inline bool nz_one_read(uint64_t workgroups, uint32_t compute_units, bool stream_out) {
+  return !stream_out && workgroups <= compute_units;
+}
 
 // S+1 packed bytes of one 8-element group, as a little-endian integer
 template <int S>

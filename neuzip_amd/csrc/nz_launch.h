@@ -8,6 +8,10 @@
 
 #include "nz_kernels.hip"
 
+// Compute units of the device in use, which nz_one_read goes by (256, or an equal part of
+// them where the GPU is partitioned); looked up once per device.
+__attribute__((visibility("hidden"))) uint32_t nz_compute_units();
+
 // Allow the register encode kernels of precision S up to 96 KiB of dynamic LDS
 // (more than 64 KiB has to be asked for once per kernel and device).
 template <int S>

@@ -36,7 +36,7 @@ void nz_launch_encode(const NzEncBatch& b, int cls, dim3 grid, dim3 block, uint3
 template <int S>
 void nz_launch_decode(const NzGeom& g, const void* comp, uint64_t comp_bytes, const void* packed, void* out,
                       uint32_t* d_status, const NzNorm& nm, uint32_t stream_out, hipStream_t st) {
-  const bool one = !stream_out && g.n_chunks <= NZ_ONE_READ_WORKGROUPS;
+  const bool one = nz_one_read(g.n_chunks, nz_compute_units(), stream_out);
   const size_t lds = NZ_DEC_LDS_BYTES(g.spc, one);
   const dim3 gd((uint32_t)g.n_chunks), bd(64 * g.spc);
 #define NZ_DEC_LAUNCH(NORM, STREAM, ONE)                                                                       \
@@ -57,7 +57,7 @@ void nz_launch_decode(const NzGeom& g, const void* comp, uint64_t comp_bytes, co
 template <int S>
 void nz_launch_decode_batch(const NzBatch& b, uint32_t grid, uint32_t max_spc, bool stream_out, uint32_t* d_status,
                             hipStream_t st) {
-  const bool one = !stream_out && grid <= NZ_ONE_READ_WORKGROUPS;
+  const bool one = nz_one_read(grid, nz_compute_units(), stream_out);
   const size_t lds = NZ_DEC_LDS_BYTES(max_spc, one);
   const dim3 gd(grid), bd(64 * max_spc);
 #define NZ_BATCH_LAUNCH(NORM, STREAM, ONE) \
@@ -89,7 +89,7 @@ void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint
 
 template <int S>
 void nz_launch_gemv(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
-  if (grid <= NZ_ONE_READ_WORKGROUPS) nz_launch_gemv_form<S, true>(b, grid, max_spc, d_status, st);
+  if (nz_one_read(grid, nz_compute_units(), false)) nz_launch_gemv_form<S, true>(b, grid, max_spc, d_status, st);
   else nz_launch_gemv_form<S, false>(b, grid, max_spc, d_status, st);
 }
 
@@ -97,7 +97,7 @@ template <int S>
 void nz_launch_rows(const NzGeom& g, const void* comp, uint64_t comp_bytes, const void* packed, uint16_t* scratch,
                     uint32_t* d_status, const NzNorm& nm, const long long* idx, uint32_t count, uint32_t row_len,
                     uint32_t cpr, hipStream_t st) {
-  const bool one = count * cpr <= NZ_ONE_READ_WORKGROUPS;
+  const bool one = nz_one_read((uint64_t)count * cpr, nz_compute_units(), false);
   const size_t lds = NZ_DEC_LDS_BYTES(g.spc, one);
   const dim3 gd(count * cpr), bd(64 * g.spc);
 #define NZ_ROWS_LAUNCH(NORM, ONE)                                                                               \
