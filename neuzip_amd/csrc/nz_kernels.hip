@@ -1795,34 +1795,15 @@ struct NzGemvWalk {
   }
 };
 
-// Decoder state of one wavefront.
-struct NzWaveDec {
-  const uint2* lut;
-  uint32_t* ring32;       // 512 dwords = 1024 words: a window of the record
+// A wavefront's record and its ring: where the record lies, what may be loaded of it, and the
+// staging of its head.
+struct NzRecord {
+  uint32_t* ring32;       // 512 dwords (NzWaveDec) or 1024 (NzWaveDecOne)
   const uint8_t* words;   // start of the record (uniform); word indices count from here
   uint32_t lim;           // largest byte offset from `words` that may be loaded: container end - 16 (uniform)
   uint32_t ring_lds;      // LDS byte address of the ring (the same in all lanes, kept in a vector register)
   uint32_t nwords;        // 16-bit units the record holds, table and states included
   uint32_t lane;
-  uint32_t x;             // this lane's rANS state
-  uint32_t base;          // words consumed by the wave (the same in all lanes, kept in a vector register)
-  uint32_t filled;        // dwords staged into the ring (multiple of 256; uniform)
-  uint32_t sel_keep, sel_shift;  // byte selectors of the renormalisation (vector registers)
-  uint4 r;                // 8 words per lane fetched during the previous group
-
-  // 16 bytes of the word stream at dword index d (multiple of 4 per lane).
-  // Addresses are clamped to the container's closing padding, so every load is
-  // unconditional and in bounds; words past the record are never consumed by
-  // a valid stream.
-  __device__ __forceinline__ uint4 fetch(uint32_t d) const {
-    const uint32_t off = 4u * d < lim ? 4u * d : lim;
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(words + off);
-    return make_uint4(q[0], q[1], q[2], q[3]);
-  }
-
-  __device__ __forceinline__ void commit(uint32_t d, const uint4& v) {
-    *reinterpret_cast<uint4*>(ring32 + (d & (NZ_RING_DWORDS - 1))) = v;
-  }
 
   // record at comp + pos of a container of comp_bytes (pos + 16 <= comp_bytes)
   __device__ __forceinline__ void attach(const uint8_t* comp, uint64_t comp_bytes, uint64_t pos, uint32_t* ring) {
@@ -1834,14 +1815,47 @@ struct NzWaveDec {
     lim = room < 0xFFFFFFF0ull ? (uint32_t)room : 0xFFFFFFF0u;
   }
 
+  // Address of byte `off` of the record, clamped to the container's closing
+  // padding: every load of up to 16 bytes through it is in bounds, so the loads
+  // are unconditional; words past the record are never consumed by a valid stream.
+  __device__ __forceinline__ const uint8_t* at(uint32_t off) const { return words + (off < lim ? off : lim); }
+
+  // 16 (8) bytes of the word stream at dword index d
+  __device__ __forceinline__ uint4 fetch(uint32_t d) const {
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(at(4u * d));
+    return make_uint4(q[0], q[1], q[2], q[3]);
+  }
+  __device__ __forceinline__ uint2 fetch2(uint32_t d) const {
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(at(4u * d));
+    return make_uint2(q[0], q[1]);
+  }
+
   // Stage the first 512 dwords of the record (table of a chunk's first record,
-  // coder states, first words) into the ring.
+  // coder states, first words) where the ring is.
   __device__ __forceinline__ void stage() {
     uint4 v[2];
 #pragma unroll
     for (uint32_t q = 0; q < 2; ++q) v[q] = fetch(256 * q + 4 * lane);
 #pragma unroll
-    for (uint32_t q = 0; q < 2; ++q) commit(256 * q + 4 * lane, v[q]);
+    for (uint32_t q = 0; q < 2; ++q) *reinterpret_cast<uint4*>(ring32 + 256 * q + 4 * lane) = v[q];
+  }
+};
+
+// Decoder state of one wavefront.
+struct NzWaveDec : NzRecord {  // the ring holds 1024 words: a window of the record
+  const uint2* lut;
+  uint32_t x;             // this lane's rANS state
+  uint32_t base;          // words consumed by the wave (the same in all lanes, kept in a vector register)
+  uint32_t filled;        // dwords staged into the ring (multiple of 256; uniform)
+  uint32_t sel_keep, sel_shift;  // byte selectors of the renormalisation (vector registers)
+  uint4 r;                // 8 words per lane fetched during the previous group
+
+  __device__ __forceinline__ void commit(uint32_t d, const uint4& v) {
+    *reinterpret_cast<uint4*>(ring32 + (d & (NZ_RING_DWORDS - 1))) = v;
+  }
+
+  __device__ __forceinline__ void stage() {
+    NzRecord::stage();
     filled = 512;
   }
 
@@ -1926,14 +1940,9 @@ struct NzWaveDec {
 // makes the entries of 256 words at a time, four per lane, with independent
 // reads; a weight's exponents take one word per six symbols or so, so that is
 // one prepared entry for six chains of half the length.
-struct NzWaveDecOne {
+struct NzWaveDecOne : NzRecord {  // the ring holds 512 entries: a window of the words
   const uint2* lut;
-  uint32_t* ring32;       // 512 entries: a window of the words
-  const uint8_t* words;   // start of the record (uniform); word indices count from here
-  uint32_t lim;           // largest byte offset from `words` that may be loaded: container end - 16 (uniform)
-  uint32_t lut_lds, ring_lds;  // LDS byte addresses (the same in all lanes, kept in vector registers)
-  uint32_t nwords;        // 16-bit units the record holds, table and states included
-  uint32_t lane;
+  uint32_t lut_lds;       // LDS byte address of the slot table, like ring_lds
   uint32_t x;             // this lane's rANS state, before the word it may still have to take
   uint32_t top;           // the state's upper bits, x << 4 with a word to take, x >> 12 without
   uint32_t widx;          // index of that word
@@ -1941,41 +1950,6 @@ struct NzWaveDecOne {
   uint32_t base;          // words consumed by the wave (the same in all lanes, kept in a vector register)
   uint32_t filled;        // words entered into the ring (multiple of 4; uniform)
   uint2 r;                // 4 words per lane fetched after the previous refill
-
-  // 16 (8) bytes of the word stream at dword index d.  Addresses are clamped to
-  // the container's closing padding, so every load is unconditional and in
-  // bounds; words past the record are never consumed by a valid stream.
-  __device__ __forceinline__ uint4 fetch(uint32_t d) const {
-    const uint32_t off = 4u * d < lim ? 4u * d : lim;
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(words + off);
-    return make_uint4(q[0], q[1], q[2], q[3]);
-  }
-  __device__ __forceinline__ uint2 fetch2(uint32_t d) const {
-    const uint32_t off = 4u * d < lim ? 4u * d : lim;
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(words + off);
-    return make_uint2(q[0], q[1]);
-  }
-
-  // record at comp + pos of a container of comp_bytes (pos + 16 <= comp_bytes)
-  __device__ __forceinline__ void attach(const uint8_t* comp, uint64_t comp_bytes, uint64_t pos, uint32_t* ring) {
-    typedef __attribute__((address_space(3))) uint32_t lds_u32;
-    ring32 = ring;
-    ring_lds = (uint32_t)(uintptr_t)((lds_u32*)ring);
-    lut_lds = (uint32_t)(uintptr_t)((lds_u32*)reinterpret_cast<const uint32_t*>(lut));
-    words = comp + pos;
-    const uint64_t room = comp_bytes - NZ_TAIL_PAD - pos;
-    lim = room < 0xFFFFFFF0ull ? (uint32_t)room : 0xFFFFFFF0u;
-  }
-
-  // Stage the first 512 dwords of the record (table of a chunk's first record,
-  // coder states, first words) where the ring will be.
-  __device__ __forceinline__ void stage() {
-    uint4 v[2];
-#pragma unroll
-    for (uint32_t q = 0; q < 2; ++q) v[q] = fetch(256 * q + 4 * lane);
-#pragma unroll
-    for (uint32_t q = 0; q < 2; ++q) *reinterpret_cast<uint4*>(ring32 + 256 * q + 4 * lane) = v[q];
-  }
 
   // the entries of words first + 4 * lane ... + 3 (first a multiple of 4) into the ring
   __device__ __forceinline__ void enter(uint32_t first, const uint2 v) {
@@ -2006,6 +1980,8 @@ struct NzWaveDecOne {
     enter(from, a);
     enter(from + NZ_ONE_BLOCK, b);
     lds_order();
+    typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
+    lut_lds = (uint32_t)(uintptr_t)((lds_cu32*)reinterpret_cast<const uint32_t*>(lut));
     x = x0;
     top = x0 >> NZ_PROB_BITS;
     widx = first_word;
@@ -2061,10 +2037,7 @@ struct NzWaveDecOne {
   // The state after the last step, with the word it took: the ring does not
   // hold the words themselves, so that one comes from the record again.
   __device__ __forceinline__ void finish() {
-    if (x < NZ_L) {
-      const uint32_t off = 2u * widx < lim ? 2u * widx : lim;
-      x = (x << 16) | *reinterpret_cast<const uint16_t*>(words + off);
-    }
+    if (x < NZ_L) x = (x << 16) | *reinterpret_cast<const uint16_t*>(at(2u * widx));
   }
 };
 
