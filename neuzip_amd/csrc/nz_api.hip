@@ -834,15 +834,21 @@ int pick_geometry(const nz_manager* m, const char* name, uint64_t n, NzGeom* g, 
     // segments of 64 to 512 symbols per lane each) when that is inside the size
     // budget and the model below promises 10 % or more; a tensor too small for
     // that may get 32 Ki chunks of eight 4 Ki segments (again: only inside the
-    // budget).  Time of a round ~ symbols per lane x time of a step, which
-    // grows with the wavefronts that share a SIMD unit (2, 4, 6 of them: about
-    // 107, 147, 215 ns per step).
+    // budget).  Time of a round ~ symbols per lane x a weight that grows with the
+    // workgroups on a compute unit.  Only the ratios of the weights matter: they
+    // are those of whole reads, 31.9, 43.8, 62.6 us with one, two, three workgroups
+    // per compute unit at 256 symbols per lane (107 : 147 : 210), where the first
+    // takes the one-read step of the decoder; products 30.0, 42.4, 53.8 us.  A
+    // smaller first weight would change the choice at the default budget for 313
+    // to 384 chunks (one longer round instead of two): there a read gains 8 % at
+    // 314 chunks (41.0 -> 37.6 us) and 3 % at 336 and loses from 344 on, a product
+    // of rows of 4096 gains 17 % at 314, 8 % at 336 and 0 to 6 % above.
     const uint64_t slots = m->slots, cus = slots / 3;
     const uint64_t chunks = (n + chunk_syms - 1) / chunk_syms;
     if (chunks <= slots && cus != 0) {
-      static const uint32_t step_ns[3] = {107, 147, 215};
+      static const uint32_t weight[3] = {107, 147, 215};
       const uint64_t per_cu = chunks ? (chunks + cus - 1) / cus : 1;  // 1..3 workgroups per compute unit
-      uint64_t best_t = (uint64_t)lane_syms * step_ns[per_cu - 1];
+      uint64_t best_t = (uint64_t)lane_syms * weight[per_cu - 1];
       bool found = false;
       for (uint32_t k = 1; k <= 3; ++k) {
         const uint64_t per_lane = (n + k * cus * 512 - 1) / (k * cus * 512);  // a chunk is 8 x 64 lanes
@@ -850,7 +856,7 @@ int pick_geometry(const nz_manager* m, const char* name, uint64_t n, NzGeom* g, 
         if (lane < 64 || lane > 512) continue;
         const uint32_t chunk = lane * NZ_LANES * NZ_MAX_SEGS_PER_CHUNK;
         if (nz_geom_check(chunk, lane) || !in_budget(n, chunk, lane, m->budget)) continue;
-        const uint64_t t = (uint64_t)lane * step_ns[k - 1];
+        const uint64_t t = (uint64_t)lane * weight[k - 1];
         if (10 * t < 9 * best_t) {  // another geometry only for a gain above 10 %
           best_t = t;
           lane_syms = lane;

@@ -1482,18 +1482,23 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 // fused rANS decode + merge: one workgroup per chunk, one wavefront per segment
 // ----------------------------------------------------------------------------
 //
-// LDS: a 4096-entry slot table of 8-byte entries
+// LDS: a 4096-entry slot table of 8-byte entries (32 KiB)
 //          lo = freq | symbol << 24      hi = slot - cum[symbol]
 //      (so that one v_mad_u32_u24 of lo's low 24 bits gives the next state and
-//      the symbol is a whole byte for v_perm_b32), per wavefront a ring of
-//      1024 16-bit units (2 KiB) that is a sliding window over the segment's
-//      record (it first holds the record's head: table, coder states, first
-//      words), and the 257 cumulative frequencies of the table parse.  Eight
-//      wavefronts per chunk need 49 KiB, so three workgroups share the 160 KiB
-//      of a CU.
-// A rANS step per lane: one table read, one multiply-add, and when the state
-// falls below 2^16 a 16-bit word taken at (words consumed so far by the wave +
-// rank of the lane among the lanes that need one).
+//      the symbol is a whole byte for v_perm_b32), and per wavefront a ring that
+//      slides over the segment's record and first holds the record's head
+//      (table, coder states, first words).  What the table parse leaves for the
+//      fill lies under the table's last slots.
+// A rANS step per lane: x = freq * (x >> 12) + hi, and when the state falls below
+// 2^16 a 16-bit word taken at (words consumed so far by the wave + rank of the
+// lane among the lanes that need one).  Two forms:
+//   NzWaveDec     slot read, then the word's read: the ring holds 1024 words
+//                 (2 KiB); a workgroup of eight wavefronts has 48 KiB, three
+//                 share the 160 KiB of a CU
+//   NzWaveDecOne  one read, of a slot or of an entry prepared from the word: the
+//                 ring holds the entries of 512 words (4 KiB); 64 KiB, two
+//                 workgroups to a CU.  For launches of at most one workgroup per
+//                 CU (nz_one_read).
 
 #define NZ_RING_ALLOC_DWORDS(one) ((one) ? 2 * NZ_ONE_WORDS : NZ_RING_DWORDS)
 // What the table parse leaves for the slot-table fill (runs, windows, flags)
@@ -1508,16 +1513,16 @@ static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 3
 // unless their output is written with streaming stores.  The line lies where the
 // figures cross for the default chunk (eight wavefronts, 256 symbols per lane;
 // MI355X, 256 compute units; two-read against one-read step, microseconds):
-//   read     8 workgroups 29.7 / 25.2, 128 33.6 / 29.7, 256 34.6 / 31.7,
-//            257 40.7 / 40.7, 320 41.2 / 41.2, 512 42.9 / 44.4, 768 62.6 / 67.1
-//   product  1 row   256 workgroups 34.0 / 29.4, 320 42.0 / 41.6, 448 42.2 / 41.9, 896 72.6 / 77.5
-//            8 rows  256 workgroups 42.0 / 39.2, 320 64.5 / 63.2, 448 65.9 / 64.3, 896 121.0 / 118.7
+//   read     8 workgroups 29.7 / 25.2, 128: 33.6 / 29.7, 256: 34.6 / 31.7,
+//            257: 40.7 / 40.7, 320: 41.2 / 41.2, 512: 42.9 / 44.4, 768: 62.6 / 67.1
+//   product  1 row   256: 34.0 / 29.4, 320: 42.0 / 41.6, 448: 42.2 / 41.9, 896: 72.6 / 77.5
+//            8 rows  256: 42.0 / 39.2, 320: 64.5 / 63.2, 448: 65.9 / 64.3, 896: 121.0 / 118.7
 //   gather   1 row 32.5 / 27.8, 256 rows 40.5 / 38.1, 320 rows 48.2 / 47.8, 512 rows 52.4 / 53.3
 // It counts workgroups and not wavefronts: chunks of four wavefronts (65536 / 256)
-// still gain above it (320 workgroups 34.6 / 30.8, 512 35.5 / 32.4, 768 39.4 / 38.3)
-// and lose at 1024 (45.2 / 61.1), and so do eight-row products (above) and reads
-// with normalizers (320 workgroups, precision 3, groups of 64: 50.3 / 47.2); all
-// of those keep the two-read step.  Below the line it costs where a wavefront
+// would still gain above it (320: 34.6 / 30.8, 512: 35.5 / 32.4, 768: 39.4 / 38.3)
+// and lose at 1024 (45.2 / 61.1); eight-row products (above) and reads with
+// normalizers (320, precision 3, groups of 64: 50.3 / 47.2) would gain as well.
+// All of those keep the two-read step.  Below the line it costs where a wavefront
 // takes many words (6 bits per exponent, 256 workgroups: 36.3 / 36.9; 8 workgroups:
 // 29.8 / 27.1) and where four streams launch 256 workgroups each at the same time
 // (342 / 370 for sixteen reads: two workgroups to a compute unit and not three;
@@ -1939,7 +1944,8 @@ struct NzWaveDec : NzRecord {  // the ring holds 1024 words: a window of the rec
 // 2^16, from the slot table otherwise, then one multiply-add.  A wavefront
 // makes the entries of 256 words at a time, four per lane, with independent
 // reads; a weight's exponents take one word per six symbols or so, so that is
-// one prepared entry for six chains of half the length.
+// one prepared entry for six chains of half the length (a read of 8 chunks of
+// 256 symbols per lane: 29.7 us with two reads per step, 25.2 us with one).
 struct NzWaveDecOne : NzRecord {  // the ring holds 512 entries: a window of the words
   const uint2* lut;
   uint32_t lut_lds;       // LDS byte address of the slot table, like ring_lds

@@ -100,10 +100,10 @@ class FusedGemv:
                 if len(g.handles) > 1:
                     self._fit_geometry(g)
 
-    # Step time of a wavefront (ns) with one, two, three 8-wavefront workgroups per
-    # compute unit, measured on MI355X; the same figures choose a tensor's geometry
-    # when it is written on its own.
-    _STEP_NS = (107, 147, 215)
+    # Time of a launch with one, two, three 8-wavefront workgroups per compute unit and
+    # equal segments, up to a common factor (MI355X); the weights that choose a tensor's
+    # geometry when it is written on its own (pick_geometry in csrc/nz_api.hip).
+    _WEIGHT = (107, 147, 215)
 
     def _fit_geometry(self, g, cus=None) -> None:
         """Matrices that one launch decodes together are stored again with ONE
@@ -123,7 +123,7 @@ class FusedGemv:
                 lane += 8  # every tensor's last chunk is rounded up
             if not 64 <= lane <= 512 or not all(be.in_budget(n, lane * 512, lane) for n in sizes):
                 continue
-            t = lane * self._STEP_NS[k - 1]
+            t = lane * self._WEIGHT[k - 1]
             if best is None or t <= best[0]:  # measured on gate/up of an 8B model: 2 x 512 chunks 73-76 us, 2 x 256 71.5, 2 x 378 69.4
                 best = (t, lane)
         if best is None:
