@@ -357,10 +357,7 @@ struct NzEncLds {
   uint32_t scan_s[4];
   uint64_t mw[4];
   uint32_t cf[256];
-  // per symbol: x = freq << 20 (renormalisation threshold), y = freq, z = cum,
-  // w = bits of a float just below 1 / freq (four units in the last place
-  // under the correctly rounded quotient)
-  uint4 tab[256];
+  uint4 tab[256];  // per symbol: nz_quot_entry
   uint32_t sbuf[NZ_MAX_SEGS_PER_CHUNK][NZ_STATE_MAX_BYTES / 4];
   uint32_t pad_sym, raw;
   // for records that go straight to their place: the chunk's record sizes, the
@@ -439,6 +436,28 @@ __device__ __forceinline__ uint64_t nz_split_tail(const uint16_t* __restrict__ i
   return e;
 }
 
+// x / f in one instruction.  The 32 bits of x, taken as those of a double, are the
+// subnormal x * 2^-1074; the table's multiplier is 2^1023 * r with r a little above
+// 1 / f (nz_quot_entry), so the fused multiply-add forms x * r * 2^-51 + 2 - 2^-52 exactly
+// and rounds once, to a multiple of 2^-51: the low word of the result is x * r - 1/2
+// rounded to nearest, which is floor(x / f) for 16 <= x < f << 20 (x * r exceeds x / f by
+// less than 2^-18, so it is never a whole number and never reaches the next one; pinned
+// on the host for every f, tests/test_quotient_fma.py).  FP64 multiply-adds run at the rate
+// of the 32-bit integer ones here, subnormals included.
+__device__ __forceinline__ uint32_t nz_quot(uint32_t x, uint32_t r_lo, uint32_t r_hi) {
+  const double xd = __builtin_bit_cast(double, (uint64_t)x);
+  const double r = __builtin_bit_cast(double, ((uint64_t)r_hi << 32) | r_lo);
+  return (uint32_t)__builtin_bit_cast(uint64_t, __builtin_fma(xd, r, 2.0 - 0x1p-52));
+}
+
+// The encoder's entry of a symbol: x = freq << 20 (renormalisation threshold), y = 4096 - freq,
+// z and w = the multiplier of nz_quot, whose 12 lowest bits give way to cum: the multiplier
+// is made 1 + 2^-39 times too large first, so that it stays above 1 / freq whatever they are.
+__device__ __forceinline__ uint4 nz_quot_entry(uint32_t f, uint32_t cum) {
+  const uint64_t r = f ? __builtin_bit_cast(uint64_t, (1.0 + 0x1p-39) / (double)f) + (1023ull << 52) : 0ull;
+  return make_uint4(f << 20, NZ_M - f, ((uint32_t)r & ~(NZ_M - 1)) | cum, (uint32_t)(r >> 32));
+}
+
 // From the chunk's histogram (cn symbols): the 12-bit frequency table (sum
 // exactly 4096), the encoder's per-symbol entries in LDS, the serialized table
 // and the chunk record.  Run by the whole workgroup (at least 256 threads).
@@ -483,7 +502,7 @@ __device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t c
     uint32_t woff = 0;
     for (uint32_t w = 0; w < (tid >> 6); ++w) woff += L.scan_s[w];
     const uint32_t cum = woff + incl - f;
-    L.tab[tid] = make_uint4(f << 20, f, cum, f ? __float_as_uint(1.0f / (float)f) - 4u : 0u);
+    L.tab[tid] = nz_quot_entry(f, cum);
   }
 
   // ---- serialise the table, in parallel ----
@@ -621,45 +640,59 @@ __device__ __forceinline__ bool nz_chunk_finalize(uint64_t c, uint64_t n, uint32
 // that codes to more than its raw size is stored raw (decided at the end of the
 // kernel, once all segments of the chunk are coded).
 
-// the 8 symbols of one group (byte j of `sy` = symbol j), last symbol first
-// (words go to the segment's slot in scratch memory, or with LDS to the
-// wavefront's staging area: word p of the slot at LDS byte address lds0 + 2 p)
-template <bool LDS>
-__device__ __forceinline__ void nz_enc_group(uint32_t& x, uint32_t& pos, const uint64_t sy,
-                                             const uint4* __restrict__ tab, uint16_t* __restrict__ slot,
-                                             const uint32_t lds0) {
-  typedef __attribute__((address_space(3))) uint16_t lds_u16;
-  // the table entries do not depend on the state: fetch four at a time, up front
-#pragma unroll
-  for (int h = 1; h >= 0; --h) {
-  uint4 e[8];
-#pragma unroll
-  for (int j = 4 * h; j < 4 * h + 4; ++j) e[j] = tab[(uint32_t)(sy >> (8 * j)) & 0xFFu];
-#pragma unroll
-  for (int j = 4 * h + 3; j >= 4 * h; --j) {
-    const uint32_t f = e[j].y;
-    const bool need = x >= e[j].x;
-    const uint64_t m = __ballot(need);
-    pos -= (uint32_t)__popcll(m);
-    if (need) {  // a 32-bit byte offset from the segment's slot: one add-shift for the address
-      if constexpr (LDS)
-        *(lds_u16*)(uintptr_t)(lds0 + ((pos + nz_rank_below(m)) << 1)) = (uint16_t)(x & 0xFFFFu);
-      else
-        *reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(slot) + ((pos + nz_rank_below(m)) << 1)) =
-            (uint16_t)(x & 0xFFFFu);
-    }
-    x = need ? (x >> 16) : x;
-    // x < f << 20 here, so the quotient x / f is below 2^20.  The float estimate
-    // x * r with r four units in the last place under 1 / f (itself within half
-    // a unit) never exceeds the quotient - the roundings of x and of the product
-    // add at most one unit each - and falls short of it by less than
-    // 2^20 * 11 * 2^-24 < 1: truncated it is the exact quotient or one less,
-    // and the remainder tells which.  With the exact quotient q the new state
-    // is (q << 12) + (x - q f) + cum = x + q (4096 - f) + cum.
-    uint32_t q = (uint32_t)((float)x * __uint_as_float(e[j].w));
-    q += (x - __umul24(q, f) >= f) ? 1u : 0u;
-    x = __umul24(q, NZ_M - f) + (x + e[j].z);
+// Table entries on their way to the encoder: four of them, those of the symbols that are coded
+// next, entry of symbol j in v[j & 3].  They do not depend on the state, so each is read four
+// steps before its use, across groups as well.
+typedef uint32_t nz_u32x4 __attribute__((ext_vector_type(4)));
+struct NzEncAhead {
+  nz_u32x4 v[4];
+
+  __device__ __forceinline__ void fetch(const uint4* __restrict__ tab, const uint64_t sy, const int j) {
+    v[j & 3] = reinterpret_cast<const nz_u32x4*>(tab)[(uint32_t)(sy >> (8 * j)) & 0xFFu];
   }
+  // the first four of a group
+  __device__ __forceinline__ void start(const uint4* __restrict__ tab, const uint64_t sy) {
+#pragma unroll
+    for (int j = 7; j >= 4; --j) fetch(tab, sy, j);
+  }
+};
+
+// the 8 symbols of one group (byte j of `sy` = symbol j), last symbol first; `sy_next`: those
+// of the group that is coded after it
+// Words go downwards from `pos`, a byte offset into the segment's slot in scratch memory or,
+// with LDS, the LDS byte address of the wavefront's staging area.  In the staging area every lane stores: a lane without a word writes one of the
+// 64 places below the words of the step (each lane its own), which the words that
+// follow overwrite.  That keeps the execution mask out of the step's chain; the
+// caller leaves 64 words of room below.
+template <bool LDS>
+__device__ __forceinline__ void nz_enc_group(uint32_t& x, uint32_t& pos, const uint64_t sy, const uint64_t sy_next,
+                                             NzEncAhead& ahead, const uint4* __restrict__ tab,
+                                             uint16_t* __restrict__ slot, const uint32_t below) {
+  typedef __attribute__((address_space(3))) uint16_t lds_u16;
+#pragma unroll
+  for (int j = 7; j >= 0; --j) {
+    nz_u32x4 e = ahead.v[j & 3];
+    asm("" : "+v"(e));  // one 16-byte read, not two of 8
+    const bool need = x >= e.x;
+    const uint64_t m = __ballot(need);
+    const uint32_t word = x;
+    x = need ? (x >> 16) : x;
+    // x < f << 20 here; with q = x / f the new state is (q << 12) + (x - q f) + cum
+    const uint32_t q = nz_quot(x, e.z, e.w);
+    uint32_t t = x + (e.z & (NZ_M - 1));
+    asm("" : "+v"(t));  // then one multiply-add
+    x = __umul24(q, e.y) + t;
+    ahead.fetch(tab, j >= 4 ? sy : sy_next, j ^ 4);
+    pos -= 2u * (uint32_t)__popcll(m);
+    if constexpr (LDS) {
+      uint32_t zero = 0;
+      asm("" : "+v"(zero));  // a vector register: the short form of the select
+      const uint32_t at = __builtin_amdgcn_mbcnt_hi(
+          (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, need ? zero : below));
+      *(lds_u16*)(uintptr_t)((at << 1) + pos) = (uint16_t)word;
+    } else if (need) {
+      *reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(slot) + ((nz_rank_below(m) << 1) + pos)) = (uint16_t)word;
+    }
   }
 }
 
@@ -959,7 +992,6 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
     asm volatile("" ::"v"((uint32_t)e), "v"((uint32_t)(e >> 32)));
 #endif
   };
-  typedef uint32_t nz_u32x4 __attribute__((ext_vector_type(4)));
   // Four groups at a time, and the loads of the next four are issued before the
   // current four are split: eight 16-byte loads per lane in flight.
   uint4 vn[4];  // the block after the current one
@@ -1051,14 +1083,18 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
     const uint32_t pad = L.pad_sym;
     // a full segment starts from 2^16 | 16 carried bits of the packed stream
     uint32_t x = NZ_L | (seg_full ? (uint32_t)reinterpret_cast<const uint16_t*>(carry_seg)[lane] : 0u);
-    uint32_t pos = cap_words;
+    // byte position of the words: the staging area stands for the last stage_w words of the slot
+    const uint32_t pos_lo = LDS ? stage_lds : 0u, pos_hi = pos_lo + 2u * (LDS ? stage_w : cap_words);
+    uint32_t pos = pos_hi;
     bool out_of_room = false;
+    NzEncAhead ahead;
     nz_static_for<NG - 1, 0, -1>([&](auto g8c) {
       constexpr int g8 = decltype(g8c)::value;
       uint32_t gv = (uint32_t)g8;
       asm volatile("" : "+s"(gv));
       if (gv < ngroups && !out_of_room) {
-        if (LDS && pos - stage_lo < NZ_GROUP * NZ_LANES) {  // a group emits at most 512 words
+        // a group emits at most 512 words and writes over the 64 places below them
+        if (LDS && pos - pos_lo < 2 * (NZ_GROUP * NZ_LANES + NZ_LANES)) {
           out_of_room = true;
         } else {
           uint64_t sy = ex[g8];
@@ -1070,14 +1106,15 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
               sy = (sy & keepm) | ((0x0101010101010101ull * pad) & ~keepm);
             }
           }
-          nz_enc_group<LDS>(x, pos, sy, L.tab, slot, stage_lds - 2u * stage_lo);
+          if (gv + 1 == ngroups) ahead.start(L.tab, sy);
+          nz_enc_group<LDS>(x, pos, sy, ex[g8 ? g8 - 1 : 0], ahead, L.tab, slot, ~lane);
         }
       }
     });
     if (out_of_room) return true;
-    nz_enc_finish(x, cap_words - pos, seg, L.sbuf[wave], lane, reinterpret_cast<uint32_t*>(it.ws + it.states),
+    nz_enc_finish(x, (pos_hi - pos) / 2, seg, L.sbuf[wave], lane, reinterpret_cast<uint32_t*>(it.ws + it.states),
                   seg_words, seg_state_bytes, &L.seg_w[wave], &L.seg_sb[wave]);
-    pos_end = pos;
+    pos_end = cap_words - (pos_hi - pos) / 2;
     return false;
   };
 #pragma nounroll
@@ -1365,22 +1402,26 @@ __global__ __launch_bounds__(NZ_ENC_LONG_THREADS) void nz_encode_long_kernel(con
     const uint32_t pad = L.pad_sym;
     const uint8_t* src = exps + seg_base;
     uint32_t x = NZ_L | (seg_n == nom ? (uint32_t)reinterpret_cast<const uint16_t*>(carry)[seg * NZ_LANES + lane] : 0u);
-    uint32_t pos = cap_words;
-    for (uint32_t gq = ngroups; gq-- > 0;) {
+    uint32_t pos = 2 * cap_words;
+    const auto group_syms = [&](uint32_t gq) {
       const uint32_t idx0 = (gq * NZ_LANES + lane) * NZ_GROUP;
-      uint64_t sy;
-      if (idx0 + 8 <= seg_n) {
-        sy = *reinterpret_cast<const uint64_t*>(src + idx0);
-      } else {
-        sy = 0;
-        for (int j = 0; j < 8; ++j) {
-          uint32_t bb = (idx0 + j < seg_n) ? src[idx0 + j] : pad;
-          sy |= (uint64_t)bb << (8 * j);
-        }
+      uint64_t sy = 0;
+      if (idx0 + 8 <= seg_n) return *reinterpret_cast<const uint64_t*>(src + idx0);
+      for (int j = 0; j < 8; ++j) {
+        uint32_t bb = (idx0 + j < seg_n) ? src[idx0 + j] : pad;
+        sy |= (uint64_t)bb << (8 * j);
       }
-      nz_enc_group<false>(x, pos, sy, L.tab, slot, 0u);
+      return sy;
+    };
+    uint64_t sy = group_syms(ngroups - 1);
+    NzEncAhead ahead;
+    ahead.start(L.tab, sy);
+    for (uint32_t gq = ngroups; gq-- > 0;) {
+      const uint64_t sy_next = group_syms(gq ? gq - 1 : 0);
+      nz_enc_group<false>(x, pos, sy, sy_next, ahead, L.tab, slot, 0u);
+      sy = sy_next;
     }
-    nz_enc_finish(x, cap_words - pos, seg, L.sbuf[wave], lane, reinterpret_cast<uint32_t*>(it.ws + it.states),
+    nz_enc_finish(x, cap_words - pos / 2, seg, L.sbuf[wave], lane, reinterpret_cast<uint32_t*>(it.ws + it.states),
                   seg_words, seg_state_bytes, &L.seg_w[wave], &L.seg_sb[wave]);
   }
   __threadfence_block();
