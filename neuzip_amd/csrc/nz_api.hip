@@ -187,19 +187,30 @@ int allow_encode_lds() {
   return NZ_OK;
 }
 
-// Words of LDS staging per wavefront for a direct encode of class `cls` with
-// workgroups of `waves` wavefronts: what a workgroup can have without lowering
-// the number of workgroups that the registers allow per compute unit (4, 6, 8
-// wavefronts per SIMD unit for 256 and more, 128, 64 symbols per lane), less the
-// kernel's own LDS.
-uint32_t stage_words_for(int cls, uint32_t waves) {
+// LDS a workgroup of `waves` wavefronts of class `cls` can have without lowering the number
+// of workgroups that the registers allow per compute unit (4, 6, 8 wavefronts per SIMD unit for
+// 256 and more, 128, 64 symbols per lane), less the kernel's own.
+uint32_t enc_dynamic_lds(int cls, uint32_t waves) {
   const uint32_t waves_per_cu = cls >= 2 ? 16u : cls == 1 ? 24u : 32u;
   const uint32_t groups = waves_per_cu / waves ? waves_per_cu / waves : 1u;
-  const uint32_t per_group = 160u * 1024u / groups;
-  const uint32_t fixed = ((uint32_t)sizeof(NzEncLds) + 511u) & ~511u;  // the kernel's own LDS
-  if (per_group <= fixed + 1024u) return 0;
-  const uint32_t per_wave = ((per_group - fixed - 512u) / waves) & ~127u;  // bytes (512: the closing slack, rounding)
-  return per_wave / 2;
+  const uint32_t per_group = 160u * 1024u / groups, fixed = (uint32_t)((sizeof(NzEncLds) + 15u) & ~15u);
+  return per_group > fixed ? per_group - fixed : 0u;
+}
+
+// The histogram takes 32 copies (32 KiB) where that LDS has room for them, which it has for
+// every geometry the library picks itself, down to 8 (8 KiB) for short chunks of short segments.
+uint32_t hist_copies_log2(int cls, uint32_t waves) {
+  uint32_t l = NZ_HIST_COPIES_LOG2;
+  if (cls < 4)
+    while (l > 3 && (1024u << l) > enc_dynamic_lds(cls, waves)) --l;
+  return l;
+}
+
+// Words of LDS staging per wavefront for a direct encode.
+uint32_t stage_words_for(int cls, uint32_t waves) {
+  const uint32_t room = enc_dynamic_lds(cls, waves);
+  if (room <= 1024u) return 0;
+  return ((room - 512u) / waves & ~127u) / 2;  // (512: the closing slack, rounding)
 }
 
 template <int S>
@@ -209,8 +220,9 @@ int launch_encode_class(NzEncBatch& b, int cls, uint32_t chunks, uint32_t max_sp
   bool direct = false;
   for (uint32_t i = 0; i < b.count; ++i) direct = direct || b.item[i].direct;
   b.stage_words = (direct && cls < 4) ? stage_words_for(cls, waves) : 0u;
-  const uint32_t lds = b.stage_words ? waves * b.stage_words * 2u + 16u : 0u;
-  nz_launch_encode<S>(b, cls, grid, block, lds, st);
+  b.copies_log2 = hist_copies_log2(cls, waves);
+  const uint32_t staging = b.stage_words ? waves * b.stage_words * 2u + 16u : 0u, hist = 1024u << b.copies_log2;
+  nz_launch_encode<S>(b, cls, grid, block, staging > hist ? staging : hist, st);
   return NZ_OK;
 }
 

@@ -21,10 +21,6 @@
 
 #include "nz_format.h"
 
-#ifndef NZ_HIST_COPIES
-#define NZ_HIST_COPIES 8u
-#endif
-#define NZ_HIST_STRIDE 257u
 #define NZ_RING_WORDS 1024u  // per-wave LDS ring of renormalisation words
 #define NZ_RING_DWORDS (NZ_RING_WORDS / 2)
 #define NZ_ONE_WORDS 512u    // the same with an 8-byte entry per word (NzWaveDecOne)
@@ -347,12 +343,38 @@ __device__ __forceinline__ uint32_t nz_block_max(uint32_t v, uint32_t* red) {
   return t;
 }
 
-// LDS of an encode workgroup.  8 histogram copies (one per lane & 7) at a
-// stride of 257 words: exponents of weights cluster on a few values, so a
-// single copy would serialise most of a wavefront's atomics on one address;
-// the odd stride keeps the copies of a bin in different banks.
+// Histogram of a workgroup, in the dynamic LDS that later holds the word staging:
+// 2^copies_log2 copies of 256 counters, one per lane modulo their number, the copies
+// of a symbol next to each other.  A wavefront's atomics then fall on banks by lane
+// and not by symbol, whatever the exponents: with 32 copies two lanes at most meet on
+// a bank, and eight atomics of a wavefront take 35 cycles of the compute unit's LDS
+// (8 copies side by side at an odd stride, where lanes with the same symbol wait for
+// each other: 144; 32 of those: 55; 64 copies of this kind: 34).
+#define NZ_HIST_COPIES_LOG2 5u
+struct NzHist {
+  uint32_t* mine;       // this lane's copy
+  uint32_t copies_log2;
+
+  static __device__ __forceinline__ void clear(uint32_t* all, uint32_t copies_log2) {
+    for (uint32_t i = threadIdx.x; i < (64u << copies_log2); i += blockDim.x)
+      reinterpret_cast<uint4*>(all)[i] = make_uint4(0u, 0u, 0u, 0u);
+  }
+  __device__ __forceinline__ void count(uint32_t symbol) const { atomicAdd(&mine[symbol << copies_log2], 1u); }
+  // a symbol's counters, 16 bytes at a time; neighbouring symbols begin at different ones (banks again)
+  static __device__ __forceinline__ uint32_t sum(const uint32_t* all, uint32_t copies_log2, uint32_t symbol) {
+    const uint4* at = reinterpret_cast<const uint4*>(all + (symbol << copies_log2));
+    const uint32_t quads = 1u << (copies_log2 - 2);
+    uint32_t c = 0;
+    for (uint32_t k = 0; k < quads; ++k) {
+      const uint4 v = at[(k + symbol) & (quads - 1)];
+      c += v.x + v.y + v.z + v.w;
+    }
+    return c;
+  }
+};
+
+// LDS of an encode workgroup (besides histogram and word staging).
 struct NzEncLds {
-  uint32_t hist[NZ_HIST_COPIES * NZ_HIST_STRIDE];
   uint32_t red[16];
   uint32_t scan_s[4];
   uint64_t mw[4];
@@ -463,17 +485,14 @@ __device__ __forceinline__ uint4 nz_quot_entry(uint32_t f, uint32_t cum) {
 // and the chunk record.  Run by the whole workgroup (at least 256 threads).
 // -> an estimate of the chunk's coded length in bits (sum of count x -log2 of
 // the quantised probability), the same in every thread.
-__device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t cn, uint8_t* __restrict__ out,
+__device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t* hist, const uint32_t copies_log2,
+                                                   const uint32_t cn, uint8_t* __restrict__ out,
                                                    NzChunkInfo* __restrict__ info_c) {
   const uint32_t tid = threadIdx.x;
   // threads 0..255 own one symbol each; the others take part in the reductions
   // with neutral values
   const bool own = tid < 256;
-  uint32_t cnt = 0;
-  if (own) {
-#pragma unroll
-    for (uint32_t k = 0; k < NZ_HIST_COPIES; ++k) cnt += L.hist[k * NZ_HIST_STRIDE + tid];
-  }
+  const uint32_t cnt = own ? NzHist::sum(hist, copies_log2, tid) : 0u;
   const uint32_t live = cnt > 0;
   const uint32_t k = nz_block_sum(live, L.red);
   // cnt * (4096 - k) fits 32 bits for chunks of up to 2^19 symbols (every geometry the library
@@ -774,6 +793,8 @@ struct NzEncItem {
 struct NzEncBatch {
   uint32_t count;
   uint32_t stage_words;  // nz_encode_kernel: 16-bit words of LDS staging per wavefront (dynamic LDS), 0 = none
+  uint32_t copies_log2;  // histogram copies (NzHist; dynamic LDS as well, used before the staging)
+  uint32_t reserved;
   NzEncItem item[NZ_ENC_BATCH_MAX];
 };
 
@@ -903,7 +924,9 @@ __device__ __forceinline__ bool nz_move_record(const NzEncItem& it, const uint64
 
 // Segments of up to 8 * NG symbols per lane: the exponents stay in registers.
 // Workgroup = max(4, segments per chunk) wavefronts; wavefront k owns segment k.
-extern __shared__ uint32_t nz_enc_stage[];  // word staging of nz_encode_kernel: stage_words / 2 dwords per wavefront + 4
+// dynamic LDS of the encode kernels: the histogram (NzHist), then the word staging of
+// nz_encode_kernel (stage_words / 2 dwords per wavefront + 4)
+extern __shared__ __attribute__((aligned(16))) uint32_t nz_enc_stage[];
 #ifdef NZ_PROBE_PHASES
 __device__ unsigned long long nz_probe_acc[8];
 #define NZ_PROBE_MARK(k)                                        \
@@ -919,7 +942,7 @@ __device__ unsigned long long nz_probe_acc[8];
 #endif
 
 template <int S, int NG>
-__global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kernel(const NzEncBatch b) {
+__global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 ? 5 : 4) void nz_encode_kernel(const NzEncBatch b) {
   __shared__ NzEncLds L;
 #ifdef NZ_PROBE_PHASES
   unsigned long long probe_t = __builtin_readcyclecounter();
@@ -964,11 +987,11 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
     L.lb[1] = it.direct ? __hip_atomic_load(lb_state + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
     L.redo = 0;
   }
-  for (uint32_t i = tid; i < NZ_HIST_COPIES * NZ_HIST_STRIDE; i += blockDim.x) L.hist[i] = 0;
+  NzHist::clear(nz_enc_stage, b.copies_log2);
   __syncthreads();
   const uint32_t lb_gen = L.lb[0];
   const bool direct = it.direct && L.lb[1] != NZ_LOOKBACK_ABORT;  // this run places its records itself
-  uint32_t* myhist = L.hist + (lane & (NZ_HIST_COPIES - 1)) * NZ_HIST_STRIDE;
+  const NzHist hist{nz_enc_stage + (lane & ((1u << b.copies_log2) - 1u)), b.copies_log2};
 
   // ---- phase 1: split.  Packed bytes go to the stored layout: segment k of a
   // chunk starts at k * seg_keep, and the last NZ_CARRY_BYTES of a full segment
@@ -987,7 +1010,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
   const auto count8 = [&](uint64_t e) {
 #ifndef NZ_PROBE_NO_HIST
 #pragma unroll
-    for (int j = 0; j < 8; ++j) atomicAdd(&myhist[(uint32_t)(e >> (8 * j)) & 0xFFu], 1u);
+    for (int j = 0; j < 8; ++j) hist.count((uint32_t)(e >> (8 * j)) & 0xFFu);
 #else  // measurement build: the split phase without its histogram (the kernel ends after the phase)
     asm volatile("" ::"v"((uint32_t)e), "v"((uint32_t)(e >> 32)));
 #endif
@@ -1044,7 +1067,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
           } else if (idx0 < seg_n) {
             const uint32_t rem = seg_n - idx0;
             ex[g4 + q] = nz_split_tail<S>(in, gi, rem, dest(g8), nm);
-            for (uint32_t j = 0; j < rem; ++j) atomicAdd(&myhist[(uint32_t)(ex[g4 + q] >> (8 * j)) & 0xFFu], 1u);
+            for (uint32_t j = 0; j < rem; ++j) hist.count((uint32_t)(ex[g4 + q] >> (8 * j)) & 0xFFu);
           }
         }
       }
@@ -1058,7 +1081,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
 #endif
 
   // ---- the chunk's table ----
-  const uint32_t est_bits = nz_build_table(L, cn, it.ws + it.tab_ser + c * NZ_TABLE_MAX_BYTES, info + c);
+  const uint32_t est_bits = nz_build_table(L, nz_enc_stage, b.copies_log2, cn, it.ws + it.tab_ser + c * NZ_TABLE_MAX_BYTES, info + c);
   NZ_PROBE_MARK(1);
 
   // ---- phase 2: code the segment from the registers, last group first ----
@@ -1106,7 +1129,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, 4) void nz_encode_kerne
               sy = (sy & keepm) | ((0x0101010101010101ull * pad) & ~keepm);
             }
           }
-          if (gv + 1 == ngroups) ahead.start(L.tab, sy);
+          if (!LDS || gv + 1 == ngroups) ahead.start(L.tab, sy);  // (across groups it would cost the slot form registers)
           nz_enc_group<LDS>(x, pos, sy, ex[g8 ? g8 - 1 : 0], ahead, L.tab, slot, ~lane);
         }
       }
@@ -1346,9 +1369,9 @@ __global__ __launch_bounds__(NZ_ENC_LONG_THREADS) void nz_encode_long_kernel(con
   const uint64_t base = c * chunk_syms;
   const uint32_t cn = (uint32_t)((n - base) < chunk_syms ? (n - base) : chunk_syms);
 
-  for (uint32_t i = tid; i < NZ_HIST_COPIES * NZ_HIST_STRIDE; i += blockDim.x) L.hist[i] = 0;
+  NzHist::clear(nz_enc_stage, b.copies_log2);
   __syncthreads();
-  uint32_t* myhist = L.hist + (tid & (NZ_HIST_COPIES - 1)) * NZ_HIST_STRIDE;
+  const NzHist hist{nz_enc_stage + (tid & ((1u << b.copies_log2) - 1u)), b.copies_log2};
 
   const uint32_t seg_keep = seg_syms / 8 * (S + 1) - NZ_CARRY_BYTES;     // of a segment of nominal length
   const uint64_t chunk_keep = (uint64_t)chunk_syms / 8 * (S + 1) - (uint64_t)NZ_CARRY_BYTES * spc;
@@ -1372,17 +1395,17 @@ __global__ __launch_bounds__(NZ_ENC_LONG_THREADS) void nz_encode_long_kernel(con
       nz_store_packed<S>(pp, f);
       *reinterpret_cast<uint64_t*>(exps + gi) = e;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) atomicAdd(&myhist[(uint32_t)(e >> (8 * j)) & 0xFFu], 1u);
+      for (int j = 0; j < 8; ++j) hist.count((uint32_t)(e >> (8 * j)) & 0xFFu);
     } else {
       e = nz_split_tail<S>(in, gi, rem, pp, nm);
       for (uint32_t j = 0; j < rem; ++j) {
         exps[gi + j] = (uint8_t)(e >> (8 * j));
-        atomicAdd(&myhist[(uint32_t)(e >> (8 * j)) & 0xFFu], 1u);
+        hist.count((uint32_t)(e >> (8 * j)) & 0xFFu);
       }
     }
   }
   __syncthreads();
-  nz_build_table(L, cn, it.ws + it.tab_ser + c * NZ_TABLE_MAX_BYTES, info + c);
+  nz_build_table(L, nz_enc_stage, b.copies_log2, cn, it.ws + it.tab_ser + c * NZ_TABLE_MAX_BYTES, info + c);
   // exponents and carried bytes of this chunk are read back below
   __threadfence_block();
   __syncthreads();

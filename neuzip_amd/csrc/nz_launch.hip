@@ -29,7 +29,7 @@ void nz_launch_encode(const NzEncBatch& b, int cls, dim3 grid, dim3 block, uint3
     case 1: hipLaunchKernelGGL((nz_encode_kernel<S, 16>), grid, block, lds, st, b); break;
     case 2: hipLaunchKernelGGL((nz_encode_kernel<S, 32>), grid, block, lds, st, b); break;
     case 3: hipLaunchKernelGGL((nz_encode_kernel<S, 36>), grid, block, lds, st, b); break;
-    default: hipLaunchKernelGGL((nz_encode_long_kernel<S>), grid, dim3(NZ_ENC_LONG_THREADS), 0, st, b); break;
+    default: hipLaunchKernelGGL((nz_encode_long_kernel<S>), grid, dim3(NZ_ENC_LONG_THREADS), lds, st, b); break;
   }
 }
 
