@@ -317,16 +317,29 @@ __device__ __forceinline__ void nz_static_for(F&& f) {
   }
 }
 
-// sums / maxima over the workgroup (at most 16 wavefronts)
-__device__ __forceinline__ uint32_t nz_block_sum(uint32_t v, uint32_t* red) {
+// sums / maxima over the workgroup (at most 16 wavefronts), two at a time; `red`: two words per wavefront
+template <class Op>
+__device__ __forceinline__ void nz_block_pair(uint32_t& a, uint32_t& b, uint32_t* red, Op second) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o, 64);
+    b = second(b, (uint32_t)__shfl_xor(b, o, 64));
+  }
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  if ((threadIdx.x & 63) == 0) reinterpret_cast<uint2*>(red)[threadIdx.x >> 6] = make_uint2(a, b);
   __syncthreads();
-  uint32_t t = 0;
-  for (uint32_t w = 0; w < blockDim.x / 64; ++w) t += red[w];
-  return t;
+  a = b = 0;
+  for (uint32_t w = 0; w < blockDim.x / 64; ++w) {
+    const uint2 v = reinterpret_cast<const uint2*>(red)[w];
+    a += v.x;
+    b = second(b, v.y);
+  }
+}
+__device__ __forceinline__ void nz_block_sum_max(uint32_t& a, uint32_t& b, uint32_t* red) {
+  nz_block_pair(a, b, red, [](uint32_t x, uint32_t y) { return x > y ? x : y; });
+}
+__device__ __forceinline__ void nz_block_sum2(uint32_t& a, uint32_t& b, uint32_t* red) {
+  nz_block_pair(a, b, red, [](uint32_t x, uint32_t y) { return x + y; });
 }
 
 __device__ __forceinline__ uint32_t nz_block_max(uint32_t v, uint32_t* red) {
@@ -375,11 +388,12 @@ struct NzHist {
 
 // LDS of an encode workgroup (besides histogram and word staging).
 struct NzEncLds {
-  uint32_t red[16];
+  uint32_t red[32];
   uint32_t scan_s[4];
   uint64_t mw[4];
   uint32_t cf[256];
   uint4 tab[256];  // per symbol: nz_quot_entry
+  uint32_t ser[NZ_TABLE_MAX_BYTES / 4];  // the serialized table
   uint32_t sbuf[NZ_MAX_SEGS_PER_CHUNK][NZ_STATE_MAX_BYTES / 4];
   uint32_t pad_sym, raw;
   // for records that go straight to their place: the chunk's record sizes, the
@@ -481,8 +495,8 @@ __device__ __forceinline__ uint4 nz_quot_entry(uint32_t f, uint32_t cum) {
 }
 
 // From the chunk's histogram (cn symbols): the 12-bit frequency table (sum
-// exactly 4096), the encoder's per-symbol entries in LDS, the serialized table
-// and the chunk record.  Run by the whole workgroup (at least 256 threads).
+// exactly 4096), the encoder's per-symbol entries in LDS, the serialized table (in LDS, and in
+// `out` for the kernels that follow) and the chunk record.  Run by the whole workgroup (at least 256 threads).
 // -> an estimate of the chunk's coded length in bits (sum of count x -log2 of
 // the quantised probability), the same in every thread.
 __device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t* hist, const uint32_t copies_log2,
@@ -494,19 +508,20 @@ __device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t* 
   const bool own = tid < 256;
   const uint32_t cnt = own ? NzHist::sum(hist, copies_log2, tid) : 0u;
   const uint32_t live = cnt > 0;
-  const uint32_t k = nz_block_sum(live, L.red);
+  // live symbols; most frequent symbol, lowest index on ties (cnt <= 2^24 fits above the index byte)
+  uint32_t k = live, key = own ? ((cnt << 8) | (255u - tid)) : 0u;
+  nz_block_sum_max(k, key, L.red);
+  const uint32_t imax = 255u - (key & 0xFFu);
   // cnt * (4096 - k) fits 32 bits for chunks of up to 2^19 symbols (every geometry the library
   // chooses itself): a 32-bit division then, a fraction of the 64-bit one's instructions
   uint32_t f = 0;
   if (cn <= (1u << 19)) f = live ? 1u + (cnt * (NZ_M - k)) / cn : 0u;
   else f = live ? 1u + (uint32_t)(((uint64_t)cnt * (NZ_M - k)) / cn) : 0u;
-  const uint32_t sum = nz_block_sum(f, L.red);
-  // most frequent symbol, lowest index on ties (cnt <= 2^24 fits above the index byte)
-  const uint32_t key = nz_block_max(own ? ((cnt << 8) | (255u - tid)) : 0u, L.red);
-  const uint32_t imax = 255u - (key & 0xFFu);
+  // (the estimate does without what the most frequent symbol is still given)
+  uint32_t sum = f, est_bits = live ? (uint32_t)((float)cnt * (12.0f - __log2f((float)f))) + 1u : 0u;
+  nz_block_sum2(sum, est_bits, L.red);
   if (tid == imax) f += NZ_M - sum;
   if (k == 1) f = (tid == imax) ? (NZ_M - 1) : ((tid == (imax ^ 1u)) ? 1u : 0u);
-  const uint32_t est_bits = nz_block_sum(live ? (uint32_t)((float)cnt * (12.0f - __log2f((float)f))) + 1u : 0u, L.red);
 
   // exclusive prefix sum over the 256 symbols
   uint32_t incl = f;
@@ -548,23 +563,24 @@ __device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t* 
   const bool run_form = runs >= 1 && runs <= NZ_MAX_RUNS;
   const uint32_t head = run_form ? 1u + 2u * runs : 33u;
   __syncthreads();
+  uint8_t* ser = reinterpret_cast<uint8_t*>(L.ser);
   // 12-bit fields, two per three bytes
   for (uint32_t pj = tid; 2 * pj < kk; pj += blockDim.x) {
     const uint32_t a = L.cf[2 * pj];
     const bool two = 2 * pj + 1 < kk;
     const uint32_t b = two ? L.cf[2 * pj + 1] : 0u;
-    uint8_t* fp = out + head + 3 * pj;
+    uint8_t* fp = ser + head + 3 * pj;
     fp[0] = (uint8_t)(a & 0xFF);
     fp[1] = (uint8_t)((a >> 8) | ((b & 0xF) << 4));
     if (two) fp[2] = (uint8_t)(b >> 4);
   }
   if (!run_form && tid < 32) {
     const uint64_t mq = tid < 8 ? m0 : (tid < 16 ? m1 : (tid < 24 ? m2 : m3));
-    out[1 + tid] = (uint8_t)(mq >> (8 * (tid & 7)));
+    ser[1 + tid] = (uint8_t)(mq >> (8 * (tid & 7)));
   }
   if (tid == 0) {
     if (run_form) {
-      out[0] = (uint8_t)runs;
+      ser[0] = (uint8_t)runs;
       const uint64_t mm[4] = {m0, m1, m2, m3};
       const uint64_t ss[4] = {s0, s1, s2, s3};
       uint32_t r = 0;
@@ -584,17 +600,17 @@ __device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t* 
               break;
             }
           }
-          out[1 + 2 * r] = (uint8_t)(64u * w + b);
-          out[2 + 2 * r] = (uint8_t)(end - (64u * w + b) - 1u);
+          ser[1 + 2 * r] = (uint8_t)(64u * w + b);
+          ser[2 + 2 * r] = (uint8_t)(end - (64u * w + b) - 1u);
           ++r;
         }
       }
     } else {
-      out[0] = NZ_MODE_BITMAP;
+      ser[0] = NZ_MODE_BITMAP;
     }
     const uint32_t bytes = head + (12 * kk + 7) / 8;
     const uint32_t padded = (bytes + 3) & ~3u;
-    for (uint32_t b = bytes; b < padded; ++b) out[b] = 0;
+    for (uint32_t b = bytes; b < padded; ++b) ser[b] = 0;
     NzChunkInfo ci;
     ci.tab_len = padded;
     ci.pad_sym = imax;
@@ -605,45 +621,43 @@ __device__ __forceinline__ uint32_t nz_build_table(NzEncLds& L, const uint32_t* 
     L.tab_len = padded;
   }
   __syncthreads();
+  for (uint32_t i = tid; i < L.tab_len / 4; i += blockDim.x) reinterpret_cast<uint32_t*>(out)[i] = L.ser[i];
   return est_bits;
 }
 
 // ----------------------------------------------------------------------------
 // per chunk: coded or raw, and the record size of each of its segments (run by one
-// thread of the encode kernel once all segments of the chunk are coded)
+// wavefront of the encode kernel, a lane per segment, once all segments of the chunk
+// are coded)
 // ----------------------------------------------------------------------------
 __device__ __forceinline__ bool nz_chunk_finalize(uint64_t c, uint64_t n, uint32_t chunk_syms,
                                                   uint32_t seg_syms, uint32_t spc, NzChunkInfo* info,
                                                   const uint32_t* lds_words, const uint32_t* lds_state_bytes,
                                                   uint32_t tab_len, uint32_t* seg_units, uint32_t* chunk_units,
                                                   uint32_t* lds_seg_units, uint32_t* lds_chunk_total) {
+  const uint32_t k = nz_lane_id();
   const uint64_t base = c * chunk_syms;
   const uint32_t cn = (uint32_t)((n - base) < chunk_syms ? (n - base) : chunk_syms);
   const uint32_t nseg = (cn + seg_syms - 1) / seg_syms;
-  uint64_t rans_total = tab_len, raw_total = 4;
-  for (uint32_t k = 0; k < nseg; ++k) {
+  uint32_t rans = 0, raws = 0;  // bytes; a record has at most ~2^23, a chunk eight records
+  if (k < nseg) {
     const uint32_t sn = (cn - k * seg_syms) < seg_syms ? (cn - k * seg_syms) : seg_syms;
-    const uint32_t w = lds_words[k];
-    rans_total += lds_state_bytes[k] + 2 * (uint64_t)((w + 1) & ~1u);
-    raw_total += ((sn + 3) & ~3u) + (sn == nz_seg_nominal(chunk_syms, seg_syms, spc, k) ? NZ_CARRY_BYTES : 0u);
+    rans = lds_state_bytes[k] + 2u * ((lds_words[k] + 1) & ~1u);
+    raws = ((sn + 3) & ~3u) + (sn == nz_seg_nominal(chunk_syms, seg_syms, spc, k) ? NZ_CARRY_BYTES : 0u);
   }
+  const uint32_t rans_total = tab_len + __builtin_amdgcn_readlane(nz_wave_scan(rans, k), 63);
+  const uint32_t raw_total = 4u + __builtin_amdgcn_readlane(nz_wave_scan(raws, k), 63);
   const bool raw = rans_total >= raw_total;
-  info[c].raw = raw ? 1u : 0u;
-  uint32_t chunk_total = 0;  // a record has at most ~2^21 units, a chunk eight records
-  for (uint32_t k = 0; k < nseg; ++k) {
-    const uint32_t sn = (cn - k * seg_syms) < seg_syms ? (cn - k * seg_syms) : seg_syms;
-    const uint32_t w = lds_words[k];
-    uint32_t bytes;
-    if (raw)
-      bytes = (k == 0 ? 4u : 0u) + ((sn + 3) & ~3u) +
-              (sn == nz_seg_nominal(chunk_syms, seg_syms, spc, k) ? NZ_CARRY_BYTES : 0u);
-    else bytes = (k == 0 ? tab_len : 0u) + lds_state_bytes[k] + 2u * ((w + 1) & ~1u);
-    seg_units[c * spc + k] = bytes / 4;
-    lds_seg_units[k] = bytes / 4;
-    chunk_total += bytes / 4;
+  if (k < nseg) {
+    const uint32_t units = (raw ? raws + (k == 0 ? 4u : 0u) : rans + (k == 0 ? tab_len : 0u)) / 4;
+    seg_units[c * spc + k] = units;
+    lds_seg_units[k] = units;
   }
-  chunk_units[c] = chunk_total;
-  *lds_chunk_total = chunk_total;
+  if (k == 0) {
+    info[c].raw = raw ? 1u : 0u;
+    chunk_units[c] = (raw ? raw_total : rans_total) / 4;
+    *lds_chunk_total = (raw ? raw_total : rans_total) / 4;
+  }
   return raw;
 }
 
@@ -824,8 +838,9 @@ __device__ __forceinline__ void nz_write_header(uint8_t* comp, const NzGeom& g, 
 // NT threads (t = 0 .. NT-1) move the record of segment `seg` = segment k of
 // chunk c to o0, counted in 4-byte units from the start of the record area
 // (`mine` = its size in the same units; ci, sbytes, w: the chunk's info, the
-// size of the coder states, the number of words; `words`: where the words are,
-// the end of the segment's slot or a staging area in LDS).  With `whole` the
+// size of the coder states, the number of words; `table`, `states`, `words`: where the
+// record's parts are, in scratch memory or in LDS; the words at the end of the segment's
+// slot or in a staging area).  With `whole` the
 // record is not assembled from its parts but copied from there (the same record
 // in another container).  They write the segment's directory entry; those of
 // the last segment add the closing entry, the header, the container size and
@@ -835,13 +850,12 @@ template <uint32_t NT>
 __device__ __forceinline__ bool nz_move_record(const NzEncItem& it, const uint64_t seg, const uint64_t c,
                                                const uint32_t k, const uint64_t o0, const uint32_t mine,
                                                const NzChunkInfo ci, const uint32_t sbytes, const uint32_t w,
-                                               const uint16_t* words, const uint8_t* whole, const uint32_t t) {
+                                               const uint32_t* table, const uint32_t* states, const uint16_t* words,
+                                               const uint8_t* whole, const uint32_t t) {
   static_assert(NT >= NZ_TAIL_PAD, "too few threads for the closing zeros");
   const NzGeom& g = it.g;
-  const uint8_t* __restrict__ tab_ser = it.ws + it.tab_ser;
   const uint8_t* __restrict__ carry = it.ws + it.carry;
   const uint16_t* __restrict__ slots = reinterpret_cast<const uint16_t*>(it.ws + it.slots);
-  const uint32_t* __restrict__ states = reinterpret_cast<const uint32_t*>(it.ws + it.states);
   uint8_t* __restrict__ comp = it.comp;
   const uint64_t o1 = o0 + mine;
   const bool fits = o1 <= 0xFFFFFFFFull && g.rec_off + 4 * o1 + NZ_TAIL_PAD <= it.comp_cap;
@@ -885,12 +899,11 @@ __device__ __forceinline__ bool nz_move_record(const NzEncItem& it, const uint64
   }
   uint32_t off = 0;
   if (k == 0) {
-    const uint8_t* tb = tab_ser + c * NZ_TABLE_MAX_BYTES;
-    for (uint32_t i = t; i < ci.tab_len; i += NT) dst[i] = tb[i];
+    for (uint32_t i = t; i < ci.tab_len / 4; i += NT) reinterpret_cast<uint32_t*>(dst)[i] = table[i];
     off = ci.tab_len;
   }
   uint32_t* sdst = reinterpret_cast<uint32_t*>(dst + off);
-  for (uint32_t i = t; i < sbytes / 4; i += NT) sdst[i] = states[seg * (NZ_STATE_MAX_BYTES / 4) + i];
+  for (uint32_t i = t; i < sbytes / 4; i += NT) sdst[i] = states[i];
   // the words are 2-byte aligned; they are moved as dwords (two aligned loads and a
   // funnel shift when the source is off by one word; the load past the last word
   // stays inside the scratch buffer or the staging area)
@@ -1015,18 +1028,21 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 
     asm volatile("" ::"v"((uint32_t)e), "v"((uint32_t)(e >> 32)));
 #endif
   };
-  // Four groups at a time, and the loads of the next four are issued before the
-  // current four are split: eight 16-byte loads per lane in flight.
-  uint4 vn[4];  // the block after the current one
-  const auto load4 = [&](uint32_t gv) {
+  // Four groups at a time, and the loads of the next eight (short segments: four) are
+  // issued before the current four are split: twelve 16-byte loads per lane in flight.
+  // (The registers are there: the exponents of the groups in flight do not exist yet.)
+  constexpr int AHEAD = NG >= 32 ? 2 : 1;
+  uint4 vn[AHEAD][4];  // block b of four groups in vn[b % AHEAD]
+  const auto load4 = [&](uint4 (&v)[4], uint32_t gv) {
     const uint16_t* src = in + seg_base + (gv * NZ_LANES + lane) * NZ_GROUP;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const nz_u32x4 r = __builtin_nontemporal_load(reinterpret_cast<const nz_u32x4*>(src + q * NZ_GROUP_SYMS));
-      vn[q] = make_uint4(r.x, r.y, r.z, r.w);
+      v[q] = make_uint4(r.x, r.y, r.z, r.w);
     }
   };
-  if (4 <= whole) load4(0);
+  if (4 <= whole) load4(vn[0], 0);
+  if (AHEAD > 1 && 8 <= whole) load4(vn[AHEAD - 1], 4);
   nz_static_for<0, NG, 4>([&](auto g4c) {
     constexpr int g4 = decltype(g4c)::value;
     // the group number as a run-time value for all address arithmetic: with
@@ -1037,8 +1053,8 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 
     if (gv + 4 <= whole) {
       uint4 v[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = vn[q];
-      if (gv + 8 <= whole) load4(gv + 4);
+      for (int q = 0; q < 4; ++q) v[q] = vn[g4 / 4 % AHEAD][q];
+      if (gv + 4 * AHEAD + 4 <= whole) load4(vn[g4 / 4 % AHEAD], gv + 4 * AHEAD);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         if (nm.bytes)
@@ -1157,10 +1173,14 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 
   }
   NZ_PROBE_MARK(2);
   // decide coded-or-raw and size the records
-  if (tid == 0) {
-    L.raw = nz_chunk_finalize(c, n, chunk_syms, seg_syms, spc, info, L.seg_w, L.seg_sb, L.tab_len, seg_units,
-                              reinterpret_cast<uint32_t*>(it.ws + it.chunk_units), L.seg_units, &L.chunk_total);
-    L.gave_up = 0;
+  if (wave == 0) {
+    const bool raw = nz_chunk_finalize(c, n, chunk_syms, seg_syms, spc, info, L.seg_w, L.seg_sb, L.tab_len, seg_units,
+                                       reinterpret_cast<uint32_t*>(it.ws + it.chunk_units), L.seg_units,
+                                       &L.chunk_total);
+    if (lane == 0) {
+      L.raw = raw;
+      L.gave_up = 0;
+    }
   }
   __syncthreads();
   if (L.raw && has_seg) {
@@ -1334,7 +1354,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 
     ci.raw = L.raw ? 1u : 0u;
     ci.reserved = 0;
     const bool fits = nz_move_record<64>(it, seg, c, wave, o0, L.seg_units[wave], ci, L.seg_sb[wave],
-                                         cap_words - pos_end, words, nullptr, lane);
+                                         cap_words - pos_end, L.ser, L.sbuf[wave], words, nullptr, lane);
     if (from_stage && !fits) unstage();
     if (lane == 0) placed[seg] = (from_stage && fits) ? 1 : 0;
   }
@@ -1449,9 +1469,12 @@ __global__ __launch_bounds__(NZ_ENC_LONG_THREADS) void nz_encode_long_kernel(con
   }
   __threadfence_block();
   __syncthreads();
-  if (tid == 0) L.raw = nz_chunk_finalize(c, n, chunk_syms, seg_syms, spc, info, L.seg_w, L.seg_sb, L.tab_len, seg_units,
-                                          reinterpret_cast<uint32_t*>(it.ws + it.chunk_units), L.seg_units,
-                                          &L.chunk_total);
+  if (tid < 64) {
+    const bool raw = nz_chunk_finalize(c, n, chunk_syms, seg_syms, spc, info, L.seg_w, L.seg_sb, L.tab_len, seg_units,
+                                       reinterpret_cast<uint32_t*>(it.ws + it.chunk_units), L.seg_units,
+                                       &L.chunk_total);
+    if (tid == 0) L.raw = raw;
+  }
   __syncthreads();
   if (L.raw && has_seg) {
     // a chunk that does not compress: its exponent bytes take the place of the words
@@ -1536,7 +1559,9 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
   const bool in_old = it.use_placed && (it.ws + it.placed)[seg] != 0;
   const uint64_t o0 = nz_block_sum64(part, red4);
   const uint16_t* words = reinterpret_cast<const uint16_t*>(it.ws + it.slots) + seg * g.seg_syms + (g.seg_syms - w);
-  nz_move_record<256>(it, seg, c, k, o0, mine, ci, sbytes, w, words,
+  nz_move_record<256>(it, seg, c, k, o0, mine, ci, sbytes, w,
+                      reinterpret_cast<const uint32_t*>(it.ws + it.tab_ser + c * NZ_TABLE_MAX_BYTES),
+                      reinterpret_cast<const uint32_t*>(it.ws + it.states) + seg * (NZ_STATE_MAX_BYTES / 4), words,
                       in_old ? it.old_comp + g.rec_off + 4 * o0 : nullptr, tid);
 }
 
