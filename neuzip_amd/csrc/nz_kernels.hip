@@ -21,10 +21,10 @@
 
 #include "nz_format.h"
 
-#define NZ_RING_WORDS 1024u  // per-wave LDS ring of renormalisation words
+#define NZ_RING_WORDS 1024u  // per-wave LDS ring of renormalisation words (NzWaveDec) ...
 #define NZ_RING_DWORDS (NZ_RING_WORDS / 2)
-#define NZ_ONE_WORDS 512u    // the same with an 8-byte entry per word (NzWaveDecOne)
-#define NZ_ONE_BLOCK 256u    // words that ring is refilled by: the most four steps of a wavefront consume
+#define NZ_RING_WIDE 512u    // ... or of 8-byte entries prepared from them (NzWaveDecOne)
+#define NZ_RING_NARROW 256u
 
 // ----------------------------------------------------------------------------
 // element-wise split / merge arithmetic
@@ -1585,11 +1585,10 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 //                 (2 KiB); a workgroup of eight wavefronts has 48 KiB, three
 //                 share the 160 KiB of a CU
 //   NzWaveDecOne  one read, of a slot or of an entry prepared from the word: the
-//                 ring holds the entries of 512 words (4 KiB); 64 KiB, two
-//                 workgroups to a CU.  For launches of at most one workgroup per
-//                 CU (nz_one_read).
+//                 ring holds the entries of 512 words (4 KiB; 64 KiB, two
+//                 workgroups to a CU) in launches of at most one workgroup per
+//                 CU (nz_one_read), of 256 in fused products of more.
 
-#define NZ_RING_ALLOC_DWORDS(one) ((one) ? 2 * NZ_ONE_WORDS : NZ_RING_DWORDS)
 // What the table parse leaves for the slot-table fill (runs, windows, flags)
 // lies in the last slots of the table itself; those are filled last, from
 // registers.
@@ -1597,7 +1596,7 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 #define NZ_TMETA_SLOT ((uint32_t)(NZ_M - 416))  /* first slot under it; a multiple of 32 */
 static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 32 == 0, "parse results fit under the tail");
 // dynamic LDS of a decode workgroup whose chunks have up to `spc` segments
-#define NZ_DEC_LDS_BYTES(spc, one) ((size_t)(2 * NZ_M + (spc) * NZ_RING_ALLOC_DWORDS(one)) * 4)
+#define NZ_DEC_LDS_BYTES(spc, one) ((size_t)8 * (NZ_M + (spc) * ((one) ? NZ_RING_WIDE : NZ_RING_NARROW)))
 // Launches of at most one workgroup per compute unit decode with NzWaveDecOne,
 // unless their output is written with streaming stores.  The line lies where the
 // figures cross for the default chunk (eight wavefronts, 256 symbols per lane;
@@ -1892,18 +1891,15 @@ struct NzGemvWalk {
 // A wavefront's record and its ring: where the record lies, what may be loaded of it, and the
 // staging of its head.
 struct NzRecord {
-  uint32_t* ring32;       // 512 dwords (NzWaveDec) or 1024 (NzWaveDecOne)
+  uint32_t* ring32;       // at least 512 dwords
   const uint8_t* words;   // start of the record (uniform); word indices count from here
   uint32_t lim;           // largest byte offset from `words` that may be loaded: container end - 16 (uniform)
-  uint32_t ring_lds;      // LDS byte address of the ring (the same in all lanes, kept in a vector register)
   uint32_t nwords;        // 16-bit units the record holds, table and states included
   uint32_t lane;
 
   // record at comp + pos of a container of comp_bytes (pos + 16 <= comp_bytes)
   __device__ __forceinline__ void attach(const uint8_t* comp, uint64_t comp_bytes, uint64_t pos, uint32_t* ring) {
-    typedef __attribute__((address_space(3))) uint32_t lds_u32;
     ring32 = ring;
-    ring_lds = (uint32_t)(uintptr_t)((lds_u32*)ring);
     words = comp + pos;
     const uint64_t room = comp_bytes - NZ_TAIL_PAD - pos;
     lim = room < 0xFFFFFFF0ull ? (uint32_t)room : 0xFFFFFFF0u;
@@ -1914,14 +1910,10 @@ struct NzRecord {
   // are unconditional; words past the record are never consumed by a valid stream.
   __device__ __forceinline__ const uint8_t* at(uint32_t off) const { return words + (off < lim ? off : lim); }
 
-  // 16 (8) bytes of the word stream at dword index d
+  // 16 bytes of the record at dword index d
   __device__ __forceinline__ uint4 fetch(uint32_t d) const {
     const uint32_t* q = reinterpret_cast<const uint32_t*>(at(4u * d));
     return make_uint4(q[0], q[1], q[2], q[3]);
-  }
-  __device__ __forceinline__ uint2 fetch2(uint32_t d) const {
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(at(4u * d));
-    return make_uint2(q[0], q[1]);
   }
 
   // Stage the first 512 dwords of the record (table of a chunk's first record,
@@ -1935,9 +1927,13 @@ struct NzRecord {
   }
 };
 
-// Decoder state of one wavefront.
-struct NzWaveDec : NzRecord {  // the ring holds 1024 words: a window of the record
+// Decoder state of one wavefront, for dense output in launches of more than one workgroup per
+// compute unit, which are bound by memory: the ring holds 1024 words, a window of the record, and
+// the loads behind it have six groups to arrive.
+struct NzWaveDec : NzRecord {
+  static_assert(NZ_RING_DWORDS == 2 * NZ_RING_NARROW, "one size of ring in larger launches");
   const uint2* lut;
+  uint32_t ring_lds;      // LDS byte address of the ring (the same in all lanes, kept in a vector register)
   uint32_t x;             // this lane's rANS state
   uint32_t base;          // words consumed by the wave (the same in all lanes, kept in a vector register)
   uint32_t filled;        // dwords staged into the ring (multiple of 256; uniform)
@@ -1960,6 +1956,8 @@ struct NzWaveDec : NzRecord {  // the ring holds 1024 words: a window of the rec
     base = first_word;
     filled = __builtin_amdgcn_readfirstlane(filled);
     r = fetch(filled + 4 * lane);  // the 512 words behind the staged window
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    ring_lds = (uint32_t)(uintptr_t)((lds_u32*)ring32);
     // keep the three per-lane constants in vector registers of their own (an
     // instruction can name only one scalar register or literal)
     sel_keep = 0x07060504u;
@@ -2018,45 +2016,63 @@ struct NzWaveDec : NzRecord {  // the ring holds 1024 words: a window of the rec
   __device__ __forceinline__ void finish() {}  // the state is complete after every step
 };
 
-// Decoder state of one wavefront, for launches with few wavefronts per SIMD.
+// Decoder state of one wavefront, for launches that are not bound by memory: those of at most one
+// workgroup per compute unit and all fused products.
 //
-// What then bounds a step is its chain of dependent operations, not its instruction
-// count.  In the plain form the chain holds two LDS round trips: the
-// renormalisation word (its place depends on the ballot of the fresh states),
+// There a step is bound by its chain of dependent operations where few wavefronts share a
+// SIMD, and by its vector instructions where many do.  In NzWaveDec the chain holds two LDS round
+// trips: the renormalisation word (its place depends on the ballot of the fresh states),
 // then the slot entry that the state with the word shifted in selects.  But a
 // state that takes a word w becomes x << 16 | w, so its slot is w & 4095, which
 // the word alone decides, and
-//   f * ((x << 16 | w) >> 12) + bias = f * (x << 4) + (f * (w >> 12) + bias).
+//   f * ((x << 16 | w) >> 12) + bias = (f << 4) * x + (f * (w >> 12) + bias).
 // The ring therefore holds, per word, the slot entry that the word selects with
-// f * (w >> 12) already added to the bias (it is below 16 f: 16 bits), and a
-// step is ONE read: from the ring at the lane's rank where the state fell below
-// 2^16, from the slot table otherwise, then one multiply-add.  A wavefront
-// makes the entries of 256 words at a time, four per lane, with independent
-// reads; a weight's exponents take one word per six symbols or so, so that is
-// one prepared entry for six chains of half the length (a read of 8 chunks of
-// 256 symbols per lane: 29.7 us with two reads per step, 25.2 us with one).
-struct NzWaveDecOne : NzRecord {  // the ring holds 512 entries: a window of the words
+// its frequency times 16 and f * (w >> 12) added to its bias (it is below 16 f: 16 bits), and
+// a step is ONE read: from the ring at the lane's rank where the state fell below
+// 2^16, from the slot table otherwise, then one multiply-add.  Table and rings are
+// numbered through in entries of 8 bytes (a ring begins at a multiple of its size), so that
+// one select and one shift make the address.  A wavefront makes the entries of
+// RING / 2 words at a time with independent reads; a weight's exponents take one word
+// per six symbols or so.
+template <uint32_t RING>
+struct NzWaveDecOne : NzRecord {
+  static constexpr uint32_t BLOCK = RING / 2;  // words the ring is refilled by
+  static constexpr uint32_t PER_LANE = BLOCK / NZ_LANES;
+  // the wide ring is looked at every so many steps, the most its block can feed; the narrow one per group
+  static constexpr int STEPS = RING == NZ_RING_WIDE ? (int)(BLOCK / NZ_LANES) : NZ_GROUP;
+
   const uint2* lut;
-  uint32_t lut_lds;       // LDS byte address of the slot table, like ring_lds
+  uint32_t ring_at;       // number of the ring's first entry (the same in all lanes, kept in a vector register)
   uint32_t x;             // this lane's rANS state, before the word it may still have to take
-  uint32_t top;           // the state's upper bits, x << 4 with a word to take, x >> 12 without
+  uint32_t top;           // what the next frequency is multiplied with: x with a word to take, x >> 12 without
   uint32_t widx;          // index of that word
   uint2 e;                // entry of the next step
   uint32_t base;          // words consumed by the wave (the same in all lanes, kept in a vector register)
+  uint32_t used;          // the same number, as of the last look at the ring (uniform)
   uint32_t filled;        // words entered into the ring (multiple of 4; uniform)
-  uint2 r;                // 4 words per lane fetched after the previous refill
+  uint32_t r[PER_LANE / 2];  // the lane's words of the next block, fetched after the previous refill
 
-  // the entries of words first + 4 * lane ... + 3 (first a multiple of 4) into the ring
-  __device__ __forceinline__ void enter(uint32_t first, const uint2 v) {
-    const uint32_t w[4] = {v.x & 0xFFFFu, v.x >> 16, v.y & 0xFFFFu, v.y >> 16};
-    uint2 t[4];
+  __device__ __forceinline__ void fetch_block(uint32_t first) {  // (first a multiple of 4)
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(at(2 * first + 2 * PER_LANE * lane));
 #pragma unroll
-    for (int k = 0; k < 4; ++k) t[k] = lut[w[k] & (NZ_M - 1)];
+    for (uint32_t k = 0; k < PER_LANE / 2; ++k) r[k] = q[k];
+  }
+  // the entries of words first + PER_LANE * lane ... into the ring
+  __device__ __forceinline__ void enter(uint32_t first, const uint32_t (&v)[PER_LANE / 2]) {
+    uint32_t w[PER_LANE];
+    uint2 t[PER_LANE];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) t[k].y += __umul24(t[k].x, w[k] >> NZ_PROB_BITS);
-    uint4* at = reinterpret_cast<uint4*>(ring32 + 2 * ((first + 4 * lane) & (NZ_ONE_WORDS - 1)));
-    at[0] = make_uint4(t[0].x, t[0].y, t[1].x, t[1].y);
-    at[1] = make_uint4(t[2].x, t[2].y, t[3].x, t[3].y);
+    for (uint32_t k = 0; k < PER_LANE; ++k) w[k] = k & 1 ? v[k / 2] >> 16 : v[k / 2] & 0xFFFFu;
+#pragma unroll
+    for (uint32_t k = 0; k < PER_LANE; ++k) t[k] = lut[w[k] & (NZ_M - 1)];
+#pragma unroll
+    for (uint32_t k = 0; k < PER_LANE; ++k) {
+      t[k].y += __umul24(t[k].x, w[k] >> NZ_PROB_BITS);
+      t[k].x += __umul24(t[k].x, 15u);  // the symbol stays in byte 3: f << 4 has 16 bits
+    }
+    uint4* to = reinterpret_cast<uint4*>(ring32 + 2 * ((first + PER_LANE * lane) & (RING - 1)));
+#pragma unroll
+    for (uint32_t k = 0; k < PER_LANE / 2; ++k) to[k] = make_uint4(t[2 * k].x, t[2 * k].y, t[2 * k + 1].x, t[2 * k + 1].y);
   }
   __device__ __forceinline__ void lds_order() const {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -2064,37 +2080,52 @@ struct NzWaveDecOne : NzRecord {  // the ring holds 512 entries: a window of the
   }
 
   // Start decoding from state x0; the words begin `first_word` 16-bit units
-  // into the record (at most 348, so the first 512 from a multiple of 4 are staged).
+  // into the record (at most 348, so the first RING from a multiple of 4 are staged).
   __device__ __forceinline__ void start(uint32_t x0, uint32_t first_word) {
     const uint32_t from = __builtin_amdgcn_readfirstlane(first_word) & ~3u;
-    filled = from + NZ_ONE_WORDS;
-    r = fetch2(filled / 2 + 2 * lane);  // the 256 words behind the ring's
-    const uint2 a = *reinterpret_cast<const uint2*>(ring32 + from / 2 + 2 * lane);
-    const uint2 b = *reinterpret_cast<const uint2*>(ring32 + from / 2 + NZ_ONE_BLOCK / 2 + 2 * lane);
+    filled = from + RING;
+    fetch_block(filled);  // the block behind the ring's
+    uint32_t v[2][PER_LANE / 2];
+#pragma unroll
+    for (uint32_t h = 0; h < 2; ++h)
+#pragma unroll
+      for (uint32_t k = 0; k < PER_LANE / 2; ++k) v[h][k] = ring32[(from + h * BLOCK + PER_LANE * lane) / 2 + k];
     lds_order();
-    enter(from, a);
-    enter(from + NZ_ONE_BLOCK, b);
+    enter(from, v[0]);
+    enter(from + BLOCK, v[1]);
     lds_order();
-    typedef __attribute__((address_space(3))) const uint32_t lds_cu32;
-    lut_lds = (uint32_t)(uintptr_t)((lds_cu32*)reinterpret_cast<const uint32_t*>(lut));
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    ring_at = (uint32_t)(uintptr_t)((lds_u32*)ring32) / 8;
     x = x0;
     top = x0 >> NZ_PROB_BITS;
     widx = first_word;
     e = lut[x0 & (NZ_M - 1)];
-    base = first_word;
+    base = used = __builtin_amdgcn_readfirstlane(first_word);
     // keep the per-lane constants in vector registers of their own
-    asm volatile("" : "+v"(lut_lds), "+v"(ring_lds), "+v"(base));
+    asm volatile("" : "+v"(ring_at), "+v"(base));
+  }
+
+  // the block that waits in registers into the ring, the one behind it on its way
+  __device__ __forceinline__ void refill() {
+    lds_order();  // entries of words already taken are written over
+    enter(filled, r);
+    filled += BLOCK;
+    lds_order();
+    fetch_block(filled);
   }
 
   // Decode the next 8 symbols of every lane into byte 3 of ew[0..7].
   //
-  // Ring upkeep, before every four steps: they consume at most 4 * 64 = 256
-  // words.  The 256 words behind the ring's window wait in registers (`r`,
-  // fetched right after the previous refill); when no more than 256 are left
-  // ahead of `base` their entries are made and written, and the next 256 are
-  // fetched.  So at least 256 words are ahead of every four steps, the window
-  // [base, filled) never exceeds the ring's 512, and for exponent data a fetch
-  // has some three groups to arrive.
+  // Ring upkeep: when no more than BLOCK words are left ahead of `base`, so that the
+  // window [base, filled) never exceeds the ring.
+  // Wide ring: looked at before every four steps, which consume at most BLOCK words; for
+  // exponent data a fetch then has some three groups to arrive.
+  // Narrow ring: looked at once per group.  A group takes 80 words or so of exponent
+  // data; one that takes more than there are finds that out by scalar instructions in every step,
+  // and refills then.  (Where many wavefronts share a SIMD those cost next to nothing, while a refill
+  // every two steps would wait not only for its words but for the loads that the same
+  // group has issued: 173 us for the Linears of a block of width 4096, and 167 us this way.  With
+  // the wide ring and few wavefronts it is the other way round: 25.5 and 26.8 us for 8 chunks.)
   //
   // [base - 64, base) may just have been read when a refill writes over it: LDS
   // operations of a wavefront run in order, and the fences keep them so.
@@ -2103,29 +2134,27 @@ struct NzWaveDecOne : NzRecord {  // the ring holds 512 entries: a window of the
     typedef __attribute__((address_space(3))) const u32x2 lds_cu64;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      if ((j & 3) == 0) {
-        const uint32_t used = __builtin_amdgcn_readfirstlane(base);
-        if (filled - used <= NZ_ONE_BLOCK) {
-          lds_order();  // entries of words already taken are written over
-          enter(filled, r);
-          filled += NZ_ONE_BLOCK;
-          lds_order();
-          r = fetch2(filled / 2 + 2 * lane);
-        }
+      if (j % STEPS == 0) {
+        if constexpr (STEPS < NZ_GROUP) used = __builtin_amdgcn_readfirstlane(base);
+        if (filled - used <= BLOCK) refill();
       }
       x = __umul24(e.x, top) + e.y;
       ew[j] = e.x;
       const bool need = x < NZ_L;
       const uint64_t m = __ballot(need);
       widx = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
-      uint32_t rw = widx & (NZ_ONE_WORDS - 1), sl = x & (NZ_M - 1);
-      asm volatile("" : "+v"(rw), "+v"(sl));  // mask, then one shift-add (not shift, mask, add)
-      const uint32_t at_ring = (rw << 3) + ring_lds, at_lut = (sl << 3) + lut_lds;
-      const uint32_t at = need ? at_ring : at_lut;
-      const u32x2 v = *(lds_cu64*)(uintptr_t)at;
+      const uint32_t entry = need ? ((widx & (RING - 1)) | ring_at) : (x & (NZ_M - 1));
+      uint32_t addr;  // entry * 8; the numbers stay below 8192.  (The 16-bit shift runs at twice the rate.)
+      asm("v_lshlrev_b16 %0, 3, %1" : "=v"(addr) : "v"(entry));
+      const uint32_t taken = (uint32_t)__popcll(m);
+      if constexpr (STEPS == NZ_GROUP) {
+        used += taken;
+        if (__builtin_expect(used > filled, 0)) refill();
+      }
+      const u32x2 v = *(lds_cu64*)(uintptr_t)addr;
       e = make_uint2(v.x, v.y);
-      top = need ? x << 4 : x >> NZ_PROB_BITS;
-      base += (uint32_t)__popcll(m);
+      top = need ? x : x >> NZ_PROB_BITS;
+      base += taken;
     }
   }
 
@@ -2214,12 +2243,12 @@ __device__ __forceinline__ void nz_decode_chunk(
   const uint32_t whole = seg_n / NZ_GROUP_SYMS < body ? seg_n / NZ_GROUP_SYMS : body;
   const uint32_t lane_off = lane * (S + 1);
   const uint32_t last_off = whole ? (whole - 1) * NZ_LANES * (S + 1) + lane_off : 0u;
-  std::conditional_t<ONE, NzWaveDecOne, NzWaveDec> w;
+  constexpr uint32_t RING = ONE ? NZ_RING_WIDE : NZ_RING_NARROW;
+  std::conditional_t<ONE || GEMV, NzWaveDecOne<RING>, NzWaveDec> w;
   w.lut = lut;
-  w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + wk * NZ_RING_ALLOC_DWORDS(ONE));
+  w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + wk * 2 * RING);
   w.nwords = rec_all / 2;
   w.lane = lane;
-  w.filled = 0;
   uint64_t sm_next = 0, nb_next = 0;
   constexpr int MR = GEMV ? GEMV : 1;  // activation rows a lane multiplies with (GEMV: 0 = plain decode)
   // the activations of the next group are fetched a group ahead, unless that would cost the
