@@ -225,19 +225,36 @@ __device__ __forceinline__ uint32_t nz_wave_scan(uint32_t v, uint32_t lane) {
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31
   return v;
 }
-// Sum of a float over the 64 lanes, by the same moves as nz_wave_scan (a fixed
-// order of additions); every lane gets the total.
-__device__ __forceinline__ float nz_wave_sum(float v) {
-#define NZ_DPP_ADD(ctrl, rows)                                                                      \
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xF, false))
-  NZ_DPP_ADD(0x111, 0xF);
-  NZ_DPP_ADD(0x112, 0xF);
-  NZ_DPP_ADD(0x114, 0xF);
-  NZ_DPP_ADD(0x118, 0xF);
-  NZ_DPP_ADD(0x142, 0xA);
-  NZ_DPP_ADD(0x143, 0xC);
-#undef NZ_DPP_ADD
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+// Sums of MR floats over the 64 lanes, all at once: lane l gets the total of v[l / (64 / MR)].
+// The lanes that are 32, 16 and 8 apart are added first; a step that has two values left puts one
+// into each half of the lanes with its exchange (eight values: seven additions and three more
+// instead of eight times six).  Then the lanes 1, 2 and 4 apart.  The tree is the same for
+// every MR, so a value's total does not depend on how many are summed beside it.
+template <int MR>
+__device__ __forceinline__ float nz_wave_sums(const float (&v)[MR], uint32_t lane) {
+  static_assert(MR == 1 || MR == 2 || MR == 4 || MR == 8, "");
+  const auto dpp = [](float f, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), decltype(ctrl)::value, 0xF, 0xF, true));
+  };
+  constexpr int A = MR > 1 ? MR / 2 : 1, B = A > 1 ? A / 2 : 1;
+  float a[A], b[B];
+#pragma unroll
+  for (int m = 0; m < A; ++m) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[m]), __float_as_uint(v[MR > 1 ? m + A : m]), false, false);
+    a[m] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+#pragma unroll
+  for (int m = 0; m < B; ++m) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[m]), __float_as_uint(a[A > 1 ? m + B : m]), false, false);
+    b[m] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  const bool upper = lane & 8u;
+  const float own = B > 1 && upper ? b[B - 1] : b[0], other = B > 1 && !upper ? b[B - 1] : b[0];
+  float t = own + dpp(other, std::integral_constant<int, 0x128>{});  // row_ror:8
+  t += dpp(t, std::integral_constant<int, 0xB1>{});                  // quad_perm:[1,0,3,2]
+  t += dpp(t, std::integral_constant<int, 0x4E>{});                  // quad_perm:[2,3,0,1]
+  t += dpp(t, std::integral_constant<int, 0x141>{});                 // row_half_mirror: the other quad
+  return t;
 }
 
 __device__ __forceinline__ uint32_t nz_get12(const uint8_t* p, uint32_t i) {
@@ -1765,22 +1782,20 @@ __device__ __forceinline__ float nz_dot8(const uint4 w, const uint4 x, float acc
 // returns both words to zero.
 template <int MR>
 struct NzGemvWalk {
-  const uint4* xq;     // x as 8-element blocks, already offset by the lane
   NzGemv gv;
   uint64_t row;
   uint64_t seg_first, seg_end;  // elements of the tensor this wave covers
   uint32_t col;        // column of the current group's first element (uniform)
   uint32_t pending;    // groups added since the last flush (uniform)
   uint32_t seg_syms, last_syms, spc, k;  // segment lengths of a chunk, this wave's segment inside it
-  uint32_t xstride;    // 16-byte blocks between two activation rows
+  uint32_t lane_off;   // bytes from a group's first activation to this lane's
   uint64_t w_rows;     // rows of the tensor (= elements between two output rows)
   float sum[MR];
 
   __device__ __forceinline__ void start(const NzGemv& g, const NzGeom& geom, uint64_t first_elem,
                                         uint32_t seg_n, uint32_t wave_in_chunk, uint32_t lane) {
     gv = g;
-    xq = reinterpret_cast<const uint4*>(g.x) + lane;
-    xstride = g.in_features / NZ_GROUP;
+    lane_off = 16u * lane;
     w_rows = geom.n / g.in_features;
     row = first_elem / g.in_features;
     col = (uint32_t)(first_elem - row * g.in_features);
@@ -1798,13 +1813,19 @@ struct NzGemvWalk {
     return col + NZ_GROUP_SYMS == gv.in_features ? 0u : col + NZ_GROUP_SYMS;
   }
   // the lane's 8 activations of every row for the group at column c (a row that
-  // does not exist reads the last one that does)
+  // does not exist reads the last one that does): a scalar address that goes from row to row and the
+  // lane's offset.  (Addresses made of row number and stride in each lane took 14 quarter-rate
+  // multiplications per group of eight rows; addresses kept, all scalar registers there are.  Eight
+  // rows through the Linears of a block of width 4096: 305 -> 264 us, with flush() below.)
   __device__ __forceinline__ NzXq<MR> load(uint32_t c) const {
     NzXq<MR> r;
+    uint32_t rows = gv.x_rows, off = lane_off;
+    asm volatile("" : "+s"(rows), "+v"(off));  // made anew for every group; 32 bits for the offset
+    const uint8_t* p = reinterpret_cast<const uint8_t*>(gv.x + c);
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
-      const uint32_t mm = (uint32_t)m < gv.x_rows ? (uint32_t)m : gv.x_rows - 1u;
-      r.v[m] = xq[(uint64_t)mm * xstride + c / NZ_GROUP];
+      r.v[m] = *reinterpret_cast<const uint4*>(p + off);
+      p += (uint32_t)(m + 1) < rows ? 2ull * gv.in_features : 0ull;
     }
     return r;
   }
@@ -1833,46 +1854,41 @@ struct NzGemvWalk {
     if (gv.bias) v += nz_bf16_to_f32(gv.bias[row]);
     gv.y[(uint64_t)m * w_rows + row] = (uint16_t)nz_f32_to_bf16(v);
   }
+  // the row's results, one lane per activation row (for a shared row of eight activations one
+  // chain of atomics, not eight after each other)
   __device__ __forceinline__ void flush(uint32_t lane) {
-    float t[MR];
-#pragma unroll
-    for (int m = 0; m < MR; ++m) t[m] = nz_wave_sum(sum[m]);
-    if (lane == 0) {
+    const float t = nz_wave_sums<MR>(sum, lane);
+    const uint32_t m = lane / (NZ_LANES / MR);
+    if (lane % (NZ_LANES / MR) == 0 && m < gv.x_rows) {
       const uint64_t first = row * gv.in_features, last = first + gv.in_features - 1;
       if (first >= seg_first && last < seg_end) {
-#pragma unroll
-        for (int m = 0; m < MR; ++m)
-          if ((uint32_t)m < gv.x_rows) store_row(t[m], (uint32_t)m);
+        store_row(t, m);
       } else {
         // Device-scope atomics execute at the L2 in the order they are issued by
         // this lane when each one waits for the value the previous returned, so
         // no cache flush is needed: the count is issued only after the sum's old
         // value has come back, the exchanges only after the count's.
         const uint32_t expected = segments_of_row(first, last);
-#pragma unroll
-        for (int m = 0; m < MR; ++m) {
-          if ((uint32_t)m >= gv.x_rows) continue;
-          unsigned long long* slot = reinterpret_cast<unsigned long long*>(gv.acc + 2 * (row * MR + m));
-          unsigned long long r0;
-          if (fabsf(t[m]) < NZ_GEMV_PART_MAX)  // false for NaN as well
-            r0 = atomicAdd(slot, (unsigned long long)__float2ll_rn(t[m] * (float)(1ull << NZ_GEMV_FRAC_BITS)));
-          else
-            r0 = atomicOr(slot + 1, 1ull << 32);
-          uint32_t zero;  // 0, but only the hardware knows: ties the next atomic to the returned value
-          asm volatile("v_and_b32 %0, 0, %1" : "=v"(zero) : "v"((uint32_t)r0));
-          const unsigned long long before = atomicAdd(slot + 1, 1ull + zero);
-          if ((uint32_t)before + 1u == expected) {
-            const long long a = (long long)atomicExch(slot, 0ull);
-            const unsigned long long f = atomicExch(slot + 1, 0ull);
-            store_row((f >> 32) ? __uint_as_float(0x7FC00000u)
-                                : (float)((double)a * (1.0 / (double)(1ull << NZ_GEMV_FRAC_BITS))),
-                      (uint32_t)m);
-          }
+        unsigned long long* slot = reinterpret_cast<unsigned long long*>(gv.acc + 2 * (row * MR + m));
+        unsigned long long r0;
+        if (fabsf(t) < NZ_GEMV_PART_MAX)  // false for NaN as well
+          r0 = atomicAdd(slot, (unsigned long long)__float2ll_rn(t * (float)(1ull << NZ_GEMV_FRAC_BITS)));
+        else
+          r0 = atomicOr(slot + 1, 1ull << 32);
+        uint32_t zero;  // 0, but only the hardware knows: ties the next atomic to the returned value
+        asm volatile("v_and_b32 %0, 0, %1" : "=v"(zero) : "v"((uint32_t)r0));
+        const unsigned long long before = atomicAdd(slot + 1, 1ull + zero);
+        if ((uint32_t)before + 1u == expected) {
+          const long long a = (long long)atomicExch(slot, 0ull);
+          const unsigned long long f = atomicExch(slot + 1, 0ull);
+          store_row((f >> 32) ? __uint_as_float(0x7FC00000u)
+                              : (float)((double)a * (1.0 / (double)(1ull << NZ_GEMV_FRAC_BITS))),
+                    m);
         }
       }
     }
 #pragma unroll
-    for (int m = 0; m < MR; ++m) sum[m] = 0.f;
+    for (int k = 0; k < MR; ++k) sum[k] = 0.f;
     pending = 0;
   }
   // add the dot products of the current group, then step to the next group
