@@ -1589,7 +1589,7 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 // ----------------------------------------------------------------------------
 //
 // LDS: a 4096-entry slot table of 8-byte entries (32 KiB)
-//          lo = freq | symbol << 24      hi = slot - cum[symbol]
+//          lo = freq | nz_rot_exp(symbol) << 24      hi = slot - cum[symbol]
 //      (so that one v_mad_u32_u24 of lo's low 24 bits gives the next state and
 //      the symbol is a whole byte for v_perm_b32), and per wavefront a ring that
 //      slides over the segment's record and first holds the record's head
@@ -1677,21 +1677,28 @@ __device__ __forceinline__ uint64_t nz_stream_sm(const uint8_t* p) {
   else return __builtin_nontemporal_load(p);
 }
 
-// Merge 8 exponents (byte 3 of ew[j]) with the group's packed bytes into 8
+// The exponent byte as the decoder's tables hold it: rotated right by one.  An exponent lies across
+// the bytes of a bf16 value, seven bits below the sign and one above the mantissa; the rotated
+// byte, put into both bytes of the value, has all eight of them in place, so that merging
+// needs no shift.
+__device__ __forceinline__ constexpr uint32_t nz_rot_exp(uint32_t e) { return (e >> 1) | ((e & 1u) << 7); }
+__device__ __forceinline__ constexpr uint32_t nz_unrot_exp(uint32_t r) { return ((r << 1) & 0xFFu) | (r >> 7); }
+
+// Merge 8 exponents (rotated, byte 3 of ew[j]) with the group's packed bytes into 8
 // bf16 values.
 template <int S>
 __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew)[8]) {
   uint32_t o[4];
   if constexpr (S == 7) {
     // out16 = sign << 15 | exp << 7 | mant, byte b = sign << 7 | mant.  Per pair:
-    //   t = exponents at bits 7..14 and 23..30 (two v_perm bytes, one shift)
+    //   t = bytes [e0 e0 e1 e1]: exponents on bits 7..14 and 23..30
     //   u = bytes [b0 b0 b1 b1]: sign lands on bit 15 / 31, mantissa on 0..6 / 16..22
     //   out = bitfield insert of t's exponent bits into u
+    // (13.4 cycles of the vector ALU per pair; with a shift of t, 17.9)
     const uint32_t lo = (uint32_t)sm, hi = (uint32_t)(sm >> 32);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const uint32_t q = __builtin_amdgcn_perm(ew[2 * k + 1], ew[2 * k], 0x0c070c03u);
-      const uint32_t t = q << 7;
+      const uint32_t t = __builtin_amdgcn_perm(ew[2 * k + 1], ew[2 * k], 0x07070303u);
       const uint32_t w = k < 2 ? lo : hi;
       const uint32_t u = __builtin_amdgcn_perm(0u, w, (k & 1) ? 0x03030202u : 0x01010000u);
       // bitfield insert: (mask & t) | (~mask & u)
@@ -1701,8 +1708,7 @@ __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew
     // Fewer mantissa bits: the same shape.  A byte that holds an element's sign
     // in bit 7 and its mantissa bits right below goes into both bytes of the
     // element's half (sign on bit 15, mantissa from bit 6 down); what else the
-    // byte holds is masked away, and the exponents, alone in their word, are
-    // or-ed in.
+    // byte holds is masked away, and the exponents' bits are or-ed in.
     const uint32_t lo = (uint32_t)sm;
     constexpr uint32_t keep = 0x80008000u | (((0x7Fu << (7 - S)) & 0x7Fu) * 0x00010001u);
     constexpr int NV = S == 3 ? 2 : (S == 1 ? 4 : 8);
@@ -1711,8 +1717,7 @@ __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew
     for (int i = 0; i < NV; ++i) v[i] = lo << (i * (S + 1));
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const uint32_t q = __builtin_amdgcn_perm(ew[2 * k + 1], ew[2 * k], 0x0c070c03u);
-      const uint32_t t = q << 7;
+      const uint32_t t = __builtin_amdgcn_perm(ew[2 * k + 1], ew[2 * k], 0x07070303u);
       uint32_t u;
       if constexpr (S == 3) {
         // byte k holds elements 2k (high nibble) and 2k + 1
@@ -1725,7 +1730,7 @@ __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew
         // one byte holds the eight signs, element 0 in bit 7
         u = __builtin_amdgcn_perm(v[2 * k + 1], v[2 * k], 0x04040000u);
       }
-      o[k] = (u & keep) | t;
+      o[k] = (u & keep) | (t & 0x7F807F80u);
     }
   }
   return make_uint4(o[0], o[1], o[2], o[3]);
@@ -1814,8 +1819,8 @@ struct NzGemvWalk {
   }
   // the lane's 8 activations of every row for the group at column c (a row that
   // does not exist reads the last one that does): a scalar address that goes from row to row and the
-  // lane's offset.  (Addresses made of row number and stride in each lane took 14 quarter-rate
-  // multiplications per group of eight rows; addresses kept, all scalar registers there are.  Eight
+  // lane's offset.  (Addresses made of row number and stride in each lane took 30 vector
+  // instructions per group of eight rows; addresses kept, all scalar registers there are.  Eight
   // rows through the Linears of a block of width 4096: 305 -> 264 us, with flush() below.)
   __device__ __forceinline__ NzXq<MR> load(uint32_t c) const {
     NzXq<MR> r;
@@ -1981,7 +1986,7 @@ struct NzWaveDec : NzRecord {
     asm volatile("" : "+v"(sel_keep), "+v"(sel_shift), "+v"(ring_lds), "+v"(base));
   }
 
-  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7].
+  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7] (rotated, nz_rot_exp).
   //
   // Ring upkeep: the 512 words that follow the staged window wait in
   // registers (`r`, fetched right after the previous commit, addresses clamped
@@ -2130,7 +2135,7 @@ struct NzWaveDecOne : NzRecord {
     fetch_block(filled);
   }
 
-  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7].
+  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7] (rotated, nz_rot_exp).
   //
   // Ring upkeep: when no more than BLOCK words are left ahead of `base`, so that the
   // window [base, filled) never exceeds the ring.
@@ -2199,7 +2204,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   uint2* lut = reinterpret_cast<uint2*>(lds);                   // 4096 x 8 bytes
   uint32_t* rings = lds + 2 * NZ_M;                             // spc rings
   uint32_t* tmeta = lds + 2 * NZ_TMETA_SLOT;                    // what the table parse leaves for the fill:
-  uint2* runs = reinterpret_cast<uint2*>(tmeta);                //   per live symbol (freq | symbol << 24, first slot)
+  uint2* runs = reinterpret_cast<uint2*>(tmeta);                //   per live symbol (freq | rotated symbol << 24, first slot)
   uint2* wins = runs + 256;                                     //   per 32 slots (bitmap of run starts, runs before)
   uint32_t* tflag = reinterpret_cast<uint32_t*>(wins + 128);    //   [0] frequencies sum to 4096, [1] table bytes
   const uint8_t* tb = reinterpret_cast<const uint8_t*>(rings);  // table bytes: start of the first record
@@ -2358,7 +2363,7 @@ __device__ __forceinline__ void nz_decode_chunk(
 #pragma unroll
         for (uint32_t j = 0; j < 4; ++j) {
           if (fr[j]) {
-            runs[k] = make_uint2(fr[j] | ((4 * lane + j) << 24), first);
+            runs[k] = make_uint2(fr[j] | (nz_rot_exp(4 * lane + j) << 24), first);
             atomicOr(&wins[first >> 5].x, 1u << (first & 31));
             ++k;
             first += fr[j];
@@ -2447,7 +2452,7 @@ __device__ __forceinline__ void nz_decode_chunk(
         const uint64_t sm = (carry && b >= keep) ? nz_load_sm<S>(tailp + (b - keep)) : nz_load_sm<S>(pk + b);
         uint32_t ew[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ew[j] = (uint32_t)((sy >> (8 * j)) & 0xFFu) << 24;
+        for (int j = 0; j < 8; ++j) ew[j] = nz_rot_exp((uint32_t)(sy >> (8 * j)) & 0xFFu) << 24;
         uint4 mv = nz_merge_group<S>(sm, ew);
         if constexpr (NORM) mv = nz_scale8<true>(mv, nz_norm_load8(nm, seg_base + idx0), nm.log2n >= 3);
         if constexpr (GEMV) walk.add(mv, walk.load(walk.col), lane);
@@ -2557,7 +2562,7 @@ __device__ __forceinline__ void nz_decode_chunk(
         const uint32_t rp = ((uint32_t)pk[bit >> 3] >> (7u - S - (bit & 7u))) & ((2u << S) - 1u);
         uint32_t sym = 0;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) sym = (uint32_t)q == j ? (ew[q] >> 24) : sym;
+        for (int q = 0; q < 8; ++q) sym = (uint32_t)q == j ? nz_unrot_exp(ew[q] >> 24) : sym;
         uint32_t h = nz_merge_one<S>(sym, rp);
         if constexpr (NORM) h = nz_norm_mul(h, nm.bytes[(seg_base + idx0 + j) >> nm.log2n]);
         dst[idx0 + j] = (uint16_t)h;
