@@ -2512,7 +2512,7 @@ __device__ __forceinline__ void nz_decode_chunk(
     if constexpr (decltype(wide)::value) return nm.bytes[e0 >> nm.log2n];
     else return nz_norm_load8(nm, e0);
   };
-  const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide) {
+  const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide, auto fetch_ahead) {
     NzXq<MR> xq;
     if constexpr (GEMV && X_AHEAD) {
       xq = xq_next;
@@ -2520,6 +2520,7 @@ __device__ __forceinline__ void nz_decode_chunk(
     } else if constexpr (GEMV) {
       xq = walk.load(walk.col);
     }
+    fetch_ahead();  // behind the activations: their wait is then not for bytes from memory as well (eight rows: 265 -> 260 us)
     uint32_t ew[8];
     w.group(ew);
     // the merge starts only here: its wait for the packed bytes must not be
@@ -2534,20 +2535,20 @@ __device__ __forceinline__ void nz_decode_chunk(
   };
   const auto full_groups = [&](auto wide) {
     uint64_t sm_a = sm_next, sm_b = 0, nb_a = nb_next, nb_b = 0;
-    if (whole > 1) {
-      sm_b = sm_at(1);
-      if constexpr (NORM) nb_b = nb_at(1, wide);
-    }
     uint32_t gq = 0;
-    for (; gq + 1 < whole; gq += 2) {
-      full_group(gq, sm_a, nb_a, wide);
+    const auto fetch_a = [&] {
       sm_a = sm_at(gq + 2);
       if constexpr (NORM) nb_a = nb_at(gq + 2, wide);
-      full_group(gq + 1, sm_b, nb_b, wide);
-      sm_b = sm_at(gq + 3);
-      if constexpr (NORM) nb_b = nb_at(gq + 3, wide);
+    };
+    const auto fetch_b = [&] {
+      sm_b = sm_at(gq + 1);
+      if constexpr (NORM) nb_b = nb_at(gq + 1, wide);
+    };
+    for (; gq + 1 < whole; gq += 2) {
+      full_group(gq, sm_a, nb_a, wide, fetch_b);
+      full_group(gq + 1, sm_b, nb_b, wide, fetch_a);
     }
-    if (gq < whole) full_group(gq, sm_a, nb_a, wide);
+    if (gq < whole) full_group(gq, sm_a, nb_a, wide, [] {});
   };
   if (!NORM || nm.log2n >= 3) full_groups(NzConst<1>{});
   else full_groups(NzConst<0>{});
