@@ -1326,8 +1326,6 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
   b.in_features = in_features;
   b.x_rows = x_rows;
   b.log2n = log2_of(m->normalizer ? m->normalizer : 1);
-  // accumulator pairs per row of a matrix: as many as the kernel that serves x_rows holds per lane
-  const uint32_t mr = x_rows <= 1 ? 1u : x_rows <= 2 ? 2u : x_rows <= 4 ? 4u : 8u;
   uint64_t grid = 0, rows = 0;
   uint32_t max_spc = 1;
   {
@@ -1338,7 +1336,7 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
       auto it = m->entries.find(names[i]);
       if (it == m->entries.end()) return fail(NZ_ERR_NOT_FOUND, "Data not found");
       blocks = blocks || it->second.pending >= 0;
-      want_rows += it->second.n / in_features * mr;
+      want_rows += it->second.n / in_features * x_rows;  // an accumulator pair per row and activation row
     }
     if (int rc = refuse_under_capture(st, blocks || m->gemv_rows < want_rows, "gemv_batch")) return rc;
     if (int rc = order_scratch_use(m, st)) return rc;
@@ -1365,7 +1363,7 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
     bi.bias = dev_bias ? (const uint16_t*)dev_bias[i] : nullptr;
     bi.y = (uint16_t*)dev_y[i];
     bi.reserved = (uint32_t)rows;  // first accumulator pair, turned into a pointer below
-    rows += ent.n / in_features * mr;
+    rows += ent.n / in_features * x_rows;
     if (grid > 0x7FFFFFFFull || rows > 0x7FFFFFFFull) return fail(NZ_ERR_ARG, "batch too large");
   }
   if (m->gemv_rows < rows) {

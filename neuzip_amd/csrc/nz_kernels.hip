@@ -225,22 +225,27 @@ __device__ __forceinline__ uint32_t nz_wave_scan(uint32_t v, uint32_t lane) {
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31
   return v;
 }
-// Sums of MR floats over the 64 lanes, all at once: lane l gets the total of v[l / (64 / MR)].
+// the next power of two
+__device__ __forceinline__ constexpr uint32_t nz_pow2(uint32_t v) { return v <= 1 ? 1u : v <= 2 ? 2u : v <= 4 ? 4u : 8u; }
+
+// Sums of MR (up to 8) floats over the 64 lanes, all at once: with P the next power of two, lane l
+// gets the total of v[l / (64 / P)], where there is one.
 // The lanes that are 32, 16 and 8 apart are added first; a step that has two values left puts one
 // into each half of the lanes with its exchange (eight values: seven additions and three more
 // instead of eight times six).  Then the lanes 1, 2 and 4 apart.  The tree is the same for
 // every MR, so a value's total does not depend on how many are summed beside it.
 template <int MR>
 __device__ __forceinline__ float nz_wave_sums(const float (&v)[MR], uint32_t lane) {
-  static_assert(MR == 1 || MR == 2 || MR == 4 || MR == 8, "");
+  static_assert(MR >= 1 && MR <= 8, "");
   const auto dpp = [](float f, auto ctrl) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), decltype(ctrl)::value, 0xF, 0xF, true));
   };
-  constexpr int A = MR > 1 ? MR / 2 : 1, B = A > 1 ? A / 2 : 1;
+  constexpr int P = nz_pow2(MR), A = P > 1 ? P / 2 : 1, B = A > 1 ? A / 2 : 1;
+  const auto bits = [&](int m) { return m < MR ? __float_as_uint(v[m]) : 0u; };
   float a[A], b[B];
 #pragma unroll
   for (int m = 0; m < A; ++m) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[m]), __float_as_uint(v[MR > 1 ? m + A : m]), false, false);
+    const auto r = __builtin_amdgcn_permlane32_swap(bits(m), bits(P > 1 ? m + A : m), false, false);
     a[m] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
   }
 #pragma unroll
@@ -1751,12 +1756,11 @@ __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew
 #define NZ_GEMV_PART_MAX 262144.0f /* 2^18 */
 
 struct NzGemv {
-  const uint16_t* x;      // x_rows activation rows of in_features bf16 values each, 16-byte aligned
+  const uint16_t* x;      // as many activation rows as the kernel is for, in_features bf16 values each, 16-byte aligned
   long long* acc;         // two words per row of this tensor and activation row (sum | count and flag), all zero between calls
-  uint16_t* y;            // x_rows rows of one bf16 per row of the tensor
+  uint16_t* y;            // for each activation row one bf16 per row of the tensor
   const uint16_t* bias;   // one bf16 per row of the tensor, or null
   uint32_t in_features;   // multiple of 512
-  uint32_t x_rows;        // activation rows that exist (1 .. the kernel's MR); the others are neither read nor written
 };
 
 // what a lane holds of the activation rows for one group of 8 weights
@@ -1817,20 +1821,19 @@ struct NzGemvWalk {
   __device__ __forceinline__ uint32_t next_col() const {
     return col + NZ_GROUP_SYMS == gv.in_features ? 0u : col + NZ_GROUP_SYMS;
   }
-  // the lane's 8 activations of every row for the group at column c (a row that
-  // does not exist reads the last one that does): a scalar address that goes from row to row and the
-  // lane's offset.  (Addresses made of row number and stride in each lane took 30 vector
+  // the lane's 8 activations of every row for the group at column c: a scalar address that goes
+  // from row to row and the lane's offset.  (Addresses made of row number and stride in each lane took 30 vector
   // instructions per group of eight rows; addresses kept, all scalar registers there are.  Eight
   // rows through the Linears of a block of width 4096: 305 -> 264 us, with flush() below.)
   __device__ __forceinline__ NzXq<MR> load(uint32_t c) const {
     NzXq<MR> r;
-    uint32_t rows = gv.x_rows, off = lane_off;
-    asm volatile("" : "+s"(rows), "+v"(off));  // made anew for every group; 32 bits for the offset
+    uint32_t stride = 2 * gv.in_features, off = lane_off;
+    asm volatile("" : "+s"(stride), "+v"(off));  // made anew for every group; 32 bits for the offset
     const uint8_t* p = reinterpret_cast<const uint8_t*>(gv.x + c);
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
       r.v[m] = *reinterpret_cast<const uint4*>(p + off);
-      p += (uint32_t)(m + 1) < rows ? 2ull * gv.in_features : 0ull;
+      p += stride;
     }
     return r;
   }
@@ -1863,8 +1866,9 @@ struct NzGemvWalk {
   // chain of atomics, not eight after each other)
   __device__ __forceinline__ void flush(uint32_t lane) {
     const float t = nz_wave_sums<MR>(sum, lane);
-    const uint32_t m = lane / (NZ_LANES / MR);
-    if (lane % (NZ_LANES / MR) == 0 && m < gv.x_rows) {
+    constexpr uint32_t PER = NZ_LANES / nz_pow2(MR);
+    const uint32_t m = lane / PER;
+    if (lane % PER == 0 && m < MR) {
       const uint64_t first = row * gv.in_features, last = first + gv.in_features - 1;
       if (first >= seg_first && last < seg_end) {
         store_row(t, m);
@@ -2274,7 +2278,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   constexpr int MR = GEMV ? GEMV : 1;  // activation rows a lane multiplies with (GEMV: 0 = plain decode)
   // the activations of the next group are fetched a group ahead, unless that would cost the
   // registers of a whole workgroup per compute unit (eight rows: 32 registers)
-  constexpr bool X_AHEAD = MR < 8;
+  constexpr bool X_AHEAD = MR <= 4;
   NzXq<X_AHEAD ? MR : 1> xq_next{};
   NzGemvWalk<MR> walk;
   if (has_seg && !bad_rec) {
@@ -2650,8 +2654,8 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_ke
                                           blockIdx.x - first, NzGemv{}, NzNorm{it.norm, b.log2n});
 }
 
-// The same walk over several matrices that multiply one activation row, or up
-// to MR of them (each decoded weight is then used MR times before it is dropped).
+// The same walk over several matrices that multiply MR activation rows (each
+// decoded weight is used MR times before it is dropped).
 template <int S, bool NORM, int MR, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
@@ -2661,7 +2665,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_ker
     ++t;
   }
   const NzBatchItem& it = b.item[t];
-  const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features, b.x_rows};
+  const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features};
   nz_decode_chunk<S, MR, NORM, false, ONE>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
                                         blockIdx.x - first, gv, NzNorm{it.norm, b.log2n});
 }

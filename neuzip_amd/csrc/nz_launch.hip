@@ -78,13 +78,21 @@ template <int S, bool ONE>
 void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
   const size_t lds = NZ_DEC_LDS_BYTES(max_spc, ONE);
   const dim3 gd(grid), bd(64 * max_spc);
-  // one activation row, or kernels that hold 2, 4 or 8 of them per lane (tensors with
-  // normalizers: one row only, the caller has checked)
-  if (b.item[0].norm) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, true, 1, ONE>), gd, bd, lds, st, b, d_status);
-  else if (b.x_rows <= 1) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 1, ONE>), gd, bd, lds, st, b, d_status);
-  else if (b.x_rows <= 2) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 2, ONE>), gd, bd, lds, st, b, d_status);
-  else if (b.x_rows <= 4) hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 4, ONE>), gd, bd, lds, st, b, d_status);
-  else hipLaunchKernelGGL((nz_decode_gemv_kernel<S, false, 8, ONE>), gd, bd, lds, st, b, d_status);
+#define NZ_GEMV_LAUNCH(NORM, MR) \
+  hipLaunchKernelGGL((nz_decode_gemv_kernel<S, NORM, MR, ONE>), gd, bd, lds, st, b, d_status)
+  // a kernel for every number of activation rows
+  if (b.item[0].norm) NZ_GEMV_LAUNCH(true, 1);  // (tensors with normalizers: one row only, the caller has checked)
+  else switch (b.x_rows) {
+    case 1: NZ_GEMV_LAUNCH(false, 1); break;
+    case 2: NZ_GEMV_LAUNCH(false, 2); break;
+    case 3: NZ_GEMV_LAUNCH(false, 3); break;
+    case 4: NZ_GEMV_LAUNCH(false, 4); break;
+    case 5: NZ_GEMV_LAUNCH(false, 5); break;
+    case 6: NZ_GEMV_LAUNCH(false, 6); break;
+    case 7: NZ_GEMV_LAUNCH(false, 7); break;
+    default: NZ_GEMV_LAUNCH(false, 8); break;
+  }
+#undef NZ_GEMV_LAUNCH
 }
 
 template <int S>

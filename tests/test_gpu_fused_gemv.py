@@ -588,3 +588,10 @@ def test_backward_of_compressed_linears_takes_weights_decoded_ahead():
     assert mgr_b._be.ahead_stats() == (0, 0)
     mgr_a._be.check()
     mgr_b._be.check()
+
+
+@pytest.mark.parametrize("m_rows,s", [(6, 7), (7, 7), (6, 1), (7, 0), (3, 0)])
+def test_every_number_of_rows_has_its_kernel(m_rows, s):
+    """Numbers of rows between the powers of two, the other precisions among them: same
+    bits as the one-row calls."""
+    test_several_activation_rows_equal_the_one_row_calls(m_rows, s)
