@@ -1990,9 +1990,7 @@ struct NzWaveDec : NzRecord {
     asm volatile("" : "+v"(sel_keep), "+v"(sel_shift), "+v"(ring_lds), "+v"(base));
   }
 
-  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7] (rotated, nz_rot_exp).
-  //
-  // Ring upkeep: the 512 words that follow the staged window wait in
+  // Ring upkeep, before every group: the 512 words that follow the staged window wait in
   // registers (`r`, fetched right after the previous commit, addresses clamped
   // to the container); at the start of a group they are committed to the ring
   // if no more than 512 words are still ahead of `base`, and the next 512 are
@@ -2000,6 +1998,18 @@ struct NzWaveDec : NzRecord {
   // words are ahead at every group start, the window [base, filled) never
   // exceeds the 1024 ring words, and a fetch has at least one group (for
   // exponent data about six) to arrive before its commit.
+  __device__ __forceinline__ void look() {
+    const uint32_t ahead = __builtin_amdgcn_readfirstlane(base);
+    if ((2 * filled - ahead) <= 512u) {
+      commit(filled + 4 * lane, r);
+      filled += 256;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      r = fetch(filled + 4 * lane);
+    }
+  }
+
+  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7] (rotated, nz_rot_exp).
   //
   // A step issues: slot read, multiply-add, compare, the lane's word index
   // (words consumed by the wave + its rank among the lanes that renormalise:
@@ -2009,14 +2019,6 @@ struct NzWaveDec : NzRecord {
   // popcount.  No execution-mask changes and three scalar instructions per
   // step (popcount and the two waits).
   __device__ __forceinline__ void group(uint32_t (&ew)[8]) {
-    const uint32_t ahead = __builtin_amdgcn_readfirstlane(base);
-    if ((2 * filled - ahead) <= 512u) {
-      commit(filled + 4 * lane, r);
-      filled += 256;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      r = fetch(filled + 4 * lane);
-    }
     typedef __attribute__((address_space(3))) const uint16_t lds_cu16;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -2139,11 +2141,9 @@ struct NzWaveDecOne : NzRecord {
     fetch_block(filled);
   }
 
-  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7] (rotated, nz_rot_exp).
-  //
-  // Ring upkeep: when no more than BLOCK words are left ahead of `base`, so that the
+  // Ring upkeep, before every group: when no more than BLOCK words are left ahead of `base`, so that the
   // window [base, filled) never exceeds the ring.
-  // Wide ring: looked at before every four steps, which consume at most BLOCK words; for
+  // Wide ring: looked at again inside a group, before every four steps, which consume at most BLOCK words; for
   // exponent data a fetch then has some three groups to arrive.
   // Narrow ring: looked at once per group.  A group takes 80 words or so of exponent
   // data; one that takes more than there are finds that out by scalar instructions in every step,
@@ -2154,15 +2154,23 @@ struct NzWaveDecOne : NzRecord {
   //
   // [base - 64, base) may just have been read when a refill writes over it: LDS
   // operations of a wavefront run in order, and the fences keep them so.
+  //
+  // The look before a group comes ahead of the group's loads: a refill waits for its words, and,
+  // because loads return in order and their number differs from way to way, for every other load
+  // under way, those from memory too.  (Four rows through the Linears of a block of width
+  // 4096: 191 -> 188 us; read of 5003 x 3001, precision 3, normalizers: 32.3 -> 31.4 us.)
+  __device__ __forceinline__ void look() {
+    if constexpr (STEPS < NZ_GROUP) used = __builtin_amdgcn_readfirstlane(base);
+    if (filled - used <= BLOCK) refill();
+  }
+
+  // Decode the next 8 symbols of every lane into byte 3 of ew[0..7] (rotated, nz_rot_exp).
   __device__ __forceinline__ void group(uint32_t (&ew)[8]) {
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     typedef __attribute__((address_space(3))) const u32x2 lds_cu64;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      if (j % STEPS == 0) {
-        if constexpr (STEPS < NZ_GROUP) used = __builtin_amdgcn_readfirstlane(base);
-        if (filled - used <= BLOCK) refill();
-      }
+      if (j % STEPS == 0 && j) look();
       x = __umul24(e.x, top) + e.y;
       ew[j] = e.x;
       const bool need = x < NZ_L;
@@ -2276,9 +2284,11 @@ __device__ __forceinline__ void nz_decode_chunk(
   w.lane = lane;
   uint64_t sm_next = 0, nb_next = 0;
   constexpr int MR = GEMV ? GEMV : 1;  // activation rows a lane multiplies with (GEMV: 0 = plain decode)
-  // the activations of the next group are fetched a group ahead, unless that would cost the
-  // registers of a whole workgroup per compute unit (eight rows: 32 registers)
-  constexpr bool X_AHEAD = MR <= 4;
+  // The activation of the next group is fetched a group ahead.  Of several rows it is this
+  // group's: the registers of the next ones' cost a workgroup per compute unit where there would
+  // be three, and gain nothing where there are two (four rows through the Linears of a block of
+  // width 4096: 188 us ahead, 185 us not; eight: 255 and 256 us).
+  constexpr bool X_AHEAD = MR == 1;
   NzXq<X_AHEAD ? MR : 1> xq_next{};
   NzGemvWalk<MR> walk;
   if (has_seg && !bad_rec) {
@@ -2517,6 +2527,7 @@ __device__ __forceinline__ void nz_decode_chunk(
     else return nz_norm_load8(nm, e0);
   };
   const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide, auto fetch_ahead) {
+    if constexpr (ONE || GEMV) w.look();  // before the group's loads: a refill waits for all that are under way
     NzXq<MR> xq;
     if constexpr (GEMV && X_AHEAD) {
       xq = xq_next;
@@ -2525,6 +2536,7 @@ __device__ __forceinline__ void nz_decode_chunk(
       xq = walk.load(walk.col);
     }
     fetch_ahead();  // behind the activations: their wait is then not for bytes from memory as well (eight rows: 265 -> 260 us)
+    if constexpr (!ONE && !GEMV) w.look();  // (behind them here: 143 us for 8192 x 28672, before them 145)
     uint32_t ew[8];
     w.group(ew);
     // the merge starts only here: its wait for the packed bytes must not be
@@ -2559,6 +2571,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   if (!GEMV && whole < body) {  // the ragged last group of the tensor
     const uint32_t idx0 = (whole * NZ_LANES + lane) * NZ_GROUP;
     uint32_t ew[8];
+    w.look();
     w.group(ew);
     if (idx0 < seg_n) {
       const uint32_t rem = seg_n - idx0 < 8 ? seg_n - idx0 : 8;
@@ -2577,7 +2590,10 @@ __device__ __forceinline__ void nz_decode_chunk(
   uint32_t ext[2][8];
 #pragma unroll
   for (uint32_t t = 0; t < 2; ++t)
-    if (t < tailg) w.group(ext[t]);
+    if (t < tailg) {
+      w.look();
+      w.group(ext[t]);
+    }
 
   // every lane must be back at the encoder's start state (2^16 | carried bits)
   // and the wave must not have read past its record
