@@ -1619,6 +1619,11 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 32 == 0, "parse results fit under the tail");
 // dynamic LDS of a decode workgroup whose chunks have up to `spc` segments
 #define NZ_DEC_LDS_BYTES(spc, one) ((size_t)8 * (NZ_M + (spc) * ((one) ? NZ_RING_WIDE : NZ_RING_NARROW)))
+// Fused products of that many rows stage activations behind the rings, in launches of more than one
+// workgroup per compute unit (two groups' worth; 64 KiB in all for eight rows and eight segments).
+#define NZ_STAGED_ROWS 6
+#define NZ_GEMV_LDS_BYTES(spc, one, rows) \
+  (NZ_DEC_LDS_BYTES(spc, one) + (!(one) && (rows) >= NZ_STAGED_ROWS ? (size_t)2048 * (rows) : 0))
 // Launches of at most one workgroup per compute unit decode with NzWaveDecOne,
 // unless their output is written with streaming stores.  The line lies where the
 // figures cross for the default chunk (eight wavefronts, 256 symbols per lane;
@@ -1763,6 +1768,8 @@ struct NzGemv {
   uint32_t in_features;   // multiple of 512
 };
 
+struct NzNoLds {};  // the activations of a group are not in LDS
+
 // what a lane holds of the activation rows for one group of 8 weights
 template <int MR>
 struct NzXq {
@@ -1904,6 +1911,15 @@ struct NzGemvWalk {
   __device__ __forceinline__ void add(const uint4 w, const NzXq<MR>& x, uint32_t lane) {
 #pragma unroll
     for (int m = 0; m < MR; ++m) sum[m] = nz_dot8(w, x.v[m], sum[m]);
+    next(lane);
+  }
+  // the same with the group's activations in LDS, 64 x 16 bytes per row
+  __device__ __forceinline__ void add(const uint4 w, const uint4* x, uint32_t lane) {
+#pragma unroll
+    for (int m = 0; m < MR; ++m) sum[m] = nz_dot8(w, x[NZ_LANES * m + lane], sum[m]);
+    next(lane);
+  }
+  __device__ __forceinline__ void next(uint32_t lane) {
     ++pending;
     col = next_col();
     if (col == 0) {
@@ -2526,13 +2542,16 @@ __device__ __forceinline__ void nz_decode_chunk(
     if constexpr (decltype(wide)::value) return nm.bytes[e0 >> nm.log2n];
     else return nz_norm_load8(nm, e0);
   };
-  const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide, auto fetch_ahead) {
+  // (`xl`: the group's activations in LDS, or NzNoLds)
+  const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide, auto fetch_ahead,
+                              auto xl) __attribute__((always_inline)) {
+    constexpr bool X_LDS = !std::is_same_v<decltype(xl), NzNoLds>;
     if constexpr (ONE || GEMV) w.look();  // before the group's loads: a refill waits for all that are under way
     NzXq<MR> xq;
     if constexpr (GEMV && X_AHEAD) {
       xq = xq_next;
       xq_next = walk.load(walk.next_col());  // always inside x
-    } else if constexpr (GEMV) {
+    } else if constexpr (GEMV && !X_LDS) {
       xq = walk.load(walk.col);
     }
     fetch_ahead();  // behind the activations: their wait is then not for bytes from memory as well (eight rows: 265 -> 260 us)
@@ -2545,11 +2564,12 @@ __device__ __forceinline__ void nz_decode_chunk(
     asm volatile("" : "+v"(sml), "+v"(smh), "+v"(ew[7]));
     uint4 mv = nz_merge_group<S>(((uint64_t)smh << 32) | sml, ew);
     if constexpr (NORM) mv = nz_scale8<true>(mv, nb, decltype(wide)::value);
-    if constexpr (GEMV) walk.add(mv, xq, lane);
+    if constexpr (X_LDS) walk.add(mv, xl, lane);
+    else if constexpr (GEMV) walk.add(mv, xq, lane);
     else if constexpr (STREAM) nz_stream_store(dst + (gq * NZ_LANES + lane) * NZ_GROUP, mv);
     else *reinterpret_cast<uint4*>(dst + (gq * NZ_LANES + lane) * NZ_GROUP) = mv;
   };
-  const auto full_groups = [&](auto wide) {
+  const auto full_groups = [&](auto wide) __attribute__((always_inline)) {
     uint64_t sm_a = sm_next, sm_b = 0, nb_a = nb_next, nb_b = 0;
     uint32_t gq = 0;
     const auto fetch_a = [&] {
@@ -2560,11 +2580,52 @@ __device__ __forceinline__ void nz_decode_chunk(
       sm_b = sm_at(gq + 1);
       if constexpr (NORM) nb_b = nb_at(gq + 1, wide);
     };
-    for (; gq + 1 < whole; gq += 2) {
-      full_group(gq, sm_a, nb_a, wide, fetch_b);
-      full_group(gq + 1, sm_b, nb_b, wide, fetch_a);
+    if constexpr (GEMV >= NZ_STAGED_ROWS && !ONE && !NORM) {
+      // Where all segments of the chunk begin a row of the matrix and have the same length, its
+      // wavefronts are at the same column all the time.  Each of the first MR then brings one
+      // activation row's part of the next group into LDS (two buffers, one barrier per group; wavefronts
+      // without a segment, or with a damaged one, have ended and are not waited for).
+      //
+      // Every wavefront by itself reads MR KiB per group, and beside a wavefront at another
+      // column the vector L1 (32 KiB) holds too little of them: with all rows at one address
+      // eight rows through the Linears of a block of width 4096 took 192 us, not 256.  Staged
+      // (gate and up projection; the others keep the loads): six, seven and eight rows
+      // 222, 239, 256 -> 219, 229, 242 us.  Up to five rows a third workgroup per compute unit
+      // is worth more than that; launches of one workgroup lose 6 to 9 us to the barriers.
+      if (g.seg_syms % gv.in_features == 0 && g.chunk_syms == g.spc * g.seg_syms && cn == g.chunk_syms &&
+          g.spc >= (uint32_t)GEMV) {
+        constexpr uint32_t GROUP_X = NZ_LANES * GEMV;  // 16-byte units of a group
+        uint4* const xbuf = reinterpret_cast<uint4*>(rings + 2 * RING * g.spc);
+        const bool mine = wave < (uint32_t)GEMV;
+        const uint16_t* const xrow = gv.x + (uint64_t)(mine ? wave : 0u) * gv.in_features + NZ_GROUP * lane;
+        uint4 xs = *reinterpret_cast<const uint4*>(xrow + walk.col);
+        const auto put_x = [&](uint32_t buffer) __attribute__((always_inline)) {
+          if (mine) xbuf[buffer * GROUP_X + NZ_LANES * wave + lane] = xs;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        };
+        const auto fetch_x = [&]() __attribute__((always_inline)) {  // always inside x
+          xs = *reinterpret_cast<const uint4*>(xrow + walk.next_col());
+        };
+        put_x(0);
+        for (; gq + 1 < whole; gq += 2) {
+          fetch_x();
+          full_group(gq, sm_a, nb_a, wide, fetch_b, (const uint4*)xbuf);
+          put_x(1);
+          fetch_x();
+          full_group(gq + 1, sm_b, nb_b, wide, fetch_a, (const uint4*)xbuf + GROUP_X);
+          put_x(0);
+        }
+        if (gq < whole) full_group(gq, sm_a, nb_a, wide, [] {}, (const uint4*)xbuf);
+        return;
+      }
     }
-    if (gq < whole) full_group(gq, sm_a, nb_a, wide, [] {});
+    for (; gq + 1 < whole; gq += 2) {
+      full_group(gq, sm_a, nb_a, wide, fetch_b, NzNoLds{});
+      full_group(gq + 1, sm_b, nb_b, wide, fetch_a, NzNoLds{});
+    }
+    if (gq < whole) full_group(gq, sm_a, nb_a, wide, [] {}, NzNoLds{});
   };
   if (!NORM || nm.log2n >= 3) full_groups(NzConst<1>{});
   else full_groups(NzConst<0>{});

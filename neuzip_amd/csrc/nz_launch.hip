@@ -76,7 +76,7 @@ void nz_launch_decode_batch(const NzBatch& b, uint32_t grid, uint32_t max_spc, b
 
 template <int S, bool ONE>
 void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
-  const size_t lds = NZ_DEC_LDS_BYTES(max_spc, ONE);
+  const size_t lds = NZ_GEMV_LDS_BYTES(max_spc, ONE, b.x_rows);
   const dim3 gd(grid), bd(64 * max_spc);
 #define NZ_GEMV_LAUNCH(NORM, MR) \
   hipLaunchKernelGGL((nz_decode_gemv_kernel<S, NORM, MR, ONE>), gd, bd, lds, st, b, d_status)

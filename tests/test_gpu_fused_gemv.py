@@ -595,3 +595,32 @@ def test_every_number_of_rows_has_its_kernel(m_rows, s):
     """Numbers of rows between the powers of two, the other precisions among them: same
     bits as the one-row calls."""
     test_several_activation_rows_equal_the_one_row_calls(m_rows, s)
+
+
+@pytest.mark.parametrize("m_rows,s", [(6, 7), (7, 3), (8, 7), (8, 0)])
+@pytest.mark.parametrize("rows,cols,chunk,lane", [
+    (1030, 4096, 131072, 256),   # chunks of 32 rows and a short one; 33 workgroups are the other form ...
+    (9000, 4096, 131072, 256),   # ... 282 are the staged one, the last chunk ragged
+    (35000, 1024, 131072, 256),  # 16 rows per segment, an odd number of whole groups
+    (70000, 512, 131072, 256),   # one group per row: the next column is the first
+    (9100, 4096, 135168, 264),   # segments that do not begin a row
+    (17000, 2048, 114688, 256),  # seven segments per chunk: staged for up to seven rows
+    (1100, 16384, 65536, 256),   # a row per segment, four segments: not staged
+])
+def test_activations_staged_in_lds(rows, cols, chunk, lane, m_rows, s):
+    """Chunks whose segments all begin a row take the activations of six to eight rows from
+    LDS, the others from memory: same bits as the one-row calls on both sides of the rule."""
+    import neuzip_amd
+
+    mgr = neuzip_amd.Manager(precision=s, chunk_size=chunk, lane_symbols=lane)
+    g = torch.Generator(device="cuda").manual_seed(rows + m_rows)
+    h = mgr.write((torch.randn(rows, cols, device="cuda", generator=g) * 0.02).to(torch.bfloat16))
+    x = torch.randn(m_rows, cols, device="cuda", generator=g).to(torch.bfloat16)
+    print(f"case {rows}x{cols} chunk={chunk} lane={lane} rows={m_rows} s={s}", flush=True)
+    out = torch.full((m_rows, rows), 7.0, dtype=torch.bfloat16, device="cuda")
+    mgr._be.gemv_batch((ctypes.c_char_p * 1)(h.encode()), x, [None], [out], m_rows)
+    for m in range(m_rows):
+        (one,) = _gemv(mgr, [h], x[m].contiguous(), [None])
+        assert torch.equal(one.view(torch.int16), out[m].view(torch.int16)), m
+    want = x.double() @ mgr.read(h).double().t()
+    assert ((out.double() - want).norm() / want.norm()).item() < 2.0 ** -8  # a bf16 rounding of each result
