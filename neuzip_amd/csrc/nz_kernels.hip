@@ -1624,20 +1624,21 @@ static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 3
 #define NZ_STAGED_ROWS 6
 #define NZ_GEMV_LDS_BYTES(spc, one, rows) \
   (NZ_DEC_LDS_BYTES(spc, one) + (!(one) && (rows) >= NZ_STAGED_ROWS ? (size_t)2048 * (rows) : 0))
-// Launches of at most one workgroup per compute unit decode with NzWaveDecOne,
-// unless their output is written with streaming stores.  The line lies where the
-// figures cross for the default chunk (eight wavefronts, 256 symbols per lane;
-// MI355X, 256 compute units; two-read against one-read step, microseconds):
+// Launches of at most one workgroup per compute unit decode with NzWaveDecOne and its
+// wide ring, unless their output is written with streaming stores.  (Fused products of more
+// workgroups take it too, with the narrow ring and in any case: the two-read step took
+// 184.5 us for the one-row products of a block of width 4096, this one 168.2.)  The line lies
+// where the figures of dense output crossed for the default chunk (eight wavefronts, 256 symbols
+// per lane; MI355X, 256 compute units; two-read against one-read step, microseconds, taken when
+// the one-read step was some 5 % longer than it is):
 //   read     8 workgroups 29.7 / 25.2, 128: 33.6 / 29.7, 256: 34.6 / 31.7,
 //            257: 40.7 / 40.7, 320: 41.2 / 41.2, 512: 42.9 / 44.4, 768: 62.6 / 67.1
-//   product  1 row   256: 34.0 / 29.4, 320: 42.0 / 41.6, 448: 42.2 / 41.9, 896: 72.6 / 77.5
-//            8 rows  256: 42.0 / 39.2, 320: 64.5 / 63.2, 448: 65.9 / 64.3, 896: 121.0 / 118.7
 //   gather   1 row 32.5 / 27.8, 256 rows 40.5 / 38.1, 320 rows 48.2 / 47.8, 512 rows 52.4 / 53.3
 // It counts workgroups and not wavefronts: chunks of four wavefronts (65536 / 256)
 // would still gain above it (320: 34.6 / 30.8, 512: 35.5 / 32.4, 768: 39.4 / 38.3)
-// and lose at 1024 (45.2 / 61.1); eight-row products (above) and reads with
-// normalizers (320, precision 3, groups of 64: 50.3 / 47.2) would gain as well.
-// All of those keep the two-read step.  Below the line it costs where a wavefront
+// and lose at 1024 (45.2 / 61.1); reads with normalizers (320, precision 3, groups of 64:
+// 50.3 / 47.2) would gain as well.
+// Those keep the two-read step.  Below the line it costs where a wavefront
 // takes many words (6 bits per exponent, 256 workgroups: 36.3 / 36.9; 8 workgroups:
 // 29.8 / 27.1) and where four streams launch 256 workgroups each at the same time
 // (342 / 370 for sixteen reads: two workgroups to a compute unit and not three;
