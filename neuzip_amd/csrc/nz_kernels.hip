@@ -1620,10 +1620,11 @@ static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 3
 // dynamic LDS of a decode workgroup whose chunks have up to `spc` segments
 #define NZ_DEC_LDS_BYTES(spc, one) ((size_t)8 * (NZ_M + (spc) * ((one) ? NZ_RING_WIDE : NZ_RING_NARROW)))
 // Fused products of that many rows stage activations behind the rings, in launches of more than one
-// workgroup per compute unit (two groups' worth; 64 KiB in all for eight rows and eight segments).
+// workgroup per compute unit whose chunks have a segment for each row (two groups' worth; 64 KiB in
+// all for eight rows and eight segments).
 #define NZ_STAGED_ROWS 6
 #define NZ_GEMV_LDS_BYTES(spc, one, rows) \
-  (NZ_DEC_LDS_BYTES(spc, one) + (!(one) && (rows) >= NZ_STAGED_ROWS ? (size_t)2048 * (rows) : 0))
+  (NZ_DEC_LDS_BYTES(spc, one) + (!(one) && (rows) >= NZ_STAGED_ROWS && (spc) >= (rows) ? (size_t)2048 * (rows) : 0))
 // Launches of at most one workgroup per compute unit decode with NzWaveDecOne and its
 // wide ring, unless their output is written with streaming stores.  (Fused products of more
 // workgroups take it too, with the narrow ring and in any case: the two-read step took
