@@ -228,12 +228,15 @@ __device__ __forceinline__ uint32_t nz_wave_scan(uint32_t v, uint32_t lane) {
 // the next power of two
 __device__ __forceinline__ constexpr uint32_t nz_pow2(uint32_t v) { return v <= 1 ? 1u : v <= 2 ? 2u : v <= 4 ? 4u : 8u; }
 
-// Sums of MR (up to 8) floats over the 64 lanes, all at once: with P the next power of two, lane l
-// gets the total of v[l / (64 / P)], where there is one.
-// The lanes that are 32, 16 and 8 apart are added first; a step that has two values left puts one
-// into each half of the lanes with its exchange (eight values: seven additions and three more
-// instead of eight times six).  Then the lanes 1, 2 and 4 apart.  The tree is the same for
-// every MR, so a value's total does not depend on how many are summed beside it.
+// Sums of MR (up to 8) floats over the 64 lanes, all at once; the lane for which nz_sum_lane
+// holds gets the total of v[nz_sum_index(lane)], where there is one.
+// Lanes 1 apart are added first, then those 2, 4, 8, 16 and 32 apart: one tree for every MR,
+// so a value's total does not depend on how many are summed beside it, and it stays
+// the same from version to version.  The steps of 1, 2 and 16 put one half of the values that are
+// left into each half of the lanes (eight values: 25 instructions or so instead of eight times seven).
+// Those of 4 and 8 are rotations of the row, which make the right pairs in the lanes with bit 2 set.
+// (Eight rows through the Linears of a block of width 4096: 243.6 us.  Steps of 32, 16, 8, 1, 2
+// and 4, all of the first three exchanges, took 243.0 and gave other bits.)
 template <int MR>
 __device__ __forceinline__ float nz_wave_sums(const float (&v)[MR], uint32_t lane) {
   static_assert(MR >= 1 && MR <= 8, "");
@@ -241,25 +244,43 @@ __device__ __forceinline__ float nz_wave_sums(const float (&v)[MR], uint32_t lan
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), decltype(ctrl)::value, 0xF, 0xF, true));
   };
   constexpr int P = nz_pow2(MR), A = P > 1 ? P / 2 : 1, B = A > 1 ? A / 2 : 1;
-  const auto bits = [&](int m) { return m < MR ? __float_as_uint(v[m]) : 0u; };
+  // lo + its partner's in the lower half of the lanes, hi + its partner's in the upper
+  const auto halves = [&](float lo, float hi, bool upper, auto ctrl) {
+    const float own = upper ? hi : lo, other = upper ? lo : hi;
+    return own + dpp(other, ctrl);
+  };
+  using Pair = std::integral_constant<int, 0xB1>;  // quad_perm:[1,0,3,2]
+  using Quad = std::integral_constant<int, 0x4E>;  // quad_perm:[2,3,0,1]
   float a[A], b[B];
 #pragma unroll
-  for (int m = 0; m < A; ++m) {
-    const auto r = __builtin_amdgcn_permlane32_swap(bits(m), bits(P > 1 ? m + A : m), false, false);
-    a[m] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  }
+  for (int m = 0; m < A; ++m)
+    if (P > 1 && m + A < MR) a[m] = halves(v[m], v[m + A < MR ? m + A : m], lane & 1u, Pair{});
+    else a[m] = v[m] + dpp(v[m], Pair{});
 #pragma unroll
   for (int m = 0; m < B; ++m) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[m]), __float_as_uint(a[A > 1 ? m + B : m]), false, false);
-    b[m] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    if (A > 1) b[m] = halves(a[m], a[m + B < A ? m + B : m], lane & 2u, Quad{});
+    else b[m] = a[m] + dpp(a[m], Quad{});
+    b[m] += dpp(b[m], std::integral_constant<int, 0x124>{});  // row_ror:4
+    b[m] += dpp(b[m], std::integral_constant<int, 0x128>{});  // row_ror:8
   }
-  const bool upper = lane & 8u;
-  const float own = B > 1 && upper ? b[B - 1] : b[0], other = B > 1 && !upper ? b[B - 1] : b[0];
-  float t = own + dpp(other, std::integral_constant<int, 0x128>{});  // row_ror:8
-  t += dpp(t, std::integral_constant<int, 0xB1>{});                  // quad_perm:[1,0,3,2]
-  t += dpp(t, std::integral_constant<int, 0x4E>{});                  // quad_perm:[2,3,0,1]
-  t += dpp(t, std::integral_constant<int, 0x141>{});                 // row_half_mirror: the other quad
-  return t;
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(b[0]), __float_as_uint(b[B - 1]), false, false);
+  const uint32_t t = __float_as_uint(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+  const auto q = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+  return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+// the value whose total a lane has, and whether it is the lane that is asked for it
+template <int MR>
+__device__ __forceinline__ uint32_t nz_sum_index(uint32_t lane) {
+  constexpr uint32_t P = nz_pow2(MR);
+  return P == 8   ? 4 * (lane & 1) + (lane & 2) + (lane >> 4 & 1)
+         : P == 4 ? 2 * (lane & 1) + (lane >> 1 & 1)
+         : P == 2 ? lane & 1
+                  : 0u;
+}
+template <int MR>
+__device__ __forceinline__ bool nz_sum_lane(uint32_t lane) {
+  constexpr uint32_t P = nz_pow2(MR), which = P == 8 ? 0x13u : P == 4 ? 3u : P == 2 ? 1u : 0u;
+  return (lane & ~which) == 4u && nz_sum_index<MR>(lane) < (uint32_t)MR;
 }
 
 __device__ __forceinline__ uint32_t nz_get12(const uint8_t* p, uint32_t i) {
@@ -1874,10 +1895,10 @@ struct NzGemvWalk {
   // the row's results, one lane per activation row (for a shared row of eight activations one
   // chain of atomics, not eight after each other)
   __device__ __forceinline__ void flush(uint32_t lane) {
+    asm volatile("" : "+v"(lane));  // which lane takes which value is worked out here, not kept across the groups
     const float t = nz_wave_sums<MR>(sum, lane);
-    constexpr uint32_t PER = NZ_LANES / nz_pow2(MR);
-    const uint32_t m = lane / PER;
-    if (lane % PER == 0 && m < MR) {
+    const uint32_t m = nz_sum_index<MR>(lane);
+    if (nz_sum_lane<MR>(lane)) {
       const uint64_t first = row * gv.in_features, last = first + gv.in_features - 1;
       if (first >= seg_first && last < seg_end) {
         store_row(t, m);

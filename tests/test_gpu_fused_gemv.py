@@ -624,3 +624,32 @@ def test_activations_staged_in_lds(rows, cols, chunk, lane, m_rows, s):
         assert torch.equal(one.view(torch.int16), out[m].view(torch.int16)), m
     want = x.double() @ mgr.read(h).double().t()
     assert ((out.double() - want).norm() / want.norm()).item() < 2.0 ** -8  # a bf16 rounding of each result
+
+
+@pytest.mark.parametrize("m_rows", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_order_of_additions_across_lanes(m_rows):
+    """The 64 partial sums of a row are added pairwise, lanes 1, 2, 4, 8, 16 and 32 apart, for
+    every number of rows: pinned with partial sums that are single weights (each activation row
+    picks one of a lane's eight) and cancel over forty binades, where another order gives other results."""
+    import neuzip_amd
+
+    rows, cols = 700, 512  # one group per row
+    rng = np.random.default_rng(m_rows)
+    w = np.ldexp(rng.choice([-1.0, 1.0], (rows, 8, 32)) * (1 + rng.integers(0, 128, (rows, 8, 32)) / 128),
+                 rng.integers(-2, 39, (rows, 8, 32)))
+    w = rng.permuted(np.concatenate([w, -w], axis=-1), axis=-1)
+    w = torch.from_numpy(w.transpose(0, 2, 1).reshape(rows, cols).astype(np.float32)).to(torch.bfloat16)
+    x = torch.zeros(m_rows, cols, dtype=torch.bfloat16)
+    for m in range(m_rows):
+        x[m, m::8] = 1
+    mgr = neuzip_amd.Manager(precision=7)
+    h = mgr.write(w.cuda())
+    out = torch.full((m_rows, rows), 7.0, dtype=torch.bfloat16, device="cuda")
+    print(f"case rows={m_rows}", flush=True)
+    mgr._be.gemv_batch((ctypes.c_char_p * 1)(h.encode()), x.cuda(), [None], [out], m_rows)
+    for m in range(m_rows):
+        t = w[:, m::8].float()
+        while t.shape[1] > 1:
+            t = t[:, 0::2] + t[:, 1::2]
+        assert torch.equal(out[m].cpu().view(torch.int16), t[:, 0].to(torch.bfloat16).view(torch.int16)), m
+    mgr._be.check()
