@@ -253,7 +253,10 @@ int nz_manager_in_budget(const nz_manager* m, uint64_t n, uint32_t chunk_size, u
    product that needs larger accumulators, a row gather - is refused with
    NZ_ERR_ARG while its stream is being captured into a graph, before it
    touches anything (the capture stays valid); reads and products of settled
-   entries are captured and replay.  Calls on one manager from several host
+   entries are captured and replay.  (A product's accumulators are sized for
+   NZ_GEMV_MAX_ROWS activation rows whatever the call has, and stay where a
+   captured product has left their address until the manager is destroyed.)
+   Calls on one manager from several host
    threads are serialised by the manager. */
 int nz_manager_write(nz_manager* m, const char* name, const void* dev_data, uint64_t n,
                      int dtype, void* stream);
@@ -395,7 +398,9 @@ int nz_manager_import(nz_manager* m, const char* name, const void* host_comp, ui
                       uint64_t norm_bytes, void* stream);
 
 /* Release the manager's scratch (the workspace of the largest write so far, the
-   accumulators of the matrix-vector product); it is allocated again on demand.
+   accumulators of the matrix-vector product, unless a captured product holds
+   their address: they are needed when its graph is replayed and are then kept);
+   it is allocated again on demand.
    The reference allocates its scratch per call (cuda/high_level.cu:81-108).
    Waits for the device. */
 int nz_manager_trim(nz_manager* m);

@@ -541,7 +541,10 @@ struct nz_manager {
   uint32_t* d_status = nullptr;  // 256 bytes: decode status | container sizes and status words of a write batch
   uint64_t* h_pin = nullptr;     // pinned, 256 bytes: [0..15] those sizes, [16] decode status, [17..24] those status words
   long long* gemv_acc = nullptr;  // row accumulators of the matrix-vector product (all zero between calls)
-  uint64_t gemv_rows = 0;         // rows the accumulator buffer can hold
+  uint64_t gemv_rows = 0;         // accumulator pairs the buffer holds
+  bool gemv_captured = false;     // a captured product holds its address: it stays until the manager is destroyed ...
+  struct { long long* acc; uint64_t rows; } gemv_kept[16];  // ... as do those it replaced: each of at least 2^16
+  uint32_t gemv_kept_n = 0;                                 // and fewer than 2^31 pairs, twice as many as the one before
   RewriteSlot rw[2];              // in-place rewrites in flight (two batches: the host runs one ahead)
   uint32_t rw_next = 0;
   // statistics: batches rewritten in place / entries that outgrew their buffer / entries whose records were
@@ -757,6 +760,7 @@ void nz_manager_destroy(nz_manager* m) {
     if (m->rw[k].ev) (void)hipEventDestroy(m->rw[k].ev);
   }
   if (m->gemv_acc) (void)hipFree(m->gemv_acc);
+  for (uint32_t k = 0; k < m->gemv_kept_n; ++k) (void)hipFree(m->gemv_kept[k].acc);
   if (m->order_ev) (void)hipEventDestroy(m->order_ev);
   if (m->d_status) (void)hipFree(m->d_status);
   if (m->h_pin) (void)hipHostFree(m->h_pin);
@@ -1058,8 +1062,10 @@ int refuse_under_capture(hipStream_t st, bool may_block, const char* what) {
 // is made to wait (an event, no host synchronisation) for what the other has
 // been given so far.  Streams under capture are left alone: what a graph holds
 // is ordered by the graph's owner.
-int order_scratch_use(nz_manager* m, hipStream_t st) {
-  if (capturing(st)) return NZ_OK;
+int order_scratch_use(nz_manager* m, hipStream_t st, bool* captured = nullptr) {
+  const bool cap = capturing(st);
+  if (captured) *captured = cap;
+  if (cap) return NZ_OK;
   if (m->has_stream && m->last_stream != st && !capturing(m->last_stream)) {
     // (a stream that has gone into capture since its last call here is left alone: an event
     // recorded on it now would become part of its graph)
@@ -1328,6 +1334,7 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
   b.log2n = log2_of(m->normalizer ? m->normalizer : 1);
   uint64_t grid = 0, rows = 0;
   uint32_t max_spc = 1;
+  bool captured = false;
   {
     bool blocks = false;
     uint64_t want_rows = 0;
@@ -1339,7 +1346,7 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
       want_rows += it->second.n / in_features * x_rows;  // an accumulator pair per row and activation row
     }
     if (int rc = refuse_under_capture(st, blocks || m->gemv_rows < want_rows, "gemv_batch")) return rc;
-    if (int rc = order_scratch_use(m, st)) return rc;
+    if (int rc = order_scratch_use(m, st, &captured)) return rc;
   }
   for (uint32_t i = 0; i < count; ++i) {
     auto it = m->entries.find(names[i]);
@@ -1369,14 +1376,30 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
   if (m->gemv_rows < rows) {
     // the buffer in use may still be read by kernels on the stream
     NZ_HIP(hipStreamSynchronize(st));
-    if (m->gemv_acc) NZ_HIP(hipFree(m->gemv_acc));
-    m->gemv_acc = nullptr;
-    m->gemv_rows = 0;
-    const uint64_t want = rows < 65536 ? 65536 : rows;
-    NZ_HIP(hipMalloc((void**)&m->gemv_acc, want * 16));
-    NZ_HIP(hipMemset(m->gemv_acc, 0, want * 16));
+    // Room for every number of activation rows this manager's products take, so that a launch
+    // that has been made with some can be captured with others.  A buffer that a graph may write
+    // to is kept; its successor is at least twice as large, so all that are kept stay below the
+    // one in use.
+    uint64_t want = rows / x_rows * (m->normalizer ? 1u : NZ_GEMV_MAX_ROWS);
+    if (m->gemv_captured && want < 2 * m->gemv_rows) want = 2 * m->gemv_rows;
+    if (want < 65536) want = 65536;
+    long long* acc = nullptr;
+    NZ_HIP(hipMalloc((void**)&acc, want * 16));
+    if (hipError_t e = hipMemset(acc, 0, want * 16)) {
+      (void)hipFree(acc);
+      return fail(NZ_ERR_HIP, std::string("gemv_batch: ") + hipGetErrorString(e));
+    }
+    if (m->gemv_captured) {
+      m->gemv_kept[m->gemv_kept_n].acc = m->gemv_acc;
+      m->gemv_kept[m->gemv_kept_n++].rows = m->gemv_rows;
+    } else if (m->gemv_acc) {
+      (void)hipFree(m->gemv_acc);
+    }
+    m->gemv_acc = acc;
     m->gemv_rows = want;
+    m->gemv_captured = false;
   }
+  if (captured) m->gemv_captured = true;
   for (uint32_t i = 0; i < count; ++i) {
     b.item[i].acc = m->gemv_acc + 2 * (uint64_t)b.item[i].reserved;
     b.item[i].reserved = 0;
@@ -1683,9 +1706,11 @@ int nz_manager_trim(nz_manager* m) {
     m->rw[k].ws = nullptr;
     m->rw[k].ws_bytes = 0;
   }
-  if (m->gemv_acc) NZ_HIP(hipFree(m->gemv_acc));
-  m->gemv_acc = nullptr;
-  m->gemv_rows = 0;
+  if (m->gemv_acc && !m->gemv_captured) {
+    NZ_HIP(hipFree(m->gemv_acc));
+    m->gemv_acc = nullptr;
+    m->gemv_rows = 0;
+  }
   return NZ_OK;
 }
 
@@ -1711,6 +1736,8 @@ int nz_manager_check(nz_manager* m, void* stream) {
   const uint32_t hs = (uint32_t)m->h_pin[16];
   // a product that met a broken container left rows half summed: start clean
   if (hs && m->gemv_acc) NZ_HIP(hipMemset(m->gemv_acc, 0, m->gemv_rows * 16));
+  for (uint32_t k = 0; hs && k < m->gemv_kept_n; ++k)
+    NZ_HIP(hipMemset(m->gemv_kept[k].acc, 0, m->gemv_kept[k].rows * 16));
   if (hs == 8u) return fail(NZ_ERR_CORRUPT, "a row gather was given an index outside the table");
   if (hs)
     return fail(NZ_ERR_CORRUPT,

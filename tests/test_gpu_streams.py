@@ -185,3 +185,44 @@ def test_size_budget_setter():
     assert chunk == 512 * lane and lane > 400 and tight.size(h3) < mgr.size(h) < loose.size(h2)
     for m_, h_ in ((mgr, h), (loose, h2), (tight, h3)):
         assert torch.equal(m_.read(h_), w)
+
+
+def test_captured_product_after_larger_products_and_a_trim():
+    """Rows of 1536 elements straddle segments, so the replayed product works on the
+    accumulators that it was captured with."""
+    import neuzip_amd
+
+    mgr = neuzip_amd.Manager()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    cols = 1536
+    handles = [mgr.write((torch.randn(r, cols, device="cuda", generator=gen) * 0.02).to(torch.bfloat16))
+               for r in (14000, 40000)]
+    mgr.flush()
+    x = torch.randn(8, cols, device="cuda", generator=gen).to(torch.bfloat16)
+    name = [(ctypes.c_char_p * 1)(h.encode()) for h in handles]
+    out = [torch.empty(8, r, dtype=torch.bfloat16, device="cuda") for r in (14000, 40000)]
+
+    def product(i, rows):
+        mgr._be.gemv_batch(name[i], x[:rows].contiguous() if rows < 8 else x, [None], [out[i][:rows]], rows)
+
+    xs = x[:5].clone()
+    y = torch.empty(5, 14000, dtype=torch.bfloat16, device="cuda")
+    product(0, 5)
+    want = out[0][:5].clone()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        mgr._be.gemv_batch(name[0], xs, [None], [y], 5)
+    for step in (lambda: product(0, 8), lambda: product(1, 8), mgr._be.trim, lambda: product(1, 3)):
+        step()
+        fill = torch.full((1 << 24,), 3, dtype=torch.int32, device="cuda")  # where memory given back would be used again
+        for _ in range(2):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        assert bool((fill == 3).all())
+        del fill
+    product(0, 8)
+    assert torch.equal(out[0][:5].view(torch.int16), want.view(torch.int16))
+    mgr._be.check()
