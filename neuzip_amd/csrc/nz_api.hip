@@ -187,11 +187,10 @@ int allow_encode_lds() {
   return NZ_OK;
 }
 
-// LDS a workgroup of `waves` wavefronts of class `cls` can have without lowering the number
-// of workgroups that the registers allow per compute unit (4, 6, 8 wavefronts per SIMD unit for
-// 256 and more, 128, 64 symbols per lane), less the kernel's own.
+// LDS a workgroup of `waves` wavefronts of class `cls` (0..3) can have without lowering the number
+// of workgroups that the registers allow per compute unit, less the kernel's own.
 uint32_t enc_dynamic_lds(int cls, uint32_t waves) {
-  const uint32_t waves_per_cu = cls >= 2 ? 16u : cls == 1 ? 24u : 32u;
+  const uint32_t waves_per_cu = 4u * nz_enc_waves(NZ_ENC_GROUPS[cls]);  // four SIMD units
   const uint32_t groups = waves_per_cu / waves ? waves_per_cu / waves : 1u;
   const uint32_t per_group = 160u * 1024u / groups, fixed = (uint32_t)((sizeof(NzEncLds) + 15u) & ~15u);
   return per_group > fixed ? per_group - fixed : 0u;

@@ -978,6 +978,15 @@ __device__ __forceinline__ bool nz_move_record(const NzEncItem& it, const uint64
   return true;
 }
 
+// Wavefronts per SIMD unit that the kernel for NG groups is compiled for: what its registers (72, 96,
+// 128 and 128 for the four NG) allow without spilling.  The host sizes the dynamic LDS by the same number.
+// (64 Mi elements in chunks of 16384 with 64 symbols per lane and of 65536 with 128: 100.8 and 77.5 us;
+// with LDS cut for 8 and 6 wavefronts and two registers spilled 104.9 and 79.0.)
+static constexpr int NZ_ENC_GROUPS[4] = {8, 16, 32, NZ_ENC_MAX_LANE_SYMS / NZ_GROUP};  // NG of the classes
+__host__ __device__ constexpr uint32_t nz_enc_waves(int ng) { return ng <= 8 ? 7u : ng <= 16 ? 5u : 4u; }
+// four wavefronts of the largest classes: four workgroups to a compute unit, each with 32 histogram copies
+static_assert(sizeof(NzEncLds) + (1024u << NZ_HIST_COPIES_LOG2) <= 160u * 1024u / nz_enc_waves(32), "");
+
 // Segments of up to 8 * NG symbols per lane: the exponents stay in registers.
 // Workgroup = max(4, segments per chunk) wavefronts; wavefront k owns segment k.
 // dynamic LDS of the encode kernels: the histogram (NzHist), then the word staging of
@@ -998,7 +1007,7 @@ __device__ unsigned long long nz_probe_acc[8];
 #endif
 
 template <int S, int NG>
-__global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 ? 5 : 4) void nz_encode_kernel(const NzEncBatch b) {
+__global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void nz_encode_kernel(const NzEncBatch b) {
   __shared__ NzEncLds L;
 #ifdef NZ_PROBE_PHASES
   unsigned long long probe_t = __builtin_readcyclecounter();
@@ -1045,8 +1054,8 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 
   }
   NzHist::clear(nz_enc_stage, b.copies_log2);
   __syncthreads();
-  const uint32_t lb_gen = L.lb[0];
-  const bool direct = it.direct && L.lb[1] != NZ_LOOKBACK_ABORT;  // this run places its records itself
+  // this run places its records itself (read again where it is asked: kept, it takes registers of the coding phase)
+  const auto places = [&] { return it.direct && L.lb[1] != NZ_LOOKBACK_ABORT; };
   const NzHist hist{nz_enc_stage + (lane & ((1u << b.copies_log2) - 1u)), b.copies_log2};
 
   // ---- phase 1: split.  Packed bytes go to the stored layout: segment k of a
@@ -1155,7 +1164,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 
   const uint32_t stage_w = b.stage_words < cap_words ? b.stage_words : cap_words;
   const uint32_t stage_lo = cap_words - stage_w;  // first word of the slot that has a place in the staging area
   const uint32_t est_seg_words = (uint32_t)(((uint64_t)est_bits * seg_syms / cn) >> 4);
-  bool staged = direct && stage_w >= 1024 && est_seg_words + (est_seg_words >> 4) + 64 <= stage_w;
+  bool staged = places() && stage_w >= 1024 && est_seg_words + (est_seg_words >> 4) + 64 <= stage_w;
   typedef __attribute__((address_space(3))) uint32_t lds_u32;
   uint32_t* stage = nz_enc_stage + wave * (b.stage_words / 2);
   const uint32_t stage_lds = (uint32_t)(uintptr_t)((lds_u32*)stage);
@@ -1238,9 +1247,10 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, NG <= 8 ? 7 : NG <= 16 
     });
   }
   if (!it.direct) return;  // the records are placed by nz_compact_kernel
+  const uint32_t lb_gen = L.lb[0];  // (only now: kept since the beginning, it was spilled for the coding phase)
   uint8_t* placed = it.ws + it.placed;  // per segment: its record is in the container and nowhere else
   const bool last_chunk = c + 1 == g.n_chunks;
-  if (!direct) {
+  if (!places()) {
     // the run before this one ended with a workgroup giving up: nothing is
     // placed, the caller is told, and the mark is taken away for the next run
     if (tid == 0) {
