@@ -1962,6 +1962,37 @@ struct NzGemvWalk {
   }
 };
 
+// The activations of a workgroup's next group of weights, in LDS, for chunks whose wavefronts are at
+// the same column all the time.  Each of the first MR wavefronts brings one activation row's
+// part (two buffers, one barrier per group).
+template <int MR>
+struct NzXStage {
+  uint4* buf;
+  const uint16_t* row;  // this lane's place in the activation row that the wavefront brings
+  uint32_t at;          // ... and in a buffer (16-byte units)
+  bool mine;            // whether it brings one
+
+  // Every segment of the chunk begins a row of the matrix and all have the same length.
+  static __device__ __forceinline__ bool fits(const NzGeom& g, const NzGemv& gv, uint32_t cn) {
+    return g.seg_syms % gv.in_features == 0 && g.chunk_syms == g.spc * g.seg_syms && cn == g.chunk_syms &&
+           g.spc >= (uint32_t)MR;
+  }
+  __device__ __forceinline__ void start(uint4* behind_rings, const NzGemv& gv, uint32_t wave, uint32_t lane) {
+    buf = behind_rings;
+    mine = wave < (uint32_t)MR;
+    at = NZ_LANES * wave + lane;
+    row = gv.x + (uint64_t)(mine ? wave : 0u) * gv.in_features + NZ_GROUP * lane;
+  }
+  __device__ __forceinline__ const uint4* buffer(uint32_t b) const { return buf + b * (NZ_LANES * MR); }
+  __device__ __forceinline__ uint4 fetch(uint32_t col) const { return *reinterpret_cast<const uint4*>(row + col); }
+  __device__ __forceinline__ void put(uint32_t b, const uint4 x) const {
+    if (mine) buf[b * (NZ_LANES * MR) + at] = x;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+};
+
 // A wavefront's record and its ring: where the record lies, what may be loaded of it, and the
 // staging of its head.
 struct NzRecord {
@@ -2483,22 +2514,15 @@ __device__ __forceinline__ void nz_decode_chunk(
   __syncthreads();
 
   if (!has_seg) return;
-  if (bad_rec) {
-    if (lane == 0) atomicOr(d_status, 2u);
-    return;
-  }
   // the chunk's first record begins with the table
   const uint32_t rec_skip = wave == 0 ? tab_len : 0u;
-  if (rec_all < rec_skip) {
-    if (lane == 0) atomicOr(d_status, 2u);
-    return;
-  }
+  const bool damaged = bad_rec || rec_all < rec_skip;
   const uint64_t rec_start = rec_pos + rec_skip;
   const uint32_t rec_bytes = rec_all - rec_skip;
 
   if (mode == NZ_MODE_RAW) {
     const uint32_t padded = (seg_n + 3) & ~3u;
-    if (rec_bytes < padded + (carry ? NZ_CARRY_BYTES : 0u)) {
+    if (damaged || rec_bytes < padded + (carry ? NZ_CARRY_BYTES : 0u)) {
       if (lane == 0) atomicOr(d_status, 2u);
       return;
     }
@@ -2535,10 +2559,6 @@ __device__ __forceinline__ void nz_decode_chunk(
     return;
   }
 
-  if (rec_bytes < 16) {
-    if (lane == 0) atomicOr(d_status, 2u);
-    return;
-  }
   // final encoder states, read from the staged window: 64 two-bit length
   // codes, then a nibble stream
   const uint32_t* rec32 = w.ring32 + rec_skip / 4;
@@ -2546,8 +2566,23 @@ __device__ __forceinline__ void nz_decode_chunk(
   const uint32_t incl = nz_wave_scan(nn, lane);
   const uint32_t at = incl - nn;
   const uint32_t sbytes = 16u + ((((__builtin_amdgcn_readlane(incl, 63) + 1u) >> 1) + 3u) & ~3u);
-  if (rec_bytes < sbytes) {
+  constexpr bool STAGED = GEMV >= NZ_STAGED_ROWS && !ONE && !NORM;
+  uint4* const xbuf = reinterpret_cast<uint4*>(rings + 2 * RING * g.spc);
+  if (damaged || rec_bytes < sbytes) {
     if (lane == 0) atomicOr(d_status, 2u);
+    if constexpr (STAGED) {
+      // the other segments of the chunk are multiplied with the activation row that this wavefront brings
+      if (NzXStage<MR>::fits(g, gv, cn)) {
+        NzXStage<MR> xs;
+        xs.start(xbuf, gv, wave, lane);
+        uint32_t col = 0;
+        xs.put(0, xs.fetch(0));
+        for (uint32_t k = 1; k <= (whole & ~1u); ++k) {  // as often as a wavefront that decodes
+          col = col + NZ_GROUP_SYMS == gv.in_features ? 0u : col + NZ_GROUP_SYMS;
+          xs.put(k & 1u, xs.fetch(col));
+        }
+      }
+    }
     return;
   }
   // the 8 bytes read here may reach into the words: still inside the window
@@ -2613,44 +2648,26 @@ __device__ __forceinline__ void nz_decode_chunk(
       sm_b = sm_at(gq + 1);
       if constexpr (NORM) nb_b = nb_at(gq + 1, wide);
     };
-    if constexpr (GEMV >= NZ_STAGED_ROWS && !ONE && !NORM) {
-      // Where all segments of the chunk begin a row of the matrix and have the same length, its
-      // wavefronts are at the same column all the time.  Each of the first MR then brings one
-      // activation row's part of the next group into LDS (two buffers, one barrier per group; wavefronts
-      // without a segment, or with a damaged one, have ended and are not waited for).
-      //
+    if constexpr (STAGED) {
       // Every wavefront by itself reads MR KiB per group, and beside a wavefront at another
       // column the vector L1 (32 KiB) holds too little of them: with all rows at one address
       // eight rows through the Linears of a block of width 4096 took 192 us, not 256.  Staged
       // (gate and up projection; the others keep the loads): six, seven and eight rows
       // 222, 239, 256 -> 219, 229, 242 us.  Up to five rows a third workgroup per compute unit
       // is worth more than that; launches of one workgroup lose 6 to 9 us to the barriers.
-      if (g.seg_syms % gv.in_features == 0 && g.chunk_syms == g.spc * g.seg_syms && cn == g.chunk_syms &&
-          g.spc >= (uint32_t)GEMV) {
-        constexpr uint32_t GROUP_X = NZ_LANES * GEMV;  // 16-byte units of a group
-        uint4* const xbuf = reinterpret_cast<uint4*>(rings + 2 * RING * g.spc);
-        const bool mine = wave < (uint32_t)GEMV;
-        const uint16_t* const xrow = gv.x + (uint64_t)(mine ? wave : 0u) * gv.in_features + NZ_GROUP * lane;
-        uint4 xs = *reinterpret_cast<const uint4*>(xrow + walk.col);
-        const auto put_x = [&](uint32_t buffer) __attribute__((always_inline)) {
-          if (mine) xbuf[buffer * GROUP_X + NZ_LANES * wave + lane] = xs;
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-          __builtin_amdgcn_s_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-        };
-        const auto fetch_x = [&]() __attribute__((always_inline)) {  // always inside x
-          xs = *reinterpret_cast<const uint4*>(xrow + walk.next_col());
-        };
-        put_x(0);
+      if (NzXStage<MR>::fits(g, gv, cn)) {
+        NzXStage<MR> xs;
+        xs.start(xbuf, gv, wave, lane);
+        xs.put(0, xs.fetch(0));
         for (; gq + 1 < whole; gq += 2) {
-          fetch_x();
-          full_group(gq, sm_a, nb_a, wide, fetch_b, (const uint4*)xbuf);
-          put_x(1);
-          fetch_x();
-          full_group(gq + 1, sm_b, nb_b, wide, fetch_a, (const uint4*)xbuf + GROUP_X);
-          put_x(0);
+          const uint4 next_b = xs.fetch(walk.next_col());  // always inside x
+          full_group(gq, sm_a, nb_a, wide, fetch_b, xs.buffer(0));
+          xs.put(1, next_b);
+          const uint4 next_a = xs.fetch(walk.next_col());
+          full_group(gq + 1, sm_b, nb_b, wide, fetch_a, xs.buffer(1));
+          xs.put(0, next_a);
         }
-        if (gq < whole) full_group(gq, sm_a, nb_a, wide, [] {}, (const uint4*)xbuf);
+        if (gq < whole) full_group(gq, sm_a, nb_a, wide, [] {}, xs.buffer(0));
         return;
       }
     }

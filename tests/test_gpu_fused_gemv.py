@@ -653,3 +653,35 @@ def test_order_of_additions_across_lanes(m_rows):
             t = t[:, 0::2] + t[:, 1::2]
         assert torch.equal(out[m].cpu().view(torch.int16), t[:, 0].to(torch.bfloat16).view(torch.int16)), m
     mgr._be.check()
+
+
+@pytest.mark.parametrize("m_rows", [5, 6, 7, 8])
+def test_damaged_records_leave_the_other_segments_right(m_rows):
+    """A segment whose record is cut short is reported; the other segments of its chunk get the products
+    they get beside an undamaged one, also where (from six rows on) the wavefront of the damaged
+    one brings an activation row for them."""
+    import neuzip_amd
+
+    rows, cols, chunk = 9000, 4096, 131072  # 282 workgroups, eight segments of four rows each
+    mgr = neuzip_amd.Manager(precision=7, chunk_size=chunk, lane_symbols=256)
+    g = torch.Generator(device="cuda").manual_seed(m_rows)
+    h = mgr.write((torch.randn(rows, cols, device="cuda", generator=g) * 0.02).to(torch.bfloat16))
+    x = torch.randn(m_rows, cols, device="cuda", generator=g).to(torch.bfloat16)
+    comp, packed, _ = mgr._be.export(h)
+    dir_off = int(comp[32:36].view(torch.int32))
+    entries = comp[dir_off:dir_off + 4 * (282 * 8 + 1)].view(torch.int32)
+    good = torch.ones(rows, dtype=torch.bool)
+    for c, k in ((3, 0), (17, 2), (100, 3), (280, 6)):
+        seg = 8 * c + k
+        entries[seg + 1] = entries[seg] + 1  # four bytes, and the next record begins inside this one
+        good[4 * seg:4 * seg + 8] = False
+    mgr._be.import_("cut", comp, packed)
+    want, got = (torch.full((m_rows, rows), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    mgr._be.gemv_batch((ctypes.c_char_p * 1)(h.encode()), x, [None], [want], m_rows)
+    mgr._be.check()
+    print(f"case rows={m_rows}", flush=True)
+    mgr._be.gemv_batch((ctypes.c_char_p * 1)(b"cut"), x, [None], [got], m_rows)
+    with pytest.raises(RuntimeError, match="validation"):
+        mgr._be.check()
+    good = good.cuda()
+    assert torch.equal(got[:, good].view(torch.int16), want[:, good].view(torch.int16))
