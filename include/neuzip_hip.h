@@ -253,9 +253,9 @@ int nz_manager_in_budget(const nz_manager* m, uint64_t n, uint32_t chunk_size, u
    product that needs larger accumulators, a row gather - is refused with
    NZ_ERR_ARG while its stream is being captured into a graph, before it
    touches anything (the capture stays valid); reads and products of settled
-   entries are captured and replay.  (A product's accumulators are sized for
-   NZ_GEMV_MAX_ROWS activation rows whatever the call has, and stay where a
-   captured product has left their address until the manager is destroyed.)
+   entries are captured and replay.  (A product's accumulators are sized for the
+   next power of two of its activation rows, and stay where a captured
+   product has left their address until the manager is destroyed.)
    Calls on one manager from several host
    threads are serialised by the manager. */
 int nz_manager_write(nz_manager* m, const char* name, const void* dev_data, uint64_t n,

@@ -543,7 +543,7 @@ struct nz_manager {
   uint64_t gemv_rows = 0;         // accumulator pairs the buffer holds
   bool gemv_captured = false;     // a captured product holds its address: it stays until the manager is destroyed ...
   struct { long long* acc; uint64_t rows; } gemv_kept[16];  // ... as do those it replaced: each of at least 2^16
-  uint32_t gemv_kept_n = 0;                                 // and fewer than 2^31 pairs, twice as many as the one before
+  uint32_t gemv_kept_n = 0;                                 // and fewer than 2^32 pairs, twice as many as the one before
   RewriteSlot rw[2];              // in-place rewrites in flight (two batches: the host runs one ahead)
   uint32_t rw_next = 0;
   // statistics: batches rewritten in place / entries that outgrew their buffer / entries whose records were
@@ -1372,31 +1372,28 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
     rows += ent.n / in_features * x_rows;
     if (grid > 0x7FFFFFFFull || rows > 0x7FFFFFFFull) return fail(NZ_ERR_ARG, "batch too large");
   }
-  if (m->gemv_rows < rows) {
+  // Room for the next power of two of activation rows, so that a launch that has been made with
+  // five can be captured with eight (a capture takes what is there if it is enough: see above).
+  const uint64_t pairs = rows / x_rows * nz_pow2(x_rows);
+  if (!captured && m->gemv_rows < pairs) {
     // the buffer in use may still be read by kernels on the stream
     NZ_HIP(hipStreamSynchronize(st));
-    // Room for every number of activation rows this manager's products take, so that a launch
-    // that has been made with some can be captured with others.  A buffer that a graph may write
-    // to is kept; its successor is at least twice as large, so all that are kept stay below the
-    // one in use.
-    uint64_t want = rows / x_rows * (m->normalizer ? 1u : NZ_GEMV_MAX_ROWS);
-    if (m->gemv_captured && want < 2 * m->gemv_rows) want = 2 * m->gemv_rows;
-    if (want < 65536) want = 65536;
-    long long* acc = nullptr;
-    NZ_HIP(hipMalloc((void**)&acc, want * 16));
-    if (hipError_t e = hipMemset(acc, 0, want * 16)) {
-      (void)hipFree(acc);
-      return fail(NZ_ERR_HIP, std::string("gemv_batch: ") + hipGetErrorString(e));
-    }
+    uint64_t want = pairs < 65536 ? 65536 : pairs;
     if (m->gemv_captured) {
+      // a graph may write to it: kept, and its successor at least twice as large, so that all
+      // that are kept stay below the one in use
+      if (want < 2 * m->gemv_rows) want = 2 * m->gemv_rows;
       m->gemv_kept[m->gemv_kept_n].acc = m->gemv_acc;
       m->gemv_kept[m->gemv_kept_n++].rows = m->gemv_rows;
     } else if (m->gemv_acc) {
-      (void)hipFree(m->gemv_acc);
+      NZ_HIP(hipFree(m->gemv_acc));
     }
-    m->gemv_acc = acc;
-    m->gemv_rows = want;
+    m->gemv_acc = nullptr;
+    m->gemv_rows = 0;
     m->gemv_captured = false;
+    NZ_HIP(hipMalloc((void**)&m->gemv_acc, want * 16));
+    NZ_HIP(hipMemset(m->gemv_acc, 0, want * 16));
+    m->gemv_rows = want;
   }
   if (captured) m->gemv_captured = true;
   for (uint32_t i = 0; i < count; ++i) {

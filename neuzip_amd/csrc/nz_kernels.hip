@@ -226,7 +226,7 @@ __device__ __forceinline__ uint32_t nz_wave_scan(uint32_t v, uint32_t lane) {
   return v;
 }
 // the next power of two
-__device__ __forceinline__ constexpr uint32_t nz_pow2(uint32_t v) { return v <= 1 ? 1u : v <= 2 ? 2u : v <= 4 ? 4u : 8u; }
+__host__ __device__ __forceinline__ constexpr uint32_t nz_pow2(uint32_t v) { return v <= 1 ? 1u : v <= 2 ? 2u : v <= 4 ? 4u : 8u; }
 
 // Sums of MR (up to 8) floats over the 64 lanes, all at once; the lane for which nz_sum_lane
 // holds gets the total of v[nz_sum_index(lane)], where there is one.

@@ -1,7 +1,7 @@
 """CPU: the row accumulators of fused products.  A graph that captured a product writes to them
-on every replay, so they outlive later calls that need more and a trim; and they are sized for every
-number of activation rows, so that a product that has been made with some rows can be captured with
-others.  The library runs in a child process on the stand-in for the HIP runtime of
+on every replay, so they outlive later calls that need more and a trim; and they are sized for the
+next power of two of a call's activation rows, so that a product that has been made with five rows can be
+captured with eight.  The library runs in a child process on the stand-in for the HIP runtime of
 test_launch_forms.py, here with a switch for capture, the addresses that are given back, and the
 kernel arguments of the last launch."""
 import subprocess
@@ -25,7 +25,7 @@ BODY = CHILD[:CHILD.index("got = {}")] + r"""
 ctypes.c_int.in_dll(stub, "stub_capturing")  # all three are there: the stand-in is the tracked one
 nfreed = ctypes.c_int.in_dll(stub, "stub_nfreed")
 freed = (ctypes.c_void_p * 64).in_dll(stub, "stub_freed")
-for chunks in (10000, 20000, 100000):  # two rows of 512 each
+for chunks in (5000, 10000, 20000, 100000):  # two rows of 512 each
     store(h, b"w%d" % chunks, chunks)
 
 
@@ -67,7 +67,7 @@ acc = product(10000, {captured_rows}, capture=True)
 {then}
 assert acc not in given_back()
 if "trim" in {then!r}:
-    assert product(10000, 8) == acc  # and are still the ones in use
+    assert product(10000, {captured_rows}) == acc  # and are still the ones in use
 again = product(10000, 8, capture=True)
 L.nz_manager_destroy(h)
 assert {{acc, again}} <= given_back()
@@ -76,9 +76,13 @@ assert {{acc, again}} <= given_back()
 
 def test_capture_with_more_rows_than_the_calls_before(child):
     child("""
-acc = product(10000, 1)
-for rows in (8, 2, 5):
-    assert product(10000, rows, capture=True) == acc
+for chunks in (5000, 10000, 20000):  # 5 x 10000 rows fit the least that is allocated, 8 x 10000 do not
+    for made, captured in ((3, (4, 2)), (5, (8, 6, 7, 1))):
+        acc = product(chunks, made)
+        for rows in captured:
+            assert product(chunks, rows, capture=True) == acc
+    for rows in (6, 8, 7, 5):
+        assert product(chunks, rows) == acc
 """)
 
 
