@@ -68,7 +68,7 @@ acc = product(10000, {captured_rows}, capture=True)
 assert acc not in given_back()
 if "trim" in {then!r}:
     assert product(10000, {captured_rows}) == acc  # and are still the ones in use
-again = product(10000, 8, capture=True)
+again = product(10000, {captured_rows}, capture=True)
 L.nz_manager_destroy(h)
 assert {{acc, again}} <= given_back()
 """)
