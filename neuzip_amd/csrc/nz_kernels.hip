@@ -2143,6 +2143,10 @@ struct NzWaveDec : NzRecord {
 // per six symbols or so.
 template <uint32_t RING>
 struct NzWaveDecOne : NzRecord {
+  // An entry's number is its LDS address over 8: the slot table is the first NZ_M of them (the dynamic LDS
+  // begins at address 0, nz_decode_chunk), a ring's number and a word's place in it are or-ed, and the
+  // address is made by a 16-bit shift.
+  static_assert(NZ_M % RING == 0 && (NZ_M + NZ_MAX_SEGS_PER_CHUNK * RING) * 8 <= 1u << 16, "");
   static constexpr uint32_t BLOCK = RING / 2;  // words the ring is refilled by
   static constexpr uint32_t PER_LANE = BLOCK / NZ_LANES;
   // the wide ring is looked at every so many steps, the most its block can feed; the narrow one per group
@@ -2292,6 +2296,8 @@ __device__ __forceinline__ void nz_decode_chunk(
     const uint8_t* __restrict__ comp, const uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
     const NzGemv& gv, const NzNorm& nm) {
+  // At LDS address 0: a kernel that decodes has no static LDS (pinned in tests/test_kernel_resources.py),
+  // because NzWaveDecOne numbers table and rings through from there.
   extern __shared__ uint32_t lds[];
   uint2* lut = reinterpret_cast<uint2*>(lds);                   // 4096 x 8 bytes
   uint32_t* rings = lds + 2 * NZ_M;                             // spc rings

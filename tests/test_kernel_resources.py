@@ -48,3 +48,11 @@ def test_register_encode_kernels_do_not_spill(kernels):
         waves = {8: 7, 16: 5, 32: 4, 36: 4}[groups]
         assert int(f[".vgpr_spill_count"]) == 0 and int(f[".private_segment_fixed_size"]) == 0, name
         assert 512 // (-(-int(f[".vgpr_count"]) // 8) * 8) >= waves, name
+
+
+def test_kernels_that_decode_have_no_static_lds(kernels):
+    """The one-read step takes the slot table, the start of the dynamic LDS, to be at LDS address 0."""
+    found = _of(kernels, "nz_decode_", 136)
+    for name, f in found.items():
+        assert int(f[".group_segment_fixed_size"]) == 0, name
+        assert int(f[".vgpr_spill_count"]) == 0 and int(f[".private_segment_fixed_size"]) == 0, name
