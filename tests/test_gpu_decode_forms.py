@@ -1,5 +1,6 @@
 """Both forms of the decode step: launches of up to one workgroup (chunk) per compute unit, 256 on
-a whole GPU, read one prepared entry per step, larger ones the slot table and the word in turn
+a whole GPU, read one prepared entry per step from a wide ring; larger ones the slot table and the
+word in turn for dense output, and one entry per step from a narrow ring for products
 (tests/test_launch_forms.py pins the rule).  Every kernel that decodes is run with as many chunks as
 the line and with one more: reads at every precision, with normalizers, of several tensors at once
 and of corrupt containers, row gathers, and products with one to eight activation rows."""
@@ -188,4 +189,34 @@ def test_products_with_normalizers(oracle, s, chunks):
     (y,) = _gemv(mgr, [h], x, None)
     # the reconstruction is what the product multiplies: lossless from here on
     _check(y, oracle.reconstruct_normalized(bits, s, 64), x, None, 7)
+    mgr._be.check()
+
+
+@pytest.mark.parametrize("kind", ["normal", "wide", "bursts"])
+@pytest.mark.parametrize("chunk,lane,cols", [(131072, 256, 4096),  # from six rows on with staged activations
+                                             (65536, 128, 1536)])  # rows straddle the segments of 8192
+def test_products_that_take_many_words(kind, chunk, lane, cols):
+    """More than 256 workgroups: the narrow ring.  It is looked at once per group of 512 symbols, when
+    at least 129 words are left in it; a group that takes more ("wide": 192, "bursts": up to 350) refills it inside."""
+    import neuzip_amd
+
+    rows = 257 * chunk // cols + 1
+    n = rows * cols
+    bits = _bits(kind, n)
+    mgr = neuzip_amd.Manager(chunk_size=chunk, lane_symbols=lane)
+    w = _dev(bits, rows, cols)
+    h = mgr.write(w)
+    assert _coded_chunks(mgr._be.export(h)[0].numpy(), n, chunk, lane) >= n // chunk > 256
+    g = torch.Generator(device="cuda").manual_seed(cols)
+    x = torch.randn(8, cols, device="cuda", generator=g).to(torch.bfloat16)
+    want = x.double() @ w.double().t()
+    # a bf16 rounding of the result; fp32 sums; partial sums of a shared row resolved to 2^-40
+    tol = 2.0 ** -8 * want.abs() + 1e-5 * (x.double().abs() @ w.double().abs().t()) + 2.0 ** -36
+    ones = torch.stack([_gemv(mgr, [h], x[m].contiguous(), None)[0] for m in range(8)])
+    assert bool(((ones.double() - want).abs() <= tol).all())
+    for m_rows in (2, 5, 6, 8):
+        print(f"case {kind} chunk={chunk} cols={cols} rows={m_rows}", flush=True)
+        out = torch.full((m_rows, rows), 7.0, dtype=torch.bfloat16, device="cuda")
+        mgr._be.gemv_batch((ctypes.c_char_p * 1)(h.encode()), x[:m_rows].contiguous(), [None], [out], m_rows)
+        assert torch.equal(out.view(torch.int16), ones[:m_rows].view(torch.int16)), m_rows
     mgr._be.check()

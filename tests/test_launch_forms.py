@@ -1,8 +1,10 @@
-"""CPU: which form of the decode step a launch gets.  The one-read form is for launches of at most
-one workgroup per compute unit of the device in use; its workgroups ask for 4 KiB of ring per
-wavefront where the two-read form asks for 2 KiB, so the dynamic LDS of a launch tells the forms
-apart.  The library runs in a child process on a stand-in for the HIP runtime (memory from the
-host, launches recorded and not run)."""
+"""CPU: which ring a launch that decodes gets, and what LDS a fused product asks for.  Launches of at
+most one workgroup per compute unit of the device in use decode with the one-read step and its wide
+ring, 4 KiB per wavefront.  Larger ones have 2 KiB: dense output a ring of words (the two-read
+step), fused products the narrow ring of prepared entries (the one-read step again); which of the
+two is a matter of the kernel, not of its LDS.  Products of six to eight rows stage activations behind the
+rings there, 2 KiB per row, where chunks have a segment for each row.  The library runs in a child
+process on a stand-in for the HIP runtime (memory from the host, launches recorded and not run)."""
 import json
 import os
 import subprocess
@@ -65,16 +67,17 @@ def form(call):
     launched.value = 0
     rc = call()
     assert rc == 0, m.last_error()
-    return {32768 + 4096: "one", 32768 + 2048: "two"}[lds[0]]
+    return {32768 + 4096: "wide", 32768 + 2048: "2 KiB"}[lds[0]]
 
 
-def store(mgr, name, chunks):
+def store(mgr, name, chunks, segs=1):
     # a well-formed header and directory; the records stay empty
-    rec = (64 + 4 * (chunks + 1) + 15) & ~15
-    total = rec + 16
-    comp = struct.pack("<6I4IQ4I", 0x315A4E41, 4, CHUNK * chunks, 0, CHUNK, LANE, chunks, chunks, 64, rec, total, 0, 0, 0, 0)
+    rec = (64 + 4 * (chunks * segs + 1) + 15) & ~15
+    total, chunk = rec + 16, CHUNK * segs
+    comp = struct.pack("<6I4IQ4I", 0x315A4E41, 4, chunk * chunks, 0, chunk, LANE, chunks, chunks * segs, 64, rec, total,
+                       0, 0, 0, 0)
     comp = ctypes.create_string_buffer(comp + bytes(total - 64), total)
-    packed = ctypes.create_string_buffer(L.nz_packed_stored_bytes(CHUNK * chunks, 7, CHUNK, LANE))
+    packed = ctypes.create_string_buffer(L.nz_packed_stored_bytes(chunk * chunks, 7, chunk, LANE))
     assert L.nz_manager_import(mgr, name, comp, total, packed, len(packed), None, 0, None) == 0, m.last_error()
 
 
@@ -96,6 +99,12 @@ for chunks in (cus, cus + 1):
         "gather": lambda: L.nz_manager_gather_rows(h, name, at, chunks, CHUNK, at, None),
     }
     got["at the line" if chunks == cus else "above"] = {k: form(f) for k, f in out.items()}
+    for segs in (4, 6, 8):
+        store(h, b"s%d" % segs, chunks, segs)
+        for rows in range(1, 9):
+            launched.value = 0
+            assert L.nz_manager_gemv_rows_batch(h, (ctypes.c_char_p * 1)(b"s%d" % segs), 1, at, rows, 512, None, ptrs, None) == 0
+            got["%d segments, %d rows, %s" % (segs, rows, "line" if chunks == cus else "above")] = lds[0]
 print(json.dumps(got))
 """
 
@@ -109,9 +118,16 @@ def runtime(tmp_path_factory):
 
 
 @pytest.mark.parametrize("cus", [256, 32])  # the whole device, one of eight partitions
-def test_one_read_form_up_to_one_workgroup_per_compute_unit(runtime, cus):
+def test_wide_ring_up_to_one_workgroup_per_compute_unit(runtime, cus):
     res = subprocess.run([sys.executable, "-c", CHILD, runtime, ROOT, str(cus)], capture_output=True, text=True, timeout=120)
     assert res.returncode == 0, res.stderr
     got = json.loads(res.stdout)
-    assert got["at the line"].pop("streaming decode") == "two" and got["above"].pop("streaming decode") == "two"
-    assert set(got["at the line"].values()) == {"one"} and set(got["above"].values()) == {"two"}, got
+    line, above = got.pop("at the line"), got.pop("above")
+    assert line.pop("streaming decode") == "2 KiB"
+    assert set(line.values()) == {"wide"} and set(above.values()) == {"2 KiB"}, (line, above)
+    for segs in (4, 6, 8):
+        for rows in range(1, 9):
+            staged = 2048 * rows if rows >= 6 and segs >= rows else 0
+            assert got.pop(f"{segs} segments, {rows} rows, line") == 32768 + 4096 * segs
+            assert got.pop(f"{segs} segments, {rows} rows, above") == 32768 + 2048 * segs + staged
+    assert not got
