@@ -850,14 +850,17 @@ int pick_geometry(const nz_manager* m, const char* name, uint64_t n, NzGeom* g, 
     // budget and the model below promises 10 % or more; a tensor too small for
     // that may get 32 Ki chunks of eight 4 Ki segments (again: only inside the
     // budget).  Time of a round ~ symbols per lane x a weight that grows with the
-    // workgroups on a compute unit.  Only the ratios of the weights matter: they
-    // are those of whole reads, 31.9, 43.8, 62.6 us with one, two, three workgroups
-    // per compute unit at 256 symbols per lane (107 : 147 : 210), where the first
-    // takes the one-read step of the decoder; products 30.0, 42.4, 53.8 us.  A
-    // smaller first weight would change the choice at the default budget for 313
-    // to 384 chunks (one longer round instead of two): there a read gains 8 % at
-    // 314 chunks (41.0 -> 37.6 us) and 3 % at 336 and loses from 344 on, a product
-    // of rows of 4096 gains 17 % at 314, 8 % at 336 and 0 to 6 % above.
+    // workgroups on a compute unit.  Only the ratios of the weights matter.  They
+    // were those of whole reads, 31.9, 43.8, 62.6 us with one, two, three workgroups
+    // per compute unit at 256 symbols per lane (107 : 147 : 210), before the decoder's
+    // one-read step was shortened and larger products took it as well; now reads
+    // take 30.2, 44.2 and (written with streaming stores) 66.9 us, products of rows of
+    // 4096 26.5, 36.8, 47.7 us for one activation row and 34.2, 49.1, 76.4 for eight.
+    // A smaller first weight would change the choice at the default budget for 313
+    // to 384 chunks (one longer round instead of two): there a read gains 12 % at
+    // 314 chunks (40.7 -> 35.9 us), 6 % at 336 and 1 to 5 % up to 368, a product of
+    // one or eight rows 13 to 15 % up to 320 chunks, 3 to 4 % at 336, and either loses
+    // up to 3 % from 368 on.
     const uint64_t slots = m->slots, cus = slots / 3;
     const uint64_t chunks = (n + chunk_syms - 1) / chunk_syms;
     if (chunks <= slots && cus != 0) {

@@ -733,13 +733,13 @@ struct NzEncAhead {
   }
 };
 
-// the 8 symbols of one group (byte j of `sy` = symbol j), last symbol first; `sy_next`: those
-// of the group that is coded after it
+// The 8 symbols of one group (byte j of `sy` = symbol j), last symbol first; `sy_next`: those
+// of the group that is coded after it.
 // Words go downwards from `pos`, a byte offset into the segment's slot in scratch memory or,
-// with LDS, the LDS byte address of the wavefront's staging area.  In the staging area every lane stores: a lane without a word writes one of the
-// 64 places below the words of the step (each lane its own), which the words that
-// follow overwrite.  That keeps the execution mask out of the step's chain; the
-// caller leaves 64 words of room below.
+// with LDS, an LDS byte address in the wavefront's staging area.  There every lane stores: a
+// lane without a word writes one of the 64 places below the words of the step (each lane its
+// own), which the words that follow overwrite.  That keeps the execution mask out of the step's
+// chain; the caller leaves 64 words of room below.
 template <bool LDS>
 __device__ __forceinline__ void nz_enc_group(uint32_t& x, uint32_t& pos, const uint64_t sy, const uint64_t sy_next,
                                              NzEncAhead& ahead, const uint4* __restrict__ tab,
@@ -1659,7 +1659,9 @@ static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 3
 // Launches of at most one workgroup per compute unit decode with NzWaveDecOne and its
 // wide ring, unless their output is written with streaming stores.  (Fused products of more
 // workgroups take it too, with the narrow ring and in any case: the two-read step took
-// 184.5 us for the one-row products of a block of width 4096, this one 168.2.)  The line lies
+// 184.5 us for the one-row products of a block of width 4096, this one 168.2.  Exponents of
+// six bits, two or three times what weights have, cost it a refill per group: one row times
+// 50257 x 1024 of those took 45.0 us and takes 46.6, 14336 x 4096 42.9 and 42.0.)  The line lies
 // where the figures of dense output crossed for the default chunk (eight wavefronts, 256 symbols
 // per lane; MI355X, 256 compute units; two-read against one-read step, microseconds, taken when
 // the one-read step was some 5 % longer than it is):

@@ -102,7 +102,10 @@ class FusedGemv:
 
     # Time of a launch with one, two, three 8-wavefront workgroups per compute unit and
     # equal segments, up to a common factor (MI355X); the weights that choose a tensor's
-    # geometry when it is written on its own (pick_geometry in csrc/nz_api.hip).
+    # geometry when it is written on its own (pick_geometry in csrc/nz_api.hip, with what
+    # such launches take).  They are for one row; eight rows times gate/up take 107.6, 80.0
+    # and 123.2 us in the three geometries below, where segments of 256 symbols per lane
+    # begin rows, share their activations in LDS and take 93.6.
     _WEIGHT = (107, 147, 215)
 
     def _fit_geometry(self, g, cus=None) -> None:
@@ -124,7 +127,7 @@ class FusedGemv:
             if not 64 <= lane <= 512 or not all(be.in_budget(n, lane * 512, lane) for n in sizes):
                 continue
             t = lane * self._WEIGHT[k - 1]
-            if best is None or t <= best[0]:  # measured on gate/up of an 8B model: 2 x 512 chunks 73-76 us, 2 x 256 71.5, 2 x 378 69.4
+            if best is None or t <= best[0]:  # measured on gate/up of an 8B model, one row: 2 x 512 chunks 59.5 us, 2 x 256 59.3, 2 x 378 58.2
                 best = (t, lane)
         if best is None:
             return
