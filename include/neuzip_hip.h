@@ -332,6 +332,12 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
                                const void* dev_x, uint32_t x_rows, uint32_t in_features,
                                const void* const* dev_bias, void* const* dev_y, void* stream);
 
+/* The same for rows of any multiple of 8 elements from 512 up: a Linear whose
+   in_features the calls above refuse. */
+int nz_manager_linear_rows_batch(nz_manager* m, const char* const* names, uint32_t count,
+                                 const void* dev_x, uint32_t x_rows, uint32_t in_features,
+                                 const void* const* dev_bias, void* const* dev_y, void* stream);
+
 /* Embedding lookup on a stored table (neuzip/nn/embedding.py:30-39 decompresses
    the WHOLE table for every forward): row dev_indices[i] (int64) of the table
    `name`, read as rows of row_len elements, goes to dev_out[i * row_len ...];

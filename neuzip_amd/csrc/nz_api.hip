@@ -1315,14 +1315,15 @@ int nz_manager_read_batch(nz_manager* m, const char* const* names, void* const* 
   return NZ_OK;
 }
 
-int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t count, const void* dev_x,
-                               uint32_t x_rows, uint32_t in_features, const void* const* dev_bias,
-                               void* const* dev_y, void* stream) {
+// The fused product for rows of W that are multiples of `unit` elements (512: a group lies in one row).
+static int gemv_rows(nz_manager* m, const char* const* names, uint32_t count, const void* dev_x, uint32_t x_rows,
+                     uint32_t in_features, uint32_t unit, const void* const* dev_bias, void* const* dev_y,
+                     void* stream) {
   if (!m || !names || !dev_y || !dev_x) return fail(NZ_ERR_ARG, "null manager, names, input or outputs");
   if (count == 0 || count > NZ_BATCH_MAX) return fail(NZ_ERR_ARG, "between 1 and 16 matrices per call");
   if (x_rows == 0 || x_rows > NZ_GEMV_MAX_ROWS) return fail(NZ_ERR_ARG, "between 1 and 8 activation rows per call");
-  if (in_features == 0 || in_features % NZ_GROUP_SYMS)
-    return fail(NZ_ERR_ARG, "in_features must be a multiple of 512");
+  if (in_features < NZ_GROUP_SYMS || in_features % unit)
+    return fail(NZ_ERR_ARG, "in_features must be a multiple of " + std::to_string(unit) + ", at least 512");
   if ((uintptr_t)dev_x & 15) return fail(NZ_ERR_ALIGN, "activation must be 16-byte aligned");
   if (x_rows > 1 && m->normalizer)
     return fail(NZ_ERR_ARG, "several activation rows per call are not built for managers with normalizers");
@@ -1405,6 +1406,18 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
   }
   b.count = count;
   return gemv_launch(b, (uint32_t)grid, max_spc, m->precision, m->d_status, st);
+}
+
+int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t count, const void* dev_x,
+                               uint32_t x_rows, uint32_t in_features, const void* const* dev_bias,
+                               void* const* dev_y, void* stream) {
+  return gemv_rows(m, names, count, dev_x, x_rows, in_features, NZ_GROUP_SYMS, dev_bias, dev_y, stream);
+}
+
+int nz_manager_linear_rows_batch(nz_manager* m, const char* const* names, uint32_t count, const void* dev_x,
+                                 uint32_t x_rows, uint32_t in_features, const void* const* dev_bias,
+                                 void* const* dev_y, void* stream) {
+  return gemv_rows(m, names, count, dev_x, x_rows, in_features, NZ_GROUP, dev_bias, dev_y, stream);
 }
 
 int nz_manager_gemv_batch(nz_manager* m, const char* const* names, uint32_t count, const void* dev_x,

@@ -1784,8 +1784,9 @@ __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew
 // ----------------------------------------------------------------------------
 // y = W x for one activation row, W decoded on the fly and never written out
 // ----------------------------------------------------------------------------
-// A group of 512 consecutive weights lies inside one row of W (the row length
-// is a multiple of 512), so the row of a group is the same for all lanes.  A
+// A group is 512 consecutive weights, 8 in each lane.  The row length is a multiple of 8 and at
+// least 512, so a lane's weights lie in one row of W and a group in at most two (in one, always,
+// where the row length is a multiple of 512).  A
 // lane keeps an fp32 partial sum of its 8-element dot products; what happens
 // when the wave leaves a row is described at NzGemvWalk.  Row r owns acc[2r]
 // (fixed-point sum) and acc[2r + 1] (contribution count in the low half, flag
@@ -1800,7 +1801,7 @@ struct NzGemv {
   long long* acc;         // two words per row of this tensor and activation row (sum | count and flag), all zero between calls
   uint16_t* y;            // for each activation row one bf16 per row of the tensor
   const uint16_t* bias;   // one bf16 per row of the tensor, or null
-  uint32_t in_features;   // multiple of 512
+  uint32_t in_features;   // multiple of 8, at least 512
 };
 
 struct NzNoLds {};  // the activations of a group are not in LDS
@@ -1823,6 +1824,11 @@ __device__ __forceinline__ float nz_dot8(const uint4 w, const uint4 x, float acc
 
 // Position of a wavefront inside W while it walks its segment group by group.
 //
+// Rows need not be WHOLE groups.  Where one ends inside a group, the lanes up to there bring their
+// last products to it and the lanes behind begin the next row's sums.  Rows that are whole groups
+// have kernels of their own, because the other step costs them 4 % (one row through the Linears of
+// a block of width 4096: 163 us, 170 with a look at the row's end in every group).
+//
 // When the wave leaves a row it adds its 64 partial sums in a fixed order.  A row that lies inside the wave's segment is complete then: bias
 // added, rounded, stored.  A row shared with other segments goes through the
 // row's accumulator pair: the sum in 24.40 fixed point (integer addition is
@@ -1831,13 +1837,13 @@ __device__ __forceinline__ float nz_dot8(const uint4 w, const uint4 x, float acc
 // row comes out as NaN), and a counter of contributions; the wave that brings
 // the count to the number of segments the row touches converts, stores and
 // returns both words to zero.
-template <int MR>
+template <int MR, bool WHOLE>
 struct NzGemvWalk {
   NzGemv gv;
   uint64_t row;
   uint64_t seg_first, seg_end;  // elements of the tensor this wave covers
   uint32_t col;        // column of the current group's first element (uniform)
-  uint32_t pending;    // groups added since the last flush (uniform)
+  uint32_t pending;    // groups added since the last flush, or whether there are any (uniform)
   uint32_t seg_syms, last_syms, spc, k;  // segment lengths of a chunk, this wave's segment inside it
   uint32_t lane_off;   // bytes from a group's first activation to this lane's
   uint64_t w_rows;     // rows of the tensor (= elements between two output rows)
@@ -1861,7 +1867,8 @@ struct NzGemvWalk {
     for (int m = 0; m < MR; ++m) sum[m] = 0.f;
   }
   __device__ __forceinline__ uint32_t next_col() const {
-    return col + NZ_GROUP_SYMS == gv.in_features ? 0u : col + NZ_GROUP_SYMS;
+    if constexpr (WHOLE) return col + NZ_GROUP_SYMS == gv.in_features ? 0u : col + NZ_GROUP_SYMS;
+    return col + NZ_GROUP_SYMS >= gv.in_features ? col + NZ_GROUP_SYMS - gv.in_features : col + NZ_GROUP_SYMS;
   }
   // the lane's 8 activations of every row for the group at column c: a scalar address that goes
   // from row to row and the lane's offset.  (Addresses made of row number and stride in each lane took 30 vector
@@ -1870,8 +1877,13 @@ struct NzGemvWalk {
   __device__ __forceinline__ NzXq<MR> load(uint32_t c) const {
     NzXq<MR> r;
     uint32_t stride = 2 * gv.in_features, off = lane_off;
-    asm volatile("" : "+s"(stride), "+v"(off));  // made anew for every group; 32 bits for the offset
     const uint8_t* p = reinterpret_cast<const uint8_t*>(gv.x + c);
+    if constexpr (!WHOLE) {  // the lanes behind the end of the row are at the next one's beginning
+      p = reinterpret_cast<const uint8_t*>(gv.x);
+      off += 2 * c;
+      off = off - stride < off ? off - stride : off;
+    }
+    asm volatile("" : "+s"(stride), "+v"(off));  // made anew for every group; 32 bits for the offset
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
       r.v[m] = *reinterpret_cast<const uint4*>(p + off);
@@ -1944,12 +1956,37 @@ struct NzGemvWalk {
   }
   // add the dot products of the current group, then step to the next group
   __device__ __forceinline__ void add(const uint4 w, const NzXq<MR>& x, uint32_t lane) {
+    if constexpr (WHOLE) {
 #pragma unroll
-    for (int m = 0; m < MR; ++m) sum[m] = nz_dot8(w, x.v[m], sum[m]);
-    next(lane);
+      for (int m = 0; m < MR; ++m) sum[m] = nz_dot8(w, x.v[m], sum[m]);
+      next(lane);
+    } else {
+      const uint32_t left = gv.in_features - col;
+      col = next_col();
+      if (left > NZ_GROUP_SYMS) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m) sum[m] = nz_dot8(w, x.v[m], sum[m]);
+        pending = 1;
+      } else {
+        const bool ends = NZ_GROUP * lane < left;  // this lane's weights still belong to the row
+        float behind[MR];
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+          const float t = nz_dot8(w, x.v[m], ends ? sum[m] : 0.f);
+          sum[m] = ends ? t : sum[m];
+          behind[m] = ends ? 0.f : t;
+        }
+        flush(lane);
+        ++row;
+#pragma unroll
+        for (int m = 0; m < MR; ++m) sum[m] = behind[m];
+        pending = left < NZ_GROUP_SYMS && row < w_rows;  // (behind the last row there are no weights)
+      }
+    }
   }
   // the same with the group's activations in LDS, 64 x 16 bytes per row
   __device__ __forceinline__ void add(const uint4 w, const uint4* x, uint32_t lane) {
+    static_assert(WHOLE, "");
 #pragma unroll
     for (int m = 0; m < MR; ++m) sum[m] = nz_dot8(w, x[NZ_LANES * m + lane], sum[m]);
     next(lane);
@@ -2289,11 +2326,11 @@ struct NzWaveDecOne : NzRecord {
 // help to build the slot table).
 // With GEMV the decoded values are not stored: they are multiplied with the
 // activation `gv.x` and summed into `gv.acc` (the tensor is a row-major matrix
-// with rows of gv.in_features elements, a multiple of 512, so that no group is
-// ragged and no group straddles two rows).
+// with rows of gv.in_features elements, a multiple of 8: a lane's 8 weights exist
+// all or not at all, and belong to one row).
 // With NORM every merged value is multiplied by its group's factor (`nm`)
 // before it is stored or used.
-template <int S, int GEMV, bool NORM, bool STREAM, bool ONE>
+template <int S, int GEMV, bool NORM, bool STREAM, bool ONE, bool WHOLE = true>
 __device__ __forceinline__ void nz_decode_chunk(
     const uint8_t* __restrict__ comp, const uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
@@ -2378,7 +2415,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   // width 4096: 188 us ahead, 185 us not; eight: 255 and 256 us).
   constexpr bool X_AHEAD = MR == 1;
   NzXq<X_AHEAD ? MR : 1> xq_next{};
-  NzGemvWalk<MR> walk;
+  NzGemvWalk<MR, WHOLE> walk;
   if (has_seg && !bad_rec) {
     w.stage();
     if constexpr (GEMV) {
@@ -2536,23 +2573,31 @@ __device__ __forceinline__ void nz_decode_chunk(
     }
     const uint8_t* raw = comp + rec_start;
     const uint8_t* tailp = raw + padded;
+    const auto whole8 = [&](uint32_t idx0) __attribute__((always_inline)) {  // 8 elements of the tensor
+      const uint32_t b = idx0 / 8 * (S + 1);
+      uint64_t sy = (uint64_t)reinterpret_cast<const uint32_t*>(raw + idx0)[0] |
+                    ((uint64_t)reinterpret_cast<const uint32_t*>(raw + idx0)[1] << 32);
+      const uint64_t sm = (carry && b >= keep) ? nz_load_sm<S>(tailp + (b - keep)) : nz_load_sm<S>(pk + b);
+      uint32_t ew[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ew[j] = nz_rot_exp((uint32_t)(sy >> (8 * j)) & 0xFFu) << 24;
+      uint4 mv = nz_merge_group<S>(sm, ew);
+      if constexpr (NORM) mv = nz_scale8<true>(mv, nz_norm_load8(nm, seg_base + idx0), nm.log2n >= 3);
+      return mv;
+    };
     for (uint32_t gq = 0; gq < ngroups; ++gq) {
       const uint32_t idx0 = (gq * NZ_LANES + lane) * NZ_GROUP;
+      if constexpr (GEMV) {  // every lane takes part in the sums, behind the tensor's end with zeros
+        uint4 mv = make_uint4(0u, 0u, 0u, 0u);
+        if (WHOLE || idx0 < seg_n) mv = whole8(idx0);
+        walk.add(mv, walk.load(walk.col), lane);
+        continue;
+      }
       if (idx0 >= seg_n) continue;
       const uint32_t rem = seg_n - idx0;
-      const uint32_t b = idx0 / 8 * (S + 1);
       if (rem >= 8) {
-        uint64_t sy = (uint64_t)reinterpret_cast<const uint32_t*>(raw + idx0)[0] |
-                      ((uint64_t)reinterpret_cast<const uint32_t*>(raw + idx0)[1] << 32);
-        const uint64_t sm = (carry && b >= keep) ? nz_load_sm<S>(tailp + (b - keep)) : nz_load_sm<S>(pk + b);
-        uint32_t ew[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ew[j] = nz_rot_exp((uint32_t)(sy >> (8 * j)) & 0xFFu) << 24;
-        uint4 mv = nz_merge_group<S>(sm, ew);
-        if constexpr (NORM) mv = nz_scale8<true>(mv, nz_norm_load8(nm, seg_base + idx0), nm.log2n >= 3);
-        if constexpr (GEMV) walk.add(mv, walk.load(walk.col), lane);
-        else *reinterpret_cast<uint4*>(dst + idx0) = mv;
-      } else if constexpr (!GEMV) {
+        *reinterpret_cast<uint4*>(dst + idx0) = whole8(idx0);
+      } else {
         for (uint32_t j = 0; j < rem; ++j) {
           const uint32_t bit = (idx0 + j) * (S + 1);
           const uint32_t rp = ((uint32_t)pk[bit >> 3] >> (7u - S - (bit & 7u))) & ((2u << S) - 1u);
@@ -2574,7 +2619,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   const uint32_t incl = nz_wave_scan(nn, lane);
   const uint32_t at = incl - nn;
   const uint32_t sbytes = 16u + ((((__builtin_amdgcn_readlane(incl, 63) + 1u) >> 1) + 3u) & ~3u);
-  constexpr bool STAGED = GEMV >= NZ_STAGED_ROWS && !ONE && !NORM;
+  constexpr bool STAGED = GEMV >= NZ_STAGED_ROWS && !ONE && !NORM && WHOLE;
   uint4* const xbuf = reinterpret_cast<uint4*>(rings + 2 * RING * g.spc);
   if (damaged || rec_bytes < sbytes) {
     if (lane == 0) atomicOr(d_status, 2u);
@@ -2687,12 +2732,17 @@ __device__ __forceinline__ void nz_decode_chunk(
   };
   if (!NORM || nm.log2n >= 3) full_groups(NzConst<1>{});
   else full_groups(NzConst<0>{});
-  if (!GEMV && whole < body) {  // the ragged last group of the tensor
+  if ((!GEMV || !WHOLE) && whole < body) {  // the ragged last group of the tensor
     const uint32_t idx0 = (whole * NZ_LANES + lane) * NZ_GROUP;
     uint32_t ew[8];
     w.look();
     w.group(ew);
-    if (idx0 < seg_n) {
+    if constexpr (GEMV) {  // (rows of eights: a lane has all of its 8 elements or none)
+      const bool in = idx0 < seg_n;
+      uint4 mv = nz_merge_group<S>(in ? nz_load_sm<S>(pk + idx0 / 8 * (S + 1)) : 0ull, ew);
+      if constexpr (NORM) mv = nz_scale8<true>(mv, in ? nz_norm_load8(nm, seg_base + idx0) : 0ull, nm.log2n >= 3);
+      walk.add(mv, walk.load(walk.col), lane);
+    } else if (idx0 < seg_n) {
       const uint32_t rem = seg_n - idx0 < 8 ? seg_n - idx0 : 8;
       for (uint32_t j = 0; j < rem; ++j) {
         const uint32_t bit = (idx0 + j) * (S + 1);
@@ -2791,7 +2841,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_ke
 
 // The same walk over several matrices that multiply MR activation rows (each
 // decoded weight is used MR times before it is dropped).
-template <int S, bool NORM, int MR, bool ONE>
+template <int S, bool NORM, int MR, bool ONE, bool WHOLE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
   uint32_t t = 0, first = 0;
@@ -2801,7 +2851,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_ker
   }
   const NzBatchItem& it = b.item[t];
   const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features};
-  nz_decode_chunk<S, MR, NORM, false, ONE>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
+  nz_decode_chunk<S, MR, NORM, false, ONE, WHOLE>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
                                         blockIdx.x - first, gv, NzNorm{it.norm, b.log2n});
 }
 

@@ -74,12 +74,12 @@ void nz_launch_decode_batch(const NzBatch& b, uint32_t grid, uint32_t max_spc, b
 #undef NZ_BATCH_LAUNCH
 }
 
-template <int S, bool ONE>
+template <int S, bool ONE, bool WHOLE>
 void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
-  const size_t lds = NZ_GEMV_LDS_BYTES(max_spc, ONE, b.x_rows);
+  const size_t lds = WHOLE ? NZ_GEMV_LDS_BYTES(max_spc, ONE, b.x_rows) : NZ_DEC_LDS_BYTES(max_spc, ONE);
   const dim3 gd(grid), bd(64 * max_spc);
 #define NZ_GEMV_LAUNCH(NORM, MR) \
-  hipLaunchKernelGGL((nz_decode_gemv_kernel<S, NORM, MR, ONE>), gd, bd, lds, st, b, d_status)
+  hipLaunchKernelGGL((nz_decode_gemv_kernel<S, NORM, MR, ONE, WHOLE>), gd, bd, lds, st, b, d_status)
   // a kernel for every number of activation rows
   if (b.item[0].norm) NZ_GEMV_LAUNCH(true, 1);  // (tensors with normalizers: one row only, the caller has checked)
   else switch (b.x_rows) {
@@ -97,8 +97,14 @@ void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint
 
 template <int S>
 void nz_launch_gemv(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
-  if (nz_one_read(grid, nz_compute_units(), false)) nz_launch_gemv_form<S, true>(b, grid, max_spc, d_status, st);
-  else nz_launch_gemv_form<S, false>(b, grid, max_spc, d_status, st);
+  const bool one = nz_one_read(grid, nz_compute_units(), false);
+  if (b.in_features % NZ_GROUP_SYMS == 0) {
+    if (one) nz_launch_gemv_form<S, true, true>(b, grid, max_spc, d_status, st);
+    else nz_launch_gemv_form<S, false, true>(b, grid, max_spc, d_status, st);
+  } else {
+    if (one) nz_launch_gemv_form<S, true, false>(b, grid, max_spc, d_status, st);
+    else nz_launch_gemv_form<S, false, false>(b, grid, max_spc, d_status, st);
+  }
 }
 
 template <int S>
