@@ -341,14 +341,12 @@ int nz_manager_linear_rows_batch(nz_manager* m, const char* const* names, uint32
 /* Embedding lookup on a stored table (neuzip/nn/embedding.py:30-39 decompresses
    the WHOLE table for every forward): row dev_indices[i] (int64) of the table
    `name`, read as rows of row_len elements, goes to dev_out[i * row_len ...];
-   only the chunks that hold the requested rows are decoded.  An index outside
-   the table gives a row of zeros and makes the next nz_manager_check fail.
-   Every (row, chunk) pair is decoded on its own, so a call that asks for about
-   as many rows as the table has chunks is better served by nz_manager_read
-   (neuzip_amd.Manager.gather_rows makes that choice).  Uses the manager's write
-   scratch, at most a quarter GiB of it: larger requests are served in slices
-   (calls must be ordered on one stream with the writes).  Asynchronous on
-   `stream`. */
+   only the segments that hold the requested rows are decoded (and checked).  An
+   index outside the table gives a row of zeros and makes the next
+   nz_manager_check fail.  Every row is decoded on its own, so a call that asks
+   for several times as many rows as the table has chunks is better served by
+   nz_manager_read (neuzip_amd.Manager.gather_rows makes that choice).  Needs no
+   scratch memory.  Asynchronous on `stream`. */
 int nz_manager_gather_rows(nz_manager* m, const char* name, const void* dev_indices, uint64_t count,
                            uint32_t row_len, void* dev_out, void* stream);
 

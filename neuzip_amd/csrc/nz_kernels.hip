@@ -2321,6 +2321,29 @@ struct NzWaveDecOne : NzRecord {
   }
 };
 
+// The part of the tensor that a row gather takes from a chunk: elements [first, last] go to out[0] ...
+struct NzRowOut {
+  uint16_t* out;
+  uint64_t first, last;
+  bool vec;  // out 16-byte aligned and first a multiple of 8: groups of 8 can be stored whole
+
+  __device__ __forceinline__ bool overlaps(uint64_t from, uint32_t count) const {
+    return from <= last && from + count > first;
+  }
+  __device__ __forceinline__ void store1(uint64_t e, uint32_t h) const {
+    if (e >= first && e <= last) out[e - first] = (uint16_t)h;
+  }
+  __device__ __forceinline__ void store8(uint64_t e, const uint4 v) const {
+    if (vec && e >= first && e + 7 <= last) {
+      *reinterpret_cast<uint4*>(out + (e - first)) = v;
+    } else {
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) store1(e + j, w[j >> 1] >> (16 * (j & 1)) & 0xFFFFu);
+    }
+  }
+};
+
 // One workgroup decodes chunk `c` of one tensor; wavefront k of the workgroup
 // takes segment k of the chunk (wavefronts beyond the chunk's segments only
 // help to build the slot table).
@@ -2330,11 +2353,14 @@ struct NzWaveDecOne : NzRecord {
 // all or not at all, and belong to one row).
 // With NORM every merged value is multiplied by its group's factor (`nm`)
 // before it is stored or used.
-template <int S, int GEMV, bool NORM, bool STREAM, bool ONE, bool WHOLE = true>
+// With ROWS only the segments that hold elements of `row` are decoded, and only those elements
+// stored; the wavefronts of the others help with the table, and LDS has rings for the first
+// segment's record and for as many segments as a row can touch.
+template <int S, int GEMV, bool NORM, bool STREAM, bool ONE, bool WHOLE = true, bool ROWS = false>
 __device__ __forceinline__ void nz_decode_chunk(
     const uint8_t* __restrict__ comp, const uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
-    const NzGemv& gv, const NzNorm& nm) {
+    const NzGemv& gv, const NzNorm& nm, const NzRowOut& row = NzRowOut{}) {
   // At LDS address 0: a kernel that decodes has no static LDS (pinned in tests/test_kernel_resources.py),
   // because NzWaveDecOne numbers table and rings through from there.
   extern __shared__ uint32_t lds[];
@@ -2375,8 +2401,15 @@ __device__ __forceinline__ void nz_decode_chunk(
     if (tid == 0) atomicOr(d_status, 2u);
     return;
   }
-  const bool has_seg = wave < nseg;
+  bool has_seg = wave < nseg;
+  uint32_t ring = wave;  // whose ring
+  if constexpr (ROWS) {
+    const uint32_t from = row.first > chunk_base ? (uint32_t)((row.first - chunk_base) / g.seg_syms) : 0u;
+    has_seg = has_seg && row.overlaps(chunk_base + (uint64_t)wave * g.seg_syms, g.seg_syms);
+    ring = wave - (from > 1 ? from - 1 : 0u);  // the first segment's record, with the table, has the first one
+  }
   const uint32_t wk = has_seg ? wave : 0u;  // wavefronts without a segment only help with the table
+  if (wk == 0) ring = 0;
   const uint64_t seg_base = chunk_base + (uint64_t)wk * g.seg_syms;
   const uint32_t nom = nz_seg_nominal(g.chunk_syms, g.seg_syms, g.spc, wk);
   const uint32_t seg_n = (uint32_t)((g.n - seg_base) < nom ? (g.n - seg_base) : nom);
@@ -2392,6 +2425,14 @@ __device__ __forceinline__ void nz_decode_chunk(
   const uint64_t chunk_keep = (uint64_t)g.chunk_syms / 8 * (S + 1) - (uint64_t)NZ_CARRY_BYTES * g.spc;
   const uint8_t* pk = packed + c * chunk_keep + (uint64_t)wk * (g.seg_syms / 8 * (S + 1) - NZ_CARRY_BYTES);
   uint16_t* dst = out + seg_base;
+  const auto store1 = [&](uint32_t at, uint32_t h) __attribute__((always_inline)) {
+    if constexpr (ROWS) row.store1(seg_base + at, h);
+    else dst[at] = (uint16_t)h;
+  };
+  const auto store8 = [&](uint32_t at, const uint4 v) __attribute__((always_inline)) {
+    if constexpr (ROWS) row.store8(seg_base + at, v);
+    else *reinterpret_cast<uint4*>(dst + at) = v;
+  };
   // groups whose packed bytes are (partly) carried are merged after the loop
   const uint32_t tailg = carry ? (S == 0 ? 2u : 1u) : 0u;
   const uint32_t body = ngroups - tailg;
@@ -2404,7 +2445,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   constexpr uint32_t RING = ONE ? NZ_RING_WIDE : NZ_RING_NARROW;
   std::conditional_t<ONE || GEMV, NzWaveDecOne<RING>, NzWaveDec> w;
   w.lut = lut;
-  w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + wk * 2 * RING);
+  w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + ring * 2 * RING);
   w.nwords = rec_all / 2;
   w.lane = lane;
   uint64_t sm_next = 0, nb_next = 0;
@@ -2416,6 +2457,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   constexpr bool X_AHEAD = MR == 1;
   NzXq<X_AHEAD ? MR : 1> xq_next{};
   NzGemvWalk<MR, WHOLE> walk;
+  if (ROWS && wave == 0 && !has_seg && !bad_rec) w.stage();  // the table
   if (has_seg && !bad_rec) {
     w.stage();
     if constexpr (GEMV) {
@@ -2596,14 +2638,14 @@ __device__ __forceinline__ void nz_decode_chunk(
       if (idx0 >= seg_n) continue;
       const uint32_t rem = seg_n - idx0;
       if (rem >= 8) {
-        *reinterpret_cast<uint4*>(dst + idx0) = whole8(idx0);
+        store8(idx0, whole8(idx0));
       } else {
         for (uint32_t j = 0; j < rem; ++j) {
           const uint32_t bit = (idx0 + j) * (S + 1);
           const uint32_t rp = ((uint32_t)pk[bit >> 3] >> (7u - S - (bit & 7u))) & ((2u << S) - 1u);
           uint32_t h = nz_merge_one<S>(raw[idx0 + j], rp);
           if constexpr (NORM) h = nz_norm_mul(h, nm.bytes[(seg_base + idx0 + j) >> nm.log2n]);
-          dst[idx0 + j] = (uint16_t)h;
+          store1(idx0 + j, h);
         }
       }
     }
@@ -2683,12 +2725,14 @@ __device__ __forceinline__ void nz_decode_chunk(
     // hoisted in front of the rANS steps
     uint32_t sml = (uint32_t)sm, smh = (uint32_t)(sm >> 32);
     asm volatile("" : "+v"(sml), "+v"(smh), "+v"(ew[7]));
+    if constexpr (ROWS)
+      if (!row.overlaps(seg_base + gq * NZ_GROUP_SYMS, NZ_GROUP_SYMS)) return;
     uint4 mv = nz_merge_group<S>(((uint64_t)smh << 32) | sml, ew);
     if constexpr (NORM) mv = nz_scale8<true>(mv, nb, decltype(wide)::value);
     if constexpr (X_LDS) walk.add(mv, xl, lane);
     else if constexpr (GEMV) walk.add(mv, xq, lane);
     else if constexpr (STREAM) nz_stream_store(dst + (gq * NZ_LANES + lane) * NZ_GROUP, mv);
-    else *reinterpret_cast<uint4*>(dst + (gq * NZ_LANES + lane) * NZ_GROUP) = mv;
+    else store8((gq * NZ_LANES + lane) * NZ_GROUP, mv);
   };
   const auto full_groups = [&](auto wide) __attribute__((always_inline)) {
     uint64_t sm_a = sm_next, sm_b = 0, nb_a = nb_next, nb_b = 0;
@@ -2752,7 +2796,7 @@ __device__ __forceinline__ void nz_decode_chunk(
         for (int q = 0; q < 8; ++q) sym = (uint32_t)q == j ? nz_unrot_exp(ew[q] >> 24) : sym;
         uint32_t h = nz_merge_one<S>(sym, rp);
         if constexpr (NORM) h = nz_norm_mul(h, nm.bytes[(seg_base + idx0 + j) >> nm.log2n]);
-        dst[idx0 + j] = (uint16_t)h;
+        store1(idx0 + j, h);
       }
     }
   }
@@ -2785,7 +2829,7 @@ __device__ __forceinline__ void nz_decode_chunk(
         uint4 mv = nz_merge_group<S>(sm, ext[t]);
         if constexpr (NORM) mv = nz_scale8<true>(mv, nz_norm_load8(nm, seg_base + idx0), nm.log2n >= 3);
         if constexpr (GEMV) walk.add(mv, walk.load(walk.col), lane);
-        else *reinterpret_cast<uint4*>(dst + idx0) = mv;
+        else store8(idx0, mv);
       }
     }
   }
@@ -2856,51 +2900,36 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_ker
 }
 
 // ----------------------------------------------------------------------------
-// row gather (embedding lookup): decode only the chunks that hold the rows asked
-// for.  Workgroup (i, k) decodes the k-th chunk touched by row indices[i] into
-// slot i * cpr + k of `scratch` (a slot is one chunk of bf16 values); the copy
-// kernel then lifts the row out of its slots.  An index outside the table sets
-// status bit 8 and yields a row of zeros.
+// row gather (embedding lookup): decode only the segments that hold the rows asked
+// for.  Workgroup (i, k) takes the k-th chunk touched by row indices[i] and stores
+// what the row has of it; those of the first chunks come first, because few rows reach into
+// another.  An index outside the table sets status bit 8 and yields a row of zeros.
+//
+// Bound by the chain of one segment's steps, whatever the number of rows up to four workgroups per
+// compute unit (rows that lie in one segment take two rings, 40 KiB of LDS).  All segments
+// of a chunk, stored in a slot and copied from there by a second kernel, took 26.8 us for one row of
+// 128256 x 4096, 36.5 for 256, 51.6 for 512 and 107.6 for 1024; this takes 22.1, 23.7, 27.5 and 37.0.
+// One-read steps for any number of rows: with an eighth of the wavefronts decoding, the
+// chain is what counts.
 // ----------------------------------------------------------------------------
-template <int S, bool NORM, bool ONE>
+template <int S, bool NORM>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_rows_kernel(
     const uint8_t* __restrict__ comp, uint64_t comp_bytes, const uint8_t* __restrict__ packed,
-    uint16_t* __restrict__ scratch, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm,
+    uint16_t* __restrict__ out, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm,
     const long long* __restrict__ indices, uint32_t row_len, uint32_t cpr) {
-  const uint32_t i = blockIdx.x / cpr, k = blockIdx.x - i * cpr;
+  const uint32_t count = gridDim.x / cpr, k = blockIdx.x / count, i = blockIdx.x - k * count;
   const long long idx = indices[i];
+  uint16_t* dst = out + (uint64_t)i * row_len;
   if (idx < 0 || (uint64_t)idx >= g.n / row_len) {
-    if (threadIdx.x == 0 && k == 0) atomicOr(d_status, 8u);
+    if (k == 0) {
+      for (uint32_t e = threadIdx.x; e < row_len; e += blockDim.x) dst[e] = 0;
+      if (threadIdx.x == 0) atomicOr(d_status, 8u);
+    }
     return;
   }
   const uint64_t first = (uint64_t)idx * row_len, last = first + row_len - 1;
   const uint64_t c = first / g.chunk_syms + k;
   if (c > last / g.chunk_syms) return;
-  // the chunk function writes element e of the tensor to out[e]: shift `out` so
-  // that the chunk's first element lands at the start of this workgroup's slot
-  uint16_t* out = scratch + ((int64_t)blockIdx.x - (int64_t)c) * (int64_t)g.chunk_syms;
-  // (the slots are read back by the copy kernel right away: ordinary stores)
-  nz_decode_chunk<S, 0, NORM, false, ONE>(comp, comp_bytes, packed, out, g, d_status, c, NzGemv{}, nm);
+  const NzRowOut row{dst, first, last, ((uintptr_t)dst & 15u) == 0 && first % NZ_GROUP == 0};
+  nz_decode_chunk<S, 0, NORM, false, true, true, true>(comp, comp_bytes, packed, nullptr, g, d_status, c, NzGemv{}, nm, row);
 }
-
-#ifndef NZ_TEMPLATES_ONLY
-// `bx` workgroups per row, rows along the same grid dimension (no limit of
-// 65535 rows); `i` counts from the start of the slice the scratch holds.
-__global__ __launch_bounds__(256) void nz_copy_rows_kernel(const uint16_t* __restrict__ scratch,
-                                                           const long long* __restrict__ indices,
-                                                           uint64_t rows, uint32_t row_len,
-                                                           uint32_t chunk_syms, uint32_t cpr, uint32_t bx,
-                                                           uint16_t* __restrict__ out) {
-  const uint32_t i = blockIdx.x / bx, part = blockIdx.x - i * bx;
-  const long long idx = indices[i];
-  const bool ok = idx >= 0 && (uint64_t)idx < rows;
-  const uint64_t first = ok ? (uint64_t)idx * row_len : 0;
-  const uint64_t c0 = first / chunk_syms;
-  for (uint32_t e = part * 256 + threadIdx.x; e < row_len; e += bx * 256) {
-    const uint64_t ge = first + e;
-    const uint64_t c = ge / chunk_syms;
-    const uint16_t v = ok ? scratch[((uint64_t)i * cpr + (c - c0)) * chunk_syms + (ge - c * chunk_syms)] : 0;
-    out[(uint64_t)i * row_len + e] = v;
-  }
-}
-#endif  // NZ_TEMPLATES_ONLY
