@@ -2443,7 +2443,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   const uint32_t lane_off = lane * (S + 1);
   const uint32_t last_off = whole ? (whole - 1) * NZ_LANES * (S + 1) + lane_off : 0u;
   constexpr uint32_t RING = ONE ? NZ_RING_WIDE : NZ_RING_NARROW;
-  std::conditional_t<ONE || GEMV, NzWaveDecOne<RING>, NzWaveDec> w;
+  std::conditional_t<ONE || GEMV || ROWS, NzWaveDecOne<RING>, NzWaveDec> w;
   w.lut = lut;
   w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + ring * 2 * RING);
   w.nwords = rec_all / 2;
@@ -2709,7 +2709,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide, auto fetch_ahead,
                               auto xl) __attribute__((always_inline)) {
     constexpr bool X_LDS = !std::is_same_v<decltype(xl), NzNoLds>;
-    if constexpr (ONE || GEMV) w.look();  // before the group's loads: a refill waits for all that are under way
+    if constexpr (ONE || GEMV || ROWS) w.look();  // before the group's loads: a refill waits for all that are under way
     NzXq<MR> xq;
     if constexpr (GEMV && X_AHEAD) {
       xq = xq_next;
@@ -2718,7 +2718,7 @@ __device__ __forceinline__ void nz_decode_chunk(
       xq = walk.load(walk.col);
     }
     fetch_ahead();  // behind the activations: their wait is then not for bytes from memory as well (eight rows: 265 -> 260 us)
-    if constexpr (!ONE && !GEMV) w.look();  // (behind them here: 143 us for 8192 x 28672, before them 145)
+    if constexpr (!ONE && !GEMV && !ROWS) w.look();  // (behind them here: 143 us for 8192 x 28672, before them 145)
     uint32_t ew[8];
     w.group(ew);
     // the merge starts only here: its wait for the packed bytes must not be
@@ -2908,11 +2908,11 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_ker
 // Bound by the chain of one segment's steps, whatever the number of rows up to four workgroups per
 // compute unit (rows that lie in one segment take two rings, 40 KiB of LDS).  All segments
 // of a chunk, stored in a slot and copied from there by a second kernel, took 26.8 us for one row of
-// 128256 x 4096, 36.5 for 256, 51.6 for 512 and 107.6 for 1024; this takes 22.1, 23.7, 27.5 and 37.0.
-// One-read steps for any number of rows: with an eighth of the wavefronts decoding, the
-// chain is what counts.
+// 128256 x 4096, 36.5 for 256, 51.6 for 512 and 107.6 for 1024; this takes 22.1, 23.5, 28.7 and 38.0.
+// One-read steps for any number of rows (with an eighth of the wavefronts decoding, the chain is
+// what counts), with the narrow ring where there are more workgroups than compute units.
 // ----------------------------------------------------------------------------
-template <int S, bool NORM>
+template <int S, bool NORM, bool WIDE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_rows_kernel(
     const uint8_t* __restrict__ comp, uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm,
@@ -2931,5 +2931,5 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_rows_ker
   const uint64_t c = first / g.chunk_syms + k;
   if (c > last / g.chunk_syms) return;
   const NzRowOut row{dst, first, last, ((uintptr_t)dst & 15u) == 0 && first % NZ_GROUP == 0};
-  nz_decode_chunk<S, 0, NORM, false, true, true, true>(comp, comp_bytes, packed, nullptr, g, d_status, c, NzGemv{}, nm, row);
+  nz_decode_chunk<S, 0, NORM, false, WIDE, true, true>(comp, comp_bytes, packed, nullptr, g, d_status, c, NzGemv{}, nm, row);
 }

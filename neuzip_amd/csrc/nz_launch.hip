@@ -114,14 +114,20 @@ void nz_launch_rows(const NzGeom& g, const void* comp, uint64_t comp_bytes, cons
   // segments of a chunk that a row can touch (one more where the chunk's last is a short one), and the table's record
   const bool aligned = g.seg_syms % row_len == 0 && g.chunk_syms % g.seg_syms == 0;
   const uint64_t touched = aligned ? 1u : ((uint64_t)row_len + g.seg_syms - 2) / g.seg_syms + 2;
-  const size_t lds = NZ_DEC_LDS_BYTES(touched + 1 < g.spc ? (uint32_t)touched + 1 : g.spc, true);
+  const bool one = nz_one_read((uint64_t)count * cpr, nz_compute_units(), false);
+  const size_t lds = NZ_DEC_LDS_BYTES(touched + 1 < g.spc ? (uint32_t)touched + 1 : g.spc, one);
   const dim3 gd(count * cpr), bd(64 * g.spc);
-  if (nm.bytes)
-    hipLaunchKernelGGL((nz_decode_rows_kernel<S, true>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes,
-                       (const uint8_t*)packed, out, g, d_status, nm, idx, row_len, cpr);
-  else
-    hipLaunchKernelGGL((nz_decode_rows_kernel<S, false>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes,
-                       (const uint8_t*)packed, out, g, d_status, nm, idx, row_len, cpr);
+#define NZ_ROWS_LAUNCH(NORM, WIDE)                                                                               \
+  hipLaunchKernelGGL((nz_decode_rows_kernel<S, NORM, WIDE>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes, \
+                     (const uint8_t*)packed, out, g, d_status, nm, idx, row_len, cpr)
+  if (nm.bytes) {
+    if (one) NZ_ROWS_LAUNCH(true, true);
+    else NZ_ROWS_LAUNCH(true, false);
+  } else {
+    if (one) NZ_ROWS_LAUNCH(false, true);
+    else NZ_ROWS_LAUNCH(false, false);
+  }
+#undef NZ_ROWS_LAUNCH
 }
 
 // NZ_PART (optional) cuts the unit into parts that a build can compile side by side:
