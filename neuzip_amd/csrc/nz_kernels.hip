@@ -830,13 +830,15 @@ struct NzEncItem {
   uint64_t pub, nonce;
   uint64_t* d_gave_up;
   uint32_t direct, spin_limit;
-  // two words in ws (offset): [0] counts the direct encodes that have used this
+  // three words in ws (offset): [0] counts the direct encodes that have used this
   // scratch, advanced by the workgroup of the last chunk - the announcements'
   // mark is made of it and the nonce, so those of an earlier run of the very
   // same call (a replayed graph) do not pass for this run's; [1] holds
   // NZ_LOOKBACK_ABORT after a run in which a workgroup gave up: the next run
   // then leaves the placing to nz_compact_kernel as well (and says so through
-  // the same flags) and takes the mark away.  Whatever the memory held
+  // the same flags) and takes the mark away; [2] is set to what [0] becomes by a
+  // run that leaves a record out of the container, whatever the reason (a reader behind
+  // it on the stream goes by that: nz_late_kernel).  Whatever the memory held
   // before its first use is as good a start as any.
   uint64_t lb_state;
   // `placed`: one byte per segment (offset into ws), left by a direct encode: 1 =
@@ -1250,12 +1252,16 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
   const uint32_t lb_gen = L.lb[0];  // (only now: kept since the beginning, it was spilled for the coding phase)
   uint8_t* placed = it.ws + it.placed;  // per segment: its record is in the container and nowhere else
   const bool last_chunk = c + 1 == g.n_chunks;
+  const auto left_out = [&] {
+    __hip_atomic_store(lb_state + 2, lb_gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   if (!places()) {
     // the run before this one ended with a workgroup giving up: nothing is
     // placed, the caller is told, and the mark is taken away for the next run
     if (tid == 0) {
       atomicOr(it.d_status, 4u);
       if (it.d_gave_up) *it.d_gave_up = it.nonce;
+      left_out();
       if (last_chunk) {
         __hip_atomic_store(lb_state, lb_gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(lb_state + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1373,6 +1379,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
       __hip_atomic_store(lb_state + 1, NZ_LOOKBACK_ABORT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       atomicOr(it.d_status, 4u);
       if (it.d_gave_up) *it.d_gave_up = it.nonce;
+      left_out();
       if (last_chunk) __hip_atomic_store(lb_state, lb_gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (has_seg) {
@@ -1409,7 +1416,10 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
     const bool fits = nz_move_record<64>(it, seg, c, wave, o0, L.seg_units[wave], ci, L.seg_sb[wave],
                                          cap_words - pos_end, L.ser, L.sbuf[wave], words, nullptr, lane);
     if (from_stage && !fits) unstage();
-    if (lane == 0) placed[seg] = (from_stage && fits) ? 1 : 0;
+    if (lane == 0) {
+      placed[seg] = (from_stage && fits) ? 1 : 0;
+      if (!fits) left_out();
+    }
   }
   NZ_PROBE_MARK(5);
 }
@@ -1583,21 +1593,13 @@ __global__ __launch_bounds__(256) void nz_total_kernel(const NzEncBatch b) {
 // The workgroup of segment k of chunk c finds where its record goes by itself:
 // the record sizes of all chunks before c (one number per chunk, left by the
 // encode kernel) plus those of the segments before k in c.
-__global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
-  __shared__ uint64_t red4[4];
-  uint32_t t = 0, first = 0;
-  while (t + 1 < b.count && blockIdx.x >= b.item[t].seg_end) {
-    first = b.item[t].seg_end;
-    ++t;
-  }
-  const NzEncItem& it = b.item[t];
+__device__ __forceinline__ void nz_compact_segment(const NzEncItem& it, const uint64_t seg, uint64_t* red4) {
   const NzGeom& g = it.g;
   const NzChunkInfo* __restrict__ info = reinterpret_cast<const NzChunkInfo*>(it.ws + it.info);
   const uint32_t* __restrict__ seg_words = reinterpret_cast<const uint32_t*>(it.ws + it.seg_words);
   const uint32_t* __restrict__ seg_state_bytes = reinterpret_cast<const uint32_t*>(it.ws + it.seg_sbytes);
   const uint32_t* __restrict__ seg_units = reinterpret_cast<const uint32_t*>(it.ws + it.seg_units);
   const uint32_t* __restrict__ chunk_units = reinterpret_cast<const uint32_t*>(it.ws + it.chunk_units);
-  const uint64_t seg = blockIdx.x - first;
   const uint64_t c = seg / g.spc;
   const uint32_t k = (uint32_t)(seg - c * g.spc);
   const uint32_t tid = threadIdx.x;
@@ -1616,6 +1618,31 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
                       reinterpret_cast<const uint32_t*>(it.ws + it.tab_ser + c * NZ_TABLE_MAX_BYTES),
                       reinterpret_cast<const uint32_t*>(it.ws + it.states) + seg * (NZ_STATE_MAX_BYTES / 4), words,
                       in_old ? it.old_comp + g.rec_off + 4 * o0 : nullptr, tid);
+}
+__global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
+  __shared__ uint64_t red4[4];
+  uint32_t t = 0, first = 0;
+  while (t + 1 < b.count && blockIdx.x >= b.item[t].seg_end) {
+    first = b.item[t].seg_end;
+    ++t;
+  }
+  nz_compact_segment(b.item[t], blockIdx.x - first, red4);
+}
+// Between an in-place write and a read that the host enqueues before it knows how the write went:
+// the tensors of which the write has left a record out of the container (it outgrew its buffer, or
+// a chunk gave up waiting) are put together again in a buffer that holds any container, and the read
+// goes by the same two words (NzBatchItem::late).  There is next to never anything to do, so the grid
+// is small, and the words of all tensors are looked at together: 1.5 to 3 us (64 workgroups that look at one
+// tensor after the other: 4.3).
+__global__ __launch_bounds__(256) void nz_late_kernel(const NzEncBatch b) {
+  __shared__ uint64_t red4[4];
+  const uint32_t lane = threadIdx.x & 63, mine = lane < b.count ? lane : 0;  // all tensors' words at once
+  const uint2* state = reinterpret_cast<const uint2*>(b.item[mine].ws + b.item[mine].lb_state);
+  const uint32_t run = state[0].x, left_out = state[1].x;
+  for (uint64_t todo = __ballot(lane < b.count && run == left_out); todo; todo &= todo - 1) {
+    const NzEncItem& it = b.item[__builtin_ctzll(todo)];
+    for (uint64_t seg = blockIdx.x; seg < it.g.n_segs; seg += gridDim.x) nz_compact_segment(it, seg, red4);
+  }
 }
 
 #endif  // NZ_TEMPLATES_ONLY
@@ -2860,6 +2887,11 @@ struct NzBatchItem {
   NzGeom g;
   uint32_t chunk_end;
   uint32_t reserved;
+  // dense output of a tensor whose last write is not known to have fitted its buffer: the run count and
+  // mark of that write's scratch (NzEncItem::lb_state; null: all is known), and the container to take if they agree
+  const uint32_t* late;
+  const uint8_t* late_comp;
+  uint64_t late_bytes;
 };
 struct NzBatch {
   uint32_t count;
@@ -2879,8 +2911,10 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_ke
     ++t;
   }
   const NzBatchItem& it = b.item[t];
-  nz_decode_chunk<S, 0, NORM, STREAM, ONE>(it.comp, it.comp_bytes, it.packed, it.out, it.g, d_status,
-                                          blockIdx.x - first, NzGemv{}, NzNorm{it.norm, b.log2n});
+  const bool other = it.late && it.late[2] == it.late[0];
+  nz_decode_chunk<S, 0, NORM, STREAM, ONE>(other ? it.late_comp : it.comp, other ? it.late_bytes : it.comp_bytes,
+                                          it.packed, it.out, it.g, d_status, blockIdx.x - first, NzGemv{},
+                                          NzNorm{it.norm, b.log2n});
 }
 
 // The same walk over several matrices that multiply MR activation rows (each
