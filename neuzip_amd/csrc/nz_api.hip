@@ -327,7 +327,7 @@ int decode_launch(const NzGeom& g, int precision, const void* comp, uint64_t com
 }
 
 // all items of one launch share the output policy (`stream_out`)
-int decode_batch_launch(const NzBatch& b, uint32_t grid, uint32_t max_spc, int precision, bool stream_out,
+int decode_batch_launch(NzBatch& b, uint32_t grid, uint32_t max_spc, int precision, bool stream_out,
                         uint32_t* d_status, hipStream_t st) {
   if (grid == 0) return NZ_OK;
   switch (precision) {
@@ -340,7 +340,7 @@ int decode_batch_launch(const NzBatch& b, uint32_t grid, uint32_t max_spc, int p
   return NZ_OK;
 }
 
-int gemv_launch(const NzBatch& b, uint32_t grid, uint32_t max_spc, int precision, uint32_t* d_status,
+int gemv_launch(NzBatch& b, uint32_t grid, uint32_t max_spc, int precision, uint32_t* d_status,
                 hipStream_t st) {
   switch (precision) {
     case 7: nz_launch_gemv<7>(b, grid, max_spc, d_status, st); break;

@@ -1788,6 +1788,23 @@ static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 3
 NZ_HD static inline bool nz_one_read(uint64_t workgroups, uint32_t compute_units, bool stream_out) {
   return !stream_out && workgroups <= compute_units;
 }
+// Workgroups that share a chunk, where a launch would leave compute units idle: each builds the slot
+// table, and decodes an equal part of the segments.  A wavefront with a SIMD unit to itself takes its
+// steps faster than one of two, of which the younger waits for the older (140 and 158 cycles per step in a
+// workgroup of eight), and the wavefronts of a compute unit share its LDS and vector L1.  Reads of 8, 32,
+// 64 and 128 chunks 25.1, 24.9, 26.2, 27.9 -> 22.3, 22.2, 23.8, 25.1 us, products of eight
+// rows 36.4, 35.1, 32.6, 33.0 -> 30.2, 29.1, 27.3, 27.9; 160 chunks, which stay whole, 28.4 and 33.4.  Four and
+// eight streams with 128 chunks each, at once: 212 and 419 us either way; with rings for whole chunks 239 and 484.
+#define NZ_MAX_PARTS 8u
+NZ_HD static inline uint32_t nz_parts(uint64_t chunks, uint32_t spc, uint32_t compute_units, bool stream_out) {
+  uint32_t parts = 1;
+  while (!stream_out && 2 * parts <= spc && 2 * parts <= NZ_MAX_PARTS && 2 * parts * chunks <= compute_units) parts *= 2;
+  return parts;
+}
+// rings that a workgroup needs: its segments', and the first one's for the table
+NZ_HD static inline uint32_t nz_part_rings(uint32_t spc, uint32_t parts) {
+  return parts > 1 ? (spc + parts - 1) / parts + 1 : spc;
+}
 
 // S+1 packed bytes of one 8-element group, as a little-endian integer
 template <int S>
@@ -2461,6 +2478,7 @@ struct NzRowOut {
 // all or not at all, and belong to one row).
 // With NORM every merged value is multiplied by its group's factor (`nm`)
 // before it is stored or used.
+// Where several workgroups share the chunk, this one's segments are from first_seg to before end_seg.
 // With ROWS only the segments that hold elements of `row` are decoded, and only those elements
 // stored; the wavefronts of the others help with the table, and LDS has rings for the first
 // segment's record and for as many segments as a row can touch.
@@ -2468,7 +2486,8 @@ template <int S, int GEMV, bool NORM, bool STREAM, bool ONE, bool WHOLE = true, 
 __device__ __forceinline__ void nz_decode_chunk(
     const uint8_t* __restrict__ comp, const uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
-    const NzGemv& gv, const NzNorm& nm, const NzRowOut& row = NzRowOut{}) {
+    const NzGemv& gv, const NzNorm& nm, const uint32_t first_seg, const uint32_t end_seg,
+    const NzRowOut& row = NzRowOut{}) {
   // At LDS address 0: a kernel that decodes has no static LDS (pinned in tests/test_kernel_resources.py),
   // because NzWaveDecOne numbers table and rings through from there.
   extern __shared__ uint32_t lds[];
@@ -2509,12 +2528,12 @@ __device__ __forceinline__ void nz_decode_chunk(
     if (tid == 0) atomicOr(d_status, 2u);
     return;
   }
-  bool has_seg = wave < nseg;
-  uint32_t ring = wave;  // whose ring
+  bool has_seg = wave < nseg && wave >= first_seg && wave < end_seg;
+  uint32_t ring = wave - first_seg + (first_seg ? 1u : 0u);  // the first segment's record, with the table, has the first one
   if constexpr (ROWS) {
     const uint32_t from = row.first > chunk_base ? (uint32_t)((row.first - chunk_base) / g.seg_syms) : 0u;
     has_seg = has_seg && row.overlaps(chunk_base + (uint64_t)wave * g.seg_syms, g.seg_syms);
-    ring = wave - (from > 1 ? from - 1 : 0u);  // the first segment's record, with the table, has the first one
+    ring = wave - (from > 1 ? from - 1 : 0u);
   }
   const uint32_t wk = has_seg ? wave : 0u;  // wavefronts without a segment only help with the table
   if (wk == 0) ring = 0;
@@ -2565,7 +2584,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   constexpr bool X_AHEAD = MR == 1;
   NzXq<X_AHEAD ? MR : 1> xq_next{};
   NzGemvWalk<MR, WHOLE> walk;
-  if (ROWS && wave == 0 && !has_seg && !bad_rec) w.stage();  // the table
+  if (wave == 0 && !has_seg && !bad_rec) w.stage();  // the table
   if (has_seg && !bad_rec) {
     w.stage();
     if constexpr (GEMV) {
@@ -2945,11 +2964,24 @@ __device__ __forceinline__ void nz_decode_chunk(
     if (walk.pending) walk.flush(lane);
 }
 
+// Workgroup b of a launch in which `parts` share a chunk: which chunk (of the launch), which of its segments.
+struct NzPart {
+  uint32_t chunk, first, end;
+  __device__ __forceinline__ NzPart(uint32_t b, uint32_t parts, uint32_t spc) {
+    const uint32_t l = 31u - (uint32_t)__builtin_clz(parts);  // (a power of two)
+    chunk = b >> l;
+    const uint32_t per = (spc + parts - 1) >> l;
+    first = (b & (parts - 1)) * per;
+    end = first + per;
+  }
+};
+
 template <int S, bool NORM, bool STREAM, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_kernel(
     const uint8_t* __restrict__ comp, uint64_t comp_bytes, const uint8_t* __restrict__ packed,
-    uint16_t* __restrict__ out, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm) {
-  nz_decode_chunk<S, 0, NORM, STREAM, ONE>(comp, comp_bytes, packed, out, g, d_status, blockIdx.x, NzGemv{}, nm);
+    uint16_t* __restrict__ out, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm, const uint32_t parts) {
+  const NzPart p(blockIdx.x, parts, g.spc);
+  nz_decode_chunk<S, 0, NORM, STREAM, ONE>(comp, comp_bytes, packed, out, g, d_status, p.chunk, NzGemv{}, nm, p.first, p.end);
 }
 
 // Several tensors in one launch: the grid is the concatenation of their
@@ -2981,21 +3013,24 @@ struct NzBatch {
   uint32_t log2n;        // normalized tensors only
   uint32_t x_rows;       // matrix-vector product only: activation rows (1..8)
   NzBatchItem item[NZ_BATCH_MAX];
+  uint32_t parts;        // workgroups that share a chunk (nz_parts)
 };
 
 template <int S, bool NORM, bool STREAM, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
   uint32_t t = 0, first = 0;
-  while (t + 1 < b.count && blockIdx.x >= b.item[t].chunk_end) {
+  const uint32_t at = blockIdx.x >> (31u - (uint32_t)__builtin_clz(b.parts));
+  while (t + 1 < b.count && at >= b.item[t].chunk_end) {
     first = b.item[t].chunk_end;
     ++t;
   }
   const NzBatchItem& it = b.item[t];
+  const NzPart p(blockIdx.x, b.parts, it.g.spc);
   const bool other = it.late && it.late[2] == it.late[0];
   nz_decode_chunk<S, 0, NORM, STREAM, ONE>(other ? it.late_comp : it.comp, other ? it.late_bytes : it.comp_bytes,
-                                          it.packed, it.out, it.g, d_status, blockIdx.x - first, NzGemv{},
-                                          NzNorm{it.norm, b.log2n});
+                                          it.packed, it.out, it.g, d_status, at - first, NzGemv{},
+                                          NzNorm{it.norm, b.log2n}, p.first, p.end);
 }
 
 // The same walk over several matrices that multiply MR activation rows (each
@@ -3004,14 +3039,16 @@ template <int S, bool NORM, int MR, bool ONE, bool WHOLE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
   uint32_t t = 0, first = 0;
-  while (t + 1 < b.count && blockIdx.x >= b.item[t].chunk_end) {
+  const uint32_t at = blockIdx.x >> (31u - (uint32_t)__builtin_clz(b.parts));
+  while (t + 1 < b.count && at >= b.item[t].chunk_end) {
     first = b.item[t].chunk_end;
     ++t;
   }
   const NzBatchItem& it = b.item[t];
+  const NzPart p(blockIdx.x, b.parts, it.g.spc);
   const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features};
   nz_decode_chunk<S, MR, NORM, false, ONE, WHOLE>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
-                                        blockIdx.x - first, gv, NzNorm{it.norm, b.log2n});
+                                        at - first, gv, NzNorm{it.norm, b.log2n}, p.first, p.end);
 }
 
 // ----------------------------------------------------------------------------
@@ -3046,5 +3083,6 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_rows_ker
   const uint64_t c = first / g.chunk_syms + k;
   if (c > last / g.chunk_syms) return;
   const NzRowOut row{dst, first, last, ((uintptr_t)dst & 15u) == 0 && first % NZ_GROUP == 0};
-  nz_decode_chunk<S, 0, NORM, false, WIDE, true, true>(comp, comp_bytes, packed, nullptr, g, d_status, c, NzGemv{}, nm, row);
+  nz_decode_chunk<S, 0, NORM, false, WIDE, true, true>(comp, comp_bytes, packed, nullptr, g, d_status, c, NzGemv{}, nm, 0, g.spc,
+                                                          row);
 }

@@ -27,11 +27,11 @@ void nz_launch_decode(const NzGeom& g, const void* comp, uint64_t comp_bytes, co
                       uint32_t* d_status, const NzNorm& nm, uint32_t stream_out, hipStream_t st);
 
 template <int S>
-void nz_launch_decode_batch(const NzBatch& b, uint32_t grid, uint32_t max_spc, bool stream_out, uint32_t* d_status,
+void nz_launch_decode_batch(NzBatch& b, uint32_t grid, uint32_t max_spc, bool stream_out, uint32_t* d_status,
                             hipStream_t st);
 
 template <int S>
-void nz_launch_gemv(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st);
+void nz_launch_gemv(NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st);
 
 template <int S>
 void nz_launch_rows(const NzGeom& g, const void* comp, uint64_t comp_bytes, const void* packed, uint16_t* out,
@@ -44,8 +44,8 @@ void nz_launch_rows(const NzGeom& g, const void* comp, uint64_t comp_bytes, cons
   extern template void nz_launch_encode<S>(const NzEncBatch&, int, dim3, dim3, uint32_t, hipStream_t);               \
   extern template void nz_launch_decode<S>(const NzGeom&, const void*, uint64_t, const void*, void*, uint32_t*,      \
                                            const NzNorm&, uint32_t, hipStream_t);                                    \
-  extern template void nz_launch_decode_batch<S>(const NzBatch&, uint32_t, uint32_t, bool, uint32_t*, hipStream_t);  \
-  extern template void nz_launch_gemv<S>(const NzBatch&, uint32_t, uint32_t, uint32_t*, hipStream_t);                \
+  extern template void nz_launch_decode_batch<S>(NzBatch&, uint32_t, uint32_t, bool, uint32_t*, hipStream_t);  \
+  extern template void nz_launch_gemv<S>(NzBatch&, uint32_t, uint32_t, uint32_t*, hipStream_t);                \
   extern template void nz_launch_rows<S>(const NzGeom&, const void*, uint64_t, const void*, uint16_t*, uint32_t*,    \
                                          const NzNorm&, const long long*, uint32_t, uint32_t, uint32_t, hipStream_t);
 NZ_DECLARE_PRECISION(7)

@@ -37,11 +37,12 @@ template <int S>
 void nz_launch_decode(const NzGeom& g, const void* comp, uint64_t comp_bytes, const void* packed, void* out,
                       uint32_t* d_status, const NzNorm& nm, uint32_t stream_out, hipStream_t st) {
   const bool one = nz_one_read(g.n_chunks, nz_compute_units(), stream_out);
-  const size_t lds = NZ_DEC_LDS_BYTES(g.spc, one);
-  const dim3 gd((uint32_t)g.n_chunks), bd(64 * g.spc);
+  const uint32_t parts = nz_parts(g.n_chunks, g.spc, nz_compute_units(), stream_out);
+  const size_t lds = NZ_DEC_LDS_BYTES(nz_part_rings(g.spc, parts), one);
+  const dim3 gd((uint32_t)g.n_chunks * parts), bd(64 * g.spc);
 #define NZ_DEC_LAUNCH(NORM, STREAM, ONE)                                                                       \
   hipLaunchKernelGGL((nz_decode_kernel<S, NORM, STREAM, ONE>), gd, bd, lds, st, (const uint8_t*)comp, comp_bytes, \
-                     (const uint8_t*)packed, (uint16_t*)out, g, d_status, nm)
+                     (const uint8_t*)packed, (uint16_t*)out, g, d_status, nm, parts)
   if (nm.bytes) {
     if (stream_out) NZ_DEC_LAUNCH(true, true, false);
     else if (one) NZ_DEC_LAUNCH(true, false, true);
@@ -55,11 +56,12 @@ void nz_launch_decode(const NzGeom& g, const void* comp, uint64_t comp_bytes, co
 }
 
 template <int S>
-void nz_launch_decode_batch(const NzBatch& b, uint32_t grid, uint32_t max_spc, bool stream_out, uint32_t* d_status,
+void nz_launch_decode_batch(NzBatch& b, uint32_t grid, uint32_t max_spc, bool stream_out, uint32_t* d_status,
                             hipStream_t st) {
   const bool one = nz_one_read(grid, nz_compute_units(), stream_out);
-  const size_t lds = NZ_DEC_LDS_BYTES(max_spc, one);
-  const dim3 gd(grid), bd(64 * max_spc);
+  b.parts = nz_parts(grid, max_spc, nz_compute_units(), stream_out);
+  const size_t lds = NZ_DEC_LDS_BYTES(nz_part_rings(max_spc, b.parts), one);
+  const dim3 gd(grid * b.parts), bd(64 * max_spc);
 #define NZ_BATCH_LAUNCH(NORM, STREAM, ONE) \
   hipLaunchKernelGGL((nz_decode_batch_kernel<S, NORM, STREAM, ONE>), gd, bd, lds, st, b, d_status)
   if (b.item[0].norm) {
@@ -76,8 +78,9 @@ void nz_launch_decode_batch(const NzBatch& b, uint32_t grid, uint32_t max_spc, b
 
 template <int S, bool ONE, bool WHOLE>
 void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
-  const size_t lds = WHOLE ? NZ_GEMV_LDS_BYTES(max_spc, ONE, b.x_rows) : NZ_DEC_LDS_BYTES(max_spc, ONE);
-  const dim3 gd(grid), bd(64 * max_spc);
+  const size_t lds = WHOLE && b.parts == 1 ? NZ_GEMV_LDS_BYTES(max_spc, ONE, b.x_rows)
+                                           : NZ_DEC_LDS_BYTES(nz_part_rings(max_spc, b.parts), ONE);
+  const dim3 gd(grid * b.parts), bd(64 * max_spc);
 #define NZ_GEMV_LAUNCH(NORM, MR) \
   hipLaunchKernelGGL((nz_decode_gemv_kernel<S, NORM, MR, ONE, WHOLE>), gd, bd, lds, st, b, d_status)
   // a kernel for every number of activation rows
@@ -96,7 +99,8 @@ void nz_launch_gemv_form(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint
 }
 
 template <int S>
-void nz_launch_gemv(const NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
+void nz_launch_gemv(NzBatch& b, uint32_t grid, uint32_t max_spc, uint32_t* d_status, hipStream_t st) {
+  b.parts = nz_parts(grid, max_spc, nz_compute_units(), false);
   const bool one = nz_one_read(grid, nz_compute_units(), false);
   if (b.in_features % NZ_GROUP_SYMS == 0) {
     if (one) nz_launch_gemv_form<S, true, true>(b, grid, max_spc, d_status, st);
@@ -142,10 +146,10 @@ template void nz_launch_encode<NZ_S>(const NzEncBatch&, int, dim3, dim3, uint32_
 #if !defined(NZ_PART) || NZ_PART == 1 || NZ_PART == 12
 template void nz_launch_decode<NZ_S>(const NzGeom&, const void*, uint64_t, const void*, void*, uint32_t*, const NzNorm&,
                                      uint32_t, hipStream_t);
-template void nz_launch_decode_batch<NZ_S>(const NzBatch&, uint32_t, uint32_t, bool, uint32_t*, hipStream_t);
+template void nz_launch_decode_batch<NZ_S>(NzBatch&, uint32_t, uint32_t, bool, uint32_t*, hipStream_t);
 #endif
 #if !defined(NZ_PART) || NZ_PART == 2 || NZ_PART == 12
-template void nz_launch_gemv<NZ_S>(const NzBatch&, uint32_t, uint32_t, uint32_t*, hipStream_t);
+template void nz_launch_gemv<NZ_S>(NzBatch&, uint32_t, uint32_t, uint32_t*, hipStream_t);
 #endif
 #if !defined(NZ_PART) || NZ_PART == 1 || NZ_PART == 12
 template void nz_launch_rows<NZ_S>(const NzGeom&, const void*, uint64_t, const void*, uint16_t*, uint32_t*,
