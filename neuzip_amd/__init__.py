@@ -39,6 +39,12 @@ def compressed_lomo_hook(scheduler, param):
     with torch.no_grad():
         dense = param()
         dense.add_(grad_w, alpha=-_current_lr(scheduler))
-        param._manager.write(dense, param._handle)
+        # nobody else holds `dense` (unless a part in this has been replaced): it needs no copy to wait for its write
+        manager = param._manager
+        if (type(manager) is Manager and type(param) is nn.Parameter
+                and not {"read", "write"} & manager.__dict__.keys()):
+            manager._give(dense, param._handle)
+        else:
+            manager.write(dense, param._handle)
     param._gradient = None
     param.grad = None
