@@ -2600,7 +2600,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   // the first 32 table bytes hold the mode and all run descriptors there can be
   const uint4 h0 = reinterpret_cast<const uint4*>(tb)[0], h1 = reinterpret_cast<const uint4*>(tb)[1];
   const uint32_t bm_byte = tb[1 + (lane >> 1)];  // bitmap mode: the byte with this lane's four symbols
-  const uint32_t mode = h0.x & 0xFFu;
+  const uint32_t mode = (uint32_t)__builtin_amdgcn_readfirstlane(h0.x) & 0xFFu;
   uint32_t tab_len = 4;
 
   if (mode != NZ_MODE_RAW) {
@@ -2627,23 +2627,28 @@ __device__ __forceinline__ void nz_decode_chunk(
         for (uint32_t j = 0; j < 4; ++j) rk[j] = ci - c + (uint32_t)__popc(live4 & ((1u << j) - 1u));
       } else {
         head = 1 + 2 * mode;
-        const uint32_t hw[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+        // the run descriptors, 16 bits each from the second byte on, move down through scalar registers
+        const auto pair = [](uint32_t lo, uint32_t hi) {
+          return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(lo) | ((uint64_t)__builtin_amdgcn_readfirstlane(hi) << 32);
+        };
+        uint64_t q0 = pair(h0.x, h0.y), q1 = pair(h0.z, h0.w), q2 = pair(h1.x, h1.y), q3 = pair(h1.z, h1.w);
         uint32_t acc = 0;
+#pragma nounroll
+        for (uint32_t r = 0; r < mode; ++r) {
+          const uint32_t st = (uint32_t)(q0 >> 8) & 0xFFu, ln = ((uint32_t)(q0 >> 16) & 0xFFu) + 1u;
+          q0 = q0 >> 16 | q1 << 48;
+          q1 = q1 >> 16 | q2 << 48;
+          q2 = q2 >> 16 | q3 << 48;
+          q3 >>= 16;
 #pragma unroll
-        for (uint32_t r = 0; r < NZ_MAX_RUNS; ++r) {
-          if (r < mode) {
-            const uint32_t st = (hw[(1 + 2 * r) >> 2] >> (8 * ((1 + 2 * r) & 3))) & 0xFFu;
-            const uint32_t ln = ((hw[(2 + 2 * r) >> 2] >> (8 * ((2 + 2 * r) & 3))) & 0xFFu) + 1u;
-#pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
-              const uint32_t sym = 4 * lane + j;
-              if (sym >= st && sym < st + ln) {
-                live4 |= 1u << j;
-                rk[j] = acc + sym - st;
-              }
+          for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t d = 4 * lane + j - st;
+            if (d < ln) {
+              live4 |= 1u << j;
+              rk[j] = acc + d;
             }
-            acc += ln;
           }
+          acc += ln;
         }
         kk = acc;
       }
@@ -2688,36 +2693,46 @@ __device__ __forceinline__ void nz_decode_chunk(
       }
     }
     __syncthreads();
-    // slot table: consecutive threads fill consecutive slots.  The run of a
-    // slot is the number of runs that start at or before it, minus one.  (Of a
-    // table whose frequencies do not sum to 4096 nothing was written: the fill
-    // then reads zeros and the chunk is given up right after.)  The last slots
-    // lie under the parse results: their entries wait in registers until every
-    // thread has read what it needs.
+    // Slot table: a thread fills eight consecutive slots, in pairs of 16 bytes.  The run of a slot is the
+    // number of runs that start at or before it, minus one; the eight lie in one window, and rarely
+    // does a pair hold the start of a run in its second slot.  (Of a table whose frequencies
+    // do not sum to 4096 nothing was written: the fill then reads zeros and the chunk is given up
+    // right after.)  The last slots lie under the parse results: the threads' last entries wait
+    // in registers until all have read what they need.  Neighbouring lanes' pairs are in turn: eight lanes
+    // write to different banks.  (One slot at a time, two LDS reads and a write of 8 bytes for each, the
+    // fill took 2900 cycles, of some 50000 that a chunk of 256 symbols per lane takes.  With this, and the
+    // run descriptors in scalar registers above: read of 1024 x 1024 22.2 -> 21.5 us, gather of a row 21.8 -> 21.2,
+    // one and eight rows through the Linears of a block of width 4096 160.6 -> 158.4, 237.4 -> 234.0.)
     {
-      const uint32_t below = (2u << (tid & 31)) - 1u;  // bits of a window up to this thread's slot
-      const auto entry_of = [&](uint32_t slot) {
-        const uint2 wn = wins[slot >> 5];
-        const uint32_t k = wn.y + (uint32_t)__popc(wn.x & below) - 1u;
-        const uint2 rn = runs[k & 255u];
-        return make_uint2(rn.x, slot - rn.y);
-      };
-      for (uint32_t slot = tid; slot < NZ_TMETA_SLOT; slot += blockDim.x) lut[slot] = entry_of(slot);
-      // (NZ_TMETA_SLOT is a multiple of 32, so `below` fits these slots as well)
-      constexpr uint32_t LAST = (NZ_M - NZ_TMETA_SLOT + 63) / 64;  // per thread, for the smallest workgroup
-      uint2 last[LAST];
+      const auto slot_at = [&](uint32_t at, uint32_t i) { return at + 2u * ((i + (lane >> 2)) & 3u); };
+      const auto entries = [&](uint32_t at, uint4 (&en)[4]) {
+        const uint2 wn = wins[at >> 5];
 #pragma unroll
-      for (uint32_t i = 0; i < LAST; ++i) {
-        const uint32_t slot = NZ_TMETA_SLOT + tid + i * blockDim.x;
-        last[i] = slot < NZ_M ? entry_of(slot) : make_uint2(0u, 0u);
+        for (uint32_t i = 0; i < 4; ++i) {
+          const uint32_t slot = slot_at(at, i), bit = slot & 31;
+          const uint32_t k = wn.y + (uint32_t)__popc(wn.x & ((2u << bit) - 1u)) - 1u;
+          const uint2 a = runs[k & 255u];
+          uint2 b = a;
+          if ((wn.x >> (bit + 1)) & 1u) b = runs[(k + 1u) & 255u];
+          en[i] = make_uint4(a.x, slot - a.y, b.x, slot + 1u - b.y);
+        }
+      };
+      const auto put = [&](uint32_t at, const uint4 (&en)[4]) {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(lut + slot_at(at, i)) = en[i];
+      };
+      uint4 en[4];
+      // (whole rounds end at slot 3584 at the latest, with 64, 128, ... 512 threads)
+      static_assert(NZ_M - 8 * NZ_LANES <= NZ_TMETA_SLOT, "");
+      uint32_t at = 8 * tid;
+      for (uint32_t done = 8 * blockDim.x; done < NZ_M; done += 8 * blockDim.x, at += 8 * blockDim.x) {
+        entries(at, en);
+        put(at, en);
       }
+      if (at < NZ_M) entries(at, en);
       const uint32_t table_ok = tflag[0], table_len = tflag[1];
       __syncthreads();
-#pragma unroll
-      for (uint32_t i = 0; i < LAST; ++i) {
-        const uint32_t slot = NZ_TMETA_SLOT + tid + i * blockDim.x;
-        if (slot < NZ_M) lut[slot] = last[i];
-      }
+      if (at < NZ_M) put(at, en);
       if (!table_ok) {
         if (tid == 0) atomicOr(d_status, 2u);
         return;
