@@ -2488,6 +2488,8 @@ __device__ __forceinline__ void nz_decode_chunk(
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
     const NzGemv& gv, const NzNorm& nm, const uint32_t first_seg, const uint32_t end_seg,
     const NzRowOut& row = NzRowOut{}) {
+  constexpr bool ONE_READ = ONE || GEMV || ROWS;
+  constexpr bool PAIRS = GEMV || ROWS || (ONE && !NORM && S >= 3);  // how the slot table is filled
   // At LDS address 0: a kernel that decodes has no static LDS (pinned in tests/test_kernel_resources.py),
   // because NzWaveDecOne numbers table and rings through from there.
   extern __shared__ uint32_t lds[];
@@ -2570,7 +2572,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   const uint32_t lane_off = lane * (S + 1);
   const uint32_t last_off = whole ? (whole - 1) * NZ_LANES * (S + 1) + lane_off : 0u;
   constexpr uint32_t RING = ONE ? NZ_RING_WIDE : NZ_RING_NARROW;
-  std::conditional_t<ONE || GEMV || ROWS, NzWaveDecOne<RING>, NzWaveDec> w;
+  std::conditional_t<ONE_READ, NzWaveDecOne<RING>, NzWaveDec> w;
   w.lut = lut;
   w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + ring * 2 * RING);
   w.nwords = rec_all / 2;
@@ -2600,7 +2602,8 @@ __device__ __forceinline__ void nz_decode_chunk(
   // the first 32 table bytes hold the mode and all run descriptors there can be
   const uint4 h0 = reinterpret_cast<const uint4*>(tb)[0], h1 = reinterpret_cast<const uint4*>(tb)[1];
   const uint32_t bm_byte = tb[1 + (lane >> 1)];  // bitmap mode: the byte with this lane's four symbols
-  const uint32_t mode = (uint32_t)__builtin_amdgcn_readfirstlane(h0.x) & 0xFFu;
+  uint32_t mode = h0.x & 0xFFu;
+  if constexpr (PAIRS) mode = (uint32_t)__builtin_amdgcn_readfirstlane(mode);
   uint32_t tab_len = 4;
 
   if (mode != NZ_MODE_RAW) {
@@ -2627,28 +2630,48 @@ __device__ __forceinline__ void nz_decode_chunk(
         for (uint32_t j = 0; j < 4; ++j) rk[j] = ci - c + (uint32_t)__popc(live4 & ((1u << j) - 1u));
       } else {
         head = 1 + 2 * mode;
-        // the run descriptors, 16 bits each from the second byte on, move down through scalar registers
-        const auto pair = [](uint32_t lo, uint32_t hi) {
-          return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(lo) | ((uint64_t)__builtin_amdgcn_readfirstlane(hi) << 32);
-        };
-        uint64_t q0 = pair(h0.x, h0.y), q1 = pair(h0.z, h0.w), q2 = pair(h1.x, h1.y), q3 = pair(h1.z, h1.w);
         uint32_t acc = 0;
+        if constexpr (PAIRS) {
+          // the run descriptors, 16 bits each from the second byte on, move down through scalar registers
+          const auto pair = [](uint32_t lo, uint32_t hi) {
+            return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(lo) | ((uint64_t)__builtin_amdgcn_readfirstlane(hi) << 32);
+          };
+          uint64_t q0 = pair(h0.x, h0.y), q1 = pair(h0.z, h0.w), q2 = pair(h1.x, h1.y), q3 = pair(h1.z, h1.w);
 #pragma nounroll
-        for (uint32_t r = 0; r < mode; ++r) {
-          const uint32_t st = (uint32_t)(q0 >> 8) & 0xFFu, ln = ((uint32_t)(q0 >> 16) & 0xFFu) + 1u;
-          q0 = q0 >> 16 | q1 << 48;
-          q1 = q1 >> 16 | q2 << 48;
-          q2 = q2 >> 16 | q3 << 48;
-          q3 >>= 16;
+          for (uint32_t r = 0; r < mode; ++r) {
+            const uint32_t st = (uint32_t)(q0 >> 8) & 0xFFu, ln = ((uint32_t)(q0 >> 16) & 0xFFu) + 1u;
+            q0 = q0 >> 16 | q1 << 48;
+            q1 = q1 >> 16 | q2 << 48;
+            q2 = q2 >> 16 | q3 << 48;
+            q3 >>= 16;
 #pragma unroll
-          for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t d = 4 * lane + j - st;
-            if (d < ln) {
-              live4 |= 1u << j;
-              rk[j] = acc + d;
+            for (uint32_t j = 0; j < 4; ++j) {
+              const uint32_t d = 4 * lane + j - st;
+              if (d < ln) {
+                live4 |= 1u << j;
+                rk[j] = acc + d;
+              }
+            }
+            acc += ln;
+          }
+        } else {
+          const uint32_t hw[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+#pragma unroll
+          for (uint32_t r = 0; r < NZ_MAX_RUNS; ++r) {
+            if (r < mode) {
+              const uint32_t st = (hw[(1 + 2 * r) >> 2] >> (8 * ((1 + 2 * r) & 3))) & 0xFFu;
+              const uint32_t ln = ((hw[(2 + 2 * r) >> 2] >> (8 * ((2 + 2 * r) & 3))) & 0xFFu) + 1u;
+#pragma unroll
+              for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t sym = 4 * lane + j;
+                if (sym >= st && sym < st + ln) {
+                  live4 |= 1u << j;
+                  rk[j] = acc + sym - st;
+                }
+              }
+              acc += ln;
             }
           }
-          acc += ln;
         }
         kk = acc;
       }
@@ -2703,36 +2726,68 @@ __device__ __forceinline__ void nz_decode_chunk(
     // fill took 2900 cycles, of some 50000 that a chunk of 256 symbols per lane takes.  With this, and the
     // run descriptors in scalar registers above: read of 1024 x 1024 22.2 -> 21.5 us, gather of a row 21.8 -> 21.2,
     // one and eight rows through the Linears of a block of width 4096 160.6 -> 158.4, 237.4 -> 234.0.)
+    // Elsewhere consecutive threads fill consecutive slots one by one, and every thread keeps its part of the last:
+    // the compiler's code for the steps behind the fill in pairs was slower there.  With pairs and without, two-read
+    // step: 512 chunks, precision 1: 52.4 and 48.8 us; 1023 chunks, precision 0, normalizers of 8: 111.9 and 102.3;
+    // precision 7: 43.4 and 42.6.  One-read step, 256 chunks: precision 1: 35.0 and 33.2, precision 3
+    // with normalizers of 64: 37.1 and 35.3.
     {
-      const auto slot_at = [&](uint32_t at, uint32_t i) { return at + 2u * ((i + (lane >> 2)) & 3u); };
-      const auto entries = [&](uint32_t at, uint4 (&en)[4]) {
-        const uint2 wn = wins[at >> 5];
+      uint32_t table_ok, table_len;
+      if constexpr (PAIRS) {
+        const auto slot_at = [&](uint32_t at, uint32_t i) { return at + 2u * ((i + (lane >> 2)) & 3u); };
+        const auto entries = [&](uint32_t at, uint4 (&en)[4]) {
+          const uint2 wn = wins[at >> 5];
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-          const uint32_t slot = slot_at(at, i), bit = slot & 31;
-          const uint32_t k = wn.y + (uint32_t)__popc(wn.x & ((2u << bit) - 1u)) - 1u;
-          const uint2 a = runs[k & 255u];
-          uint2 b = a;
-          if ((wn.x >> (bit + 1)) & 1u) b = runs[(k + 1u) & 255u];
-          en[i] = make_uint4(a.x, slot - a.y, b.x, slot + 1u - b.y);
+          for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t slot = slot_at(at, i), bit = slot & 31;
+            const uint32_t k = wn.y + (uint32_t)__popc(wn.x & ((2u << bit) - 1u)) - 1u;
+            const uint2 a = runs[k & 255u];
+            uint2 b = a;
+            if ((wn.x >> (bit + 1)) & 1u) b = runs[(k + 1u) & 255u];
+            en[i] = make_uint4(a.x, slot - a.y, b.x, slot + 1u - b.y);
+          }
+        };
+        const auto put = [&](uint32_t at, const uint4 (&en)[4]) {
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(lut + slot_at(at, i)) = en[i];
+        };
+        uint4 en[4];
+        // (whole rounds end at slot 3584 at the latest, with 64, 128, ... 512 threads)
+        static_assert(NZ_M - 8 * NZ_LANES <= NZ_TMETA_SLOT, "");
+        uint32_t at = 8 * tid;
+        for (uint32_t done = 8 * blockDim.x; done < NZ_M; done += 8 * blockDim.x, at += 8 * blockDim.x) {
+          entries(at, en);
+          put(at, en);
         }
-      };
-      const auto put = [&](uint32_t at, const uint4 (&en)[4]) {
+        if (at < NZ_M) entries(at, en);
+        table_ok = tflag[0], table_len = tflag[1];
+        __syncthreads();
+        if (at < NZ_M) put(at, en);
+      } else {
+        const uint32_t below = (2u << (tid & 31)) - 1u;  // bits of a window up to this thread's slot
+        const auto entry_of = [&](uint32_t slot) {
+          const uint2 wn = wins[slot >> 5];
+          const uint32_t k = wn.y + (uint32_t)__popc(wn.x & below) - 1u;
+          const uint2 rn = runs[k & 255u];
+          return make_uint2(rn.x, slot - rn.y);
+        };
+        for (uint32_t slot = tid; slot < NZ_TMETA_SLOT; slot += blockDim.x) lut[slot] = entry_of(slot);
+        // (NZ_TMETA_SLOT is a multiple of 32, so `below` fits these slots as well)
+        constexpr uint32_t LAST = (NZ_M - NZ_TMETA_SLOT + 63) / 64;  // per thread, for the smallest workgroup
+        uint2 last[LAST];
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(lut + slot_at(at, i)) = en[i];
-      };
-      uint4 en[4];
-      // (whole rounds end at slot 3584 at the latest, with 64, 128, ... 512 threads)
-      static_assert(NZ_M - 8 * NZ_LANES <= NZ_TMETA_SLOT, "");
-      uint32_t at = 8 * tid;
-      for (uint32_t done = 8 * blockDim.x; done < NZ_M; done += 8 * blockDim.x, at += 8 * blockDim.x) {
-        entries(at, en);
-        put(at, en);
+        for (uint32_t i = 0; i < LAST; ++i) {
+          const uint32_t slot = NZ_TMETA_SLOT + tid + i * blockDim.x;
+          last[i] = slot < NZ_M ? entry_of(slot) : make_uint2(0u, 0u);
+        }
+        table_ok = tflag[0], table_len = tflag[1];
+        __syncthreads();
+#pragma unroll
+        for (uint32_t i = 0; i < LAST; ++i) {
+          const uint32_t slot = NZ_TMETA_SLOT + tid + i * blockDim.x;
+          if (slot < NZ_M) lut[slot] = last[i];
+        }
       }
-      if (at < NZ_M) entries(at, en);
-      const uint32_t table_ok = tflag[0], table_len = tflag[1];
-      __syncthreads();
-      if (at < NZ_M) put(at, en);
       if (!table_ok) {
         if (tid == 0) atomicOr(d_status, 2u);
         return;
@@ -2851,7 +2906,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide, auto fetch_ahead,
                               auto xl) __attribute__((always_inline)) {
     constexpr bool X_LDS = !std::is_same_v<decltype(xl), NzNoLds>;
-    if constexpr (ONE || GEMV || ROWS) w.look();  // before the group's loads: a refill waits for all that are under way
+    if constexpr (ONE_READ) w.look();  // before the group's loads: a refill waits for all that are under way
     NzXq<MR> xq;
     if constexpr (GEMV && X_AHEAD) {
       xq = xq_next;
@@ -2860,7 +2915,7 @@ __device__ __forceinline__ void nz_decode_chunk(
       xq = walk.load(walk.col);
     }
     fetch_ahead();  // behind the activations: their wait is then not for bytes from memory as well (eight rows: 265 -> 260 us)
-    if constexpr (!ONE && !GEMV && !ROWS) w.look();  // (behind them here: 143 us for 8192 x 28672, before them 145)
+    if constexpr (!ONE_READ) w.look();  // (behind them here: 143 us for 8192 x 28672, before them 145)
     uint32_t ew[8];
     w.group(ew);
     // the merge starts only here: its wait for the packed bytes must not be
