@@ -2488,8 +2488,12 @@ __device__ __forceinline__ void nz_decode_chunk(
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
     const NzGemv& gv, const NzNorm& nm, const uint32_t first_seg, const uint32_t end_seg,
     const NzRowOut& row = NzRowOut{}) {
-  constexpr bool ONE_READ = ONE || GEMV || ROWS;
-  constexpr bool PAIRS = GEMV || ROWS || (ONE && !NORM && S >= 3);  // how the slot table is filled
+  // One read per step with the narrow ring for normalizers as well (precision 3 and 7; 264 to 512 chunks): precision 3, groups of
+  // 64: 320 chunks 45.8 -> 42.8 us, 512 48.1 -> 46.8, groups of 2: 59.9 -> 56.1, 66.9 -> 62.3, precision 7: 44.7 -> 41.5,
+  // 46.5 -> 44.4.  With the wide ring 320 chunks take 46.5; precision 0, groups of 8, loses (512: 51.5 -> 54.5).
+  constexpr bool NORM_ONE = NORM && !STREAM && !ONE && S >= 3;
+  constexpr bool ONE_READ = ONE || GEMV || ROWS || NORM_ONE;
+  constexpr bool PAIRS = GEMV || ROWS || NORM_ONE || (ONE && !NORM && S >= 3);  // how the slot table is filled
   // At LDS address 0: a kernel that decodes has no static LDS (pinned in tests/test_kernel_resources.py),
   // because NzWaveDecOne numbers table and rings through from there.
   extern __shared__ uint32_t lds[];
