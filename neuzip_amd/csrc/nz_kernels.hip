@@ -2733,8 +2733,8 @@ __device__ __forceinline__ void nz_decode_chunk(
     // Elsewhere consecutive threads fill consecutive slots one by one, and every thread keeps its part of the last:
     // the compiler's code for the steps behind the fill in pairs was slower there.  With pairs and without, two-read
     // step: 512 chunks, precision 1: 52.4 and 48.8 us; 1023 chunks, precision 0, normalizers of 8: 111.9 and 102.3;
-    // precision 7: 43.4 and 42.6.  One-read step, 256 chunks: precision 1: 35.0 and 33.2, precision 3
-    // with normalizers of 64: 37.1 and 35.3.
+    // precision 7: 43.4 and 42.6.  One-read step, 128 chunks: precision 0: 28.5 and 26.7,
+    // precision 7 with normalizers of 64: 30.5 and 29.3.
     {
       uint32_t table_ok, table_len;
       if constexpr (PAIRS) {
