@@ -86,7 +86,7 @@ EncLayout enc_layout(const NzGeom& g) {
   L.chunk_units = take((g.n_chunks + 1) * 4);
   L.pub = take(g.n_chunks * 32);  // size and running-total announcements of the chunks (records placed by the encode kernel)
   L.placed = take(g.n_segs);      // per segment: its record is in the container only
-  L.lb_state = take(12);          // run count and abort mark of the announcements, mark of a record left out
+  L.lb_state = take(sizeof(NzLbWords));
   L.bytes = o;
   return L;
 }
@@ -1128,7 +1128,8 @@ void late_item(const nz_manager* m, const char* name, const Entry& ent, NzBatchI
   const RewriteSlot& s = m->rw[ent.pending];
   for (uint32_t j = 0; j < s.count; ++j)
     if (s.names[j] == name) {
-      bi->late = reinterpret_cast<const uint32_t*>(s.b.item[j].ws + s.b.item[j].lb_state);
+      bi->late = reinterpret_cast<const NzLbWords*>(s.b.item[j].ws + s.b.item[j].lb_state);
+      bi->late_nonce = s.b.item[j].nonce;
       bi->late_comp = (const uint8_t*)s.late + s.late_at[j];
       bi->late_bytes = s.late_at[j + 1] - s.late_at[j];
     }

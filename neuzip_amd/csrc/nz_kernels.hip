@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "nz_format.h"
+#include "nz_lookback.h"
 
 #define NZ_RING_WORDS 1024u  // per-wave LDS ring of renormalisation words (NzWaveDec) ...
 #define NZ_RING_DWORDS (NZ_RING_WORDS / 2)
@@ -891,7 +892,6 @@ __device__ __forceinline__ void nz_enc_finish(const uint32_t x, const uint32_t w
 // concatenation of their chunks, that of the scan kernel one workgroup per
 // tensor, that of the compaction the concatenation of their segments.
 #define NZ_ENC_BATCH_MAX 16
-#define NZ_LOOKBACK_ABORT 0xAB0F7EDDu
 struct NzEncItem {
   const uint16_t* in;   // dense input
   uint8_t* packed;      // stored sign|mantissa stream
@@ -911,17 +911,7 @@ struct NzEncItem {
   uint64_t pub, nonce;
   uint64_t* d_gave_up;
   uint32_t direct, spin_limit;
-  // three words in ws (offset): [0] counts the direct encodes that have used this
-  // scratch, advanced by the workgroup of the last chunk - the announcements'
-  // mark is made of it and the nonce, so those of an earlier run of the very
-  // same call (a replayed graph) do not pass for this run's; [1] holds
-  // NZ_LOOKBACK_ABORT after a run in which a workgroup gave up: the next run
-  // then leaves the placing to nz_compact_kernel as well (and says so through
-  // the same flags) and takes the mark away; [2] is set to what [0] becomes by a
-  // run that leaves a record out of the container, whatever the reason (a reader behind
-  // it on the stream goes by that: nz_late_kernel).  Whatever the memory held
-  // before its first use is as good a start as any.
-  uint64_t lb_state;
+  uint64_t lb_state;  // NzLbWords (offset into ws)
   // `placed`: one byte per segment (offset into ws), left by a direct encode: 1 =
   // the record is in the container and not in the scratch (its words went there
   // from LDS).  nz_compact_kernel with `use_placed` takes such records from
@@ -1129,10 +1119,10 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
   // once, by one thread, long before it is needed, and handed to the others
   // through LDS, so that every thread of the workgroup acts on the same values
   // (another workgroup may change the words while this one starts).
-  uint32_t* lb_state = reinterpret_cast<uint32_t*>(it.ws + it.lb_state);
+  NzLbWords* lb_state = reinterpret_cast<NzLbWords*>(it.ws + it.lb_state);
   if (tid == 0) {
-    L.lb[0] = it.direct ? __hip_atomic_load(lb_state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-    L.lb[1] = it.direct ? __hip_atomic_load(lb_state + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    L.lb[0] = it.direct ? __hip_atomic_load(&lb_state->runs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    L.lb[1] = it.direct ? __hip_atomic_load(&lb_state->abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
     L.redo = 0;
   }
   NzHist::clear(nz_enc_stage, b.copies_log2);
@@ -1333,20 +1323,13 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
   const uint32_t lb_gen = L.lb[0];  // (only now: kept since the beginning, it was spilled for the coding phase)
   uint8_t* placed = it.ws + it.placed;  // per segment: its record is in the container and nowhere else
   const bool last_chunk = c + 1 == g.n_chunks;
-  const auto left_out = [&] {
-    __hip_atomic_store(lb_state + 2, lb_gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
   if (!places()) {
     // the run before this one ended with a workgroup giving up: nothing is
     // placed, the caller is told, and the mark is taken away for the next run
     if (tid == 0) {
       atomicOr(it.d_status, 4u);
       if (it.d_gave_up) *it.d_gave_up = it.nonce;
-      left_out();
-      if (last_chunk) {
-        __hip_atomic_store(lb_state, lb_gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(lb_state + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+      nz_lb_unplaced(lb_state, it.nonce, lb_gen, last_chunk);
     }
     if (has_seg && lane == 0) placed[seg] = 0;
     return;
@@ -1453,15 +1436,11 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
     const uint16_t* sw = reinterpret_cast<const uint16_t*>(stage);
     for (uint32_t p = pos_end + lane; p < cap_words; p += NZ_LANES) slot[p] = sw[p - stage_lo];
   };
-  // the workgroup of the last chunk has seen every other announce (or has given
-  // up): all of them have read the count, which can now move on
   if (L.gave_up) {
     if (tid == 0) {
-      __hip_atomic_store(lb_state + 1, NZ_LOOKBACK_ABORT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       atomicOr(it.d_status, 4u);
       if (it.d_gave_up) *it.d_gave_up = it.nonce;
-      left_out();
-      if (last_chunk) __hip_atomic_store(lb_state, lb_gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      nz_lb_gave_up(lb_state, it.nonce, lb_gen, last_chunk);
     }
     if (has_seg) {
       if (staged && !L.raw) unstage();
@@ -1469,9 +1448,8 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
     }
     return;
   }
-  if (last_chunk && tid == 0)
-    __hip_atomic_store(lb_state, lb_gen + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (tid == 0) {
+    nz_lb_placed(lb_state, lb_gen, last_chunk);
     // the running total up to and including this chunk, for the chunks that come later (32 bits
     // of 4-byte units: a container beyond 16 GiB announces none, and its chunks walk on)
     uint64_t upto = L.chunk_total;
@@ -1499,7 +1477,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK, nz_enc_waves(NG)) void 
     if (from_stage && !fits) unstage();
     if (lane == 0) {
       placed[seg] = (from_stage && fits) ? 1 : 0;
-      if (!fits) left_out();
+      if (!fits) nz_lb_left_out(lb_state, it.nonce);
     }
   }
   NZ_PROBE_MARK(5);
@@ -1712,15 +1690,15 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 // Between an in-place write and a read that the host enqueues before it knows how the write went:
 // the tensors of which the write has left a record out of the container (it outgrew its buffer, or
 // a chunk gave up waiting) are put together again in a buffer that holds any container, and the read
-// goes by the same two words (NzBatchItem::late).  There is next to never anything to do, so the grid
-// is small, and the words of all tensors are looked at together: 1.5 to 3 us (64 workgroups that look at one
+// goes by the same mark (NzBatchItem::late).  There is next to never anything to do, so the grid
+// is small, and the marks of all tensors are looked at together: 1.5 to 3 us (64 workgroups that look at one
 // tensor after the other: 4.3).
 __global__ __launch_bounds__(256) void nz_late_kernel(const NzEncBatch b) {
   __shared__ uint64_t red4[4];
-  const uint32_t lane = threadIdx.x & 63, mine = lane < b.count ? lane : 0;  // all tensors' words at once
-  const uint2* state = reinterpret_cast<const uint2*>(b.item[mine].ws + b.item[mine].lb_state);
-  const uint32_t run = state[0].x, left_out = state[1].x;
-  for (uint64_t todo = __ballot(lane < b.count && run == left_out); todo; todo &= todo - 1) {
+  const uint32_t lane = threadIdx.x & 63, mine = lane < b.count ? lane : 0;  // all tensors' marks at once
+  const NzLbWords* words = reinterpret_cast<const NzLbWords*>(b.item[mine].ws + b.item[mine].lb_state);
+  const bool not_whole = nz_lb_not_whole(words, b.item[mine].nonce);
+  for (uint64_t todo = __ballot(lane < b.count && not_whole); todo; todo &= todo - 1) {
     const NzEncItem& it = b.item[__builtin_ctzll(todo)];
     for (uint64_t seg = blockIdx.x; seg < it.g.n_segs; seg += gridDim.x) nz_compact_segment(it, seg, red4);
   }
@@ -3074,9 +3052,10 @@ struct NzBatchItem {
   NzGeom g;
   uint32_t chunk_end;
   uint32_t reserved;
-  // dense output of a tensor whose last write is not known to have fitted its buffer: the run count and
-  // mark of that write's scratch (NzEncItem::lb_state; null: all is known), and the container to take if they agree
-  const uint32_t* late;
+  // dense output of a tensor whose last write is not known to have fitted its buffer: the words in that
+  // write's scratch (null: all is known), its nonce, and the container to take if they say it is not whole
+  const NzLbWords* late;
+  uint64_t late_nonce;
   const uint8_t* late_comp;
   uint64_t late_bytes;
 };
@@ -3101,7 +3080,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_ke
   }
   const NzBatchItem& it = b.item[t];
   const NzPart p(blockIdx.x, b.parts, it.g.spc);
-  const bool other = it.late && it.late[2] == it.late[0];
+  const bool other = it.late && nz_lb_not_whole(it.late, it.late_nonce);
   nz_decode_chunk<S, 0, NORM, STREAM, ONE>(other ? it.late_comp : it.comp, other ? it.late_bytes : it.comp_bytes,
                                           it.packed, it.out, it.g, d_status, at - first, NzGemv{},
                                           NzNorm{it.norm, b.log2n}, p.first, p.end);
