@@ -333,7 +333,10 @@ int nz_manager_gemv_rows_batch(nz_manager* m, const char* const* names, uint32_t
                                const void* const* dev_bias, void* const* dev_y, void* stream);
 
 /* The same for rows of any multiple of 8 elements from 512 up: a Linear whose
-   in_features the calls above refuse. */
+   in_features the calls above refuse.  Of rows that are not whole groups of 512,
+   those that several wavefronts share are sums of the wavefronts' fp32 sums in
+   the order of the elements, whatever order they arrive in: they have fp32's
+   range and infinities.  (In multiples of 512 a row is summed as above.) */
 int nz_manager_linear_rows_batch(nz_manager* m, const char* const* names, uint32_t count,
                                  const void* dev_x, uint32_t x_rows, uint32_t in_features,
                                  const void* const* dev_bias, void* const* dev_y, void* stream);

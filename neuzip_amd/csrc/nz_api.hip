@@ -1424,6 +1424,13 @@ int nz_manager_read_batch(nz_manager* m, const char* const* names, void* const* 
   return read_batch(m, names, dev_outs, cap_elems, count, (hipStream_t)stream);
 }
 
+// Accumulator of a row, in words of 32 bits: a pair of 64, or what rows that are not whole groups need.
+static uint32_t acc_words(const Entry& ent, uint32_t in_features) {
+  if (in_features % NZ_GROUP_SYMS == 0 || ent.chunk_syms == 0) return 4;
+  const uint32_t seg = ent.lane_syms * NZ_LANES, last = (ent.chunk_syms - 1) % seg + 1;  // a chunk's last segment may be shorter
+  return nz_row_acc_words(in_features, last < seg ? last : seg);
+}
+
 // The fused product for rows of W that are multiples of `unit` elements (512: a group lies in one row).
 static int gemv_rows(nz_manager* m, const char* const* names, uint32_t count, const void* dev_x, uint32_t x_rows,
                      uint32_t in_features, uint32_t unit, const void* const* dev_bias, void* const* dev_y,
@@ -1454,8 +1461,9 @@ static int gemv_rows(nz_manager* m, const char* const* names, uint32_t count, co
       if (!names[i]) return fail(NZ_ERR_ARG, "null name");
       auto it = m->entries.find(names[i]);
       if (it == m->entries.end()) return fail(NZ_ERR_NOT_FOUND, "Data not found");
-      blocks = blocks || it->second.pending >= 0;
-      want_rows += it->second.n / in_features * x_rows;  // an accumulator pair per row and activation row
+      const Entry& ent = it->second;
+      blocks = blocks || ent.pending >= 0;
+      want_rows += ent.n / in_features * x_rows * (acc_words(ent, in_features) / 4);
     }
     if (int rc = refuse_under_capture(st, blocks || m->gemv_rows < want_rows, "gemv_batch")) return rc;
     if (int rc = order_scratch_use(m, st, &captured)) return rc;
@@ -1481,8 +1489,8 @@ static int gemv_rows(nz_manager* m, const char* const* names, uint32_t count, co
     if (g.spc > max_spc) max_spc = g.spc;
     bi.bias = dev_bias ? (const uint16_t*)dev_bias[i] : nullptr;
     bi.y = (uint16_t*)dev_y[i];
-    bi.reserved = (uint32_t)rows;  // first accumulator pair, turned into a pointer below
-    rows += ent.n / in_features * x_rows;
+    bi.acc_words = (uint32_t)rows;  // first accumulator pair, turned into a pointer below
+    rows += ent.n / in_features * x_rows * (acc_words(ent, in_features) / 4);
     if (grid > 0x7FFFFFFFull || rows > 0x7FFFFFFFull) return fail(NZ_ERR_ARG, "batch too large");
   }
   // Room for the next power of two of activation rows, so that a launch that has been made with
@@ -1510,8 +1518,8 @@ static int gemv_rows(nz_manager* m, const char* const* names, uint32_t count, co
   }
   if (captured) m->gemv_captured = true;
   for (uint32_t i = 0; i < count; ++i) {
-    b.item[i].acc = m->gemv_acc + 2 * (uint64_t)b.item[i].reserved;
-    b.item[i].reserved = 0;
+    b.item[i].acc = m->gemv_acc + 2 * (uint64_t)b.item[i].acc_words;
+    b.item[i].acc_words = acc_words(m->entries.find(names[i])->second, in_features);
   }
   b.count = count;
   return gemv_launch(b, (uint32_t)grid, max_spc, m->precision, m->d_status, st);

@@ -1891,8 +1891,8 @@ __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew
 // least 512, so a lane's weights lie in one row of W and a group in at most two (in one, always,
 // where the row length is a multiple of 512).  A
 // lane keeps an fp32 partial sum of its 8-element dot products; what happens
-// when the wave leaves a row is described at NzGemvWalk.  Row r owns acc[2r]
-// (fixed-point sum) and acc[2r + 1] (contribution count in the low half, flag
+// when the wave leaves a row is described at NzGemvWalk.  Where rows are whole groups, row r owns
+// acc[2r] (fixed-point sum) and acc[2r + 1] (contribution count in the low half, flag
 // in bit 32).
 // 40 fraction bits: an absolute resolution of 9e-13 per partial sum; up to 16
 // partial sums below 2^18 in magnitude cannot overflow 64 bits.
@@ -1901,11 +1901,19 @@ __device__ __forceinline__ uint4 nz_merge_group(uint64_t sm, const uint32_t (&ew
 
 struct NzGemv {
   const uint16_t* x;      // as many activation rows as the kernel is for, in_features bf16 values each, 16-byte aligned
-  long long* acc;         // two words per row of this tensor and activation row (sum | count and flag), all zero between calls
+  long long* acc;         // accumulators of this tensor, all zero between calls: rows that are whole groups, two words per row
+                          // and activation row (sum | count and flag); else acc_words words of 32 bits (count, a partial
+                          // sum of each segment that a row can touch)
   uint16_t* y;            // for each activation row one bf16 per row of the tensor
   const uint16_t* bias;   // one bf16 per row of the tensor, or null
   uint32_t in_features;   // multiple of 8, at least 512
+  uint32_t acc_words;
 };
+// 32-bit words of a row's accumulator where rows are not whole groups, in fours: a row of L elements that
+// touches k segments holds k - 2 of them, of the shortest `min_seg` elements, and an element of two more
+NZ_HD static inline uint32_t nz_row_acc_words(uint32_t in_features, uint32_t min_seg) {
+  return (1u + (in_features - 2u) / min_seg + 2u + 3u) & ~3u;
+}
 
 struct NzNoLds {};  // the activations of a group are not in LDS
 
@@ -1934,12 +1942,16 @@ __device__ __forceinline__ float nz_dot8(const uint4 w, const uint4 x, float acc
 //
 // When the wave leaves a row it adds its 64 partial sums in a fixed order.  A row that lies inside the wave's segment is complete then: bias
 // added, rounded, stored.  A row shared with other segments goes through the
-// row's accumulator pair: the sum in 24.40 fixed point (integer addition is
+// row's accumulator: the partial sums of its segments, and a counter of contributions; the wave that brings
+// the count to the number of segments the row touches finishes the row and returns the words to zero.
+// Where rows are whole groups, the partial sums are added in 24.40 fixed point (integer addition is
 // associative, so the result does not depend on which wave arrives first; a
 // partial sum that is NaN, infinite or beyond 2^18 sets a flag instead and the
-// row comes out as NaN), and a counter of contributions; the wave that brings
-// the count to the number of segments the row touches converts, stores and
-// returns both words to zero.
+// row comes out as NaN).  Where they are not, each segment leaves its fp32 sum in a word of its own and
+// the last wave adds them in the order of the segments: such Linears are products of the GEMM library
+// where this kernel does not serve them, so the sums keep fp32's range, infinities and small values.
+// (Fixed point brought zero for sums below 2^-41 and NaN for infinite ones.  A block of width 4224, one and
+// eight rows: 164.0 and 269.7 us in fixed point, 163.8 and 271.6 with words.)
 template <int MR, bool WHOLE>
 struct NzGemvWalk {
   NzGemv gv;
@@ -1994,10 +2006,10 @@ struct NzGemvWalk {
     }
     return r;
   }
-  // Segments the row [first, last] touches, this wave's included: walk over the
-  // segment boundaries to the left and to the right (a row rarely spans more
+  // Segments the row [first, last] touches, this wave's included, and how many of them come before it: walk
+  // over the segment boundaries to the left and to the right (a row rarely spans more
   // than two or three segments; no division).
-  __device__ __forceinline__ uint32_t segments_of_row(uint64_t first, uint64_t last) const {
+  __device__ __forceinline__ uint32_t segments_of_row(uint64_t first, uint64_t last, uint32_t* before) const {
     uint32_t count = 1;
     uint64_t at = seg_first;
     uint32_t kk = k;
@@ -2006,6 +2018,7 @@ struct NzGemvWalk {
       at -= kk == spc - 1 ? last_syms : seg_syms;
       ++count;
     }
+    *before = count - 1;
     at = seg_end;
     kk = k;
     while (at <= last) {  // so does the segment that starts at `at`
@@ -2034,22 +2047,35 @@ struct NzGemvWalk {
         // this lane when each one waits for the value the previous returned, so
         // no cache flush is needed: the count is issued only after the sum's old
         // value has come back, the exchanges only after the count's.
-        const uint32_t expected = segments_of_row(first, last);
-        unsigned long long* slot = reinterpret_cast<unsigned long long*>(gv.acc + 2 * (row * MR + m));
-        unsigned long long r0;
-        if (fabsf(t) < NZ_GEMV_PART_MAX)  // false for NaN as well
-          r0 = atomicAdd(slot, (unsigned long long)__float2ll_rn(t * (float)(1ull << NZ_GEMV_FRAC_BITS)));
-        else
-          r0 = atomicOr(slot + 1, 1ull << 32);
+        uint32_t place;
+        const uint32_t expected = segments_of_row(first, last, &place);
         uint32_t zero;  // 0, but only the hardware knows: ties the next atomic to the returned value
-        asm volatile("v_and_b32 %0, 0, %1" : "=v"(zero) : "v"((uint32_t)r0));
-        const unsigned long long before = atomicAdd(slot + 1, 1ull + zero);
-        if ((uint32_t)before + 1u == expected) {
-          const long long a = (long long)atomicExch(slot, 0ull);
-          const unsigned long long f = atomicExch(slot + 1, 0ull);
-          store_row((f >> 32) ? __uint_as_float(0x7FC00000u)
-                              : (float)((double)a * (1.0 / (double)(1ull << NZ_GEMV_FRAC_BITS))),
-                    m);
+        if constexpr (WHOLE) {
+          unsigned long long* slot = reinterpret_cast<unsigned long long*>(gv.acc + 2 * (row * MR + m));
+          unsigned long long r0;
+          if (fabsf(t) < NZ_GEMV_PART_MAX)  // false for NaN as well
+            r0 = atomicAdd(slot, (unsigned long long)__float2ll_rn(t * (float)(1ull << NZ_GEMV_FRAC_BITS)));
+          else
+            r0 = atomicOr(slot + 1, 1ull << 32);
+          asm volatile("v_and_b32 %0, 0, %1" : "=v"(zero) : "v"((uint32_t)r0));
+          const unsigned long long before = atomicAdd(slot + 1, 1ull + zero);
+          if ((uint32_t)before + 1u == expected) {
+            const long long a = (long long)atomicExch(slot, 0ull);
+            const unsigned long long f = atomicExch(slot + 1, 0ull);
+            store_row((f >> 32) ? __uint_as_float(0x7FC00000u)
+                                : (float)((double)a * (1.0 / (double)(1ull << NZ_GEMV_FRAC_BITS))),
+                      m);
+          }
+        } else {
+          uint32_t* slot = reinterpret_cast<uint32_t*>(gv.acc) + (row * MR + m) * gv.acc_words;
+          const uint32_t r0 = atomicExch(slot + 1 + place, __float_as_uint(t));
+          asm volatile("v_and_b32 %0, 0, %1" : "=v"(zero) : "v"(r0));
+          if (atomicAdd(slot, 1u + zero) + 1u == expected) {
+            double a = 0.0;  // (exact for two partial sums of like size, so that the rounding below is the only one)
+            for (uint32_t q = 0; q < expected; ++q) a += (double)__uint_as_float(atomicExch(slot + 1 + q, 0u));
+            atomicExch(slot, 0u);
+            store_row((float)a, m);
+          }
         }
       }
     }
@@ -3051,7 +3077,7 @@ struct NzBatchItem {
   const uint8_t* norm; // group bytes of a normalized tensor
   NzGeom g;
   uint32_t chunk_end;
-  uint32_t reserved;
+  uint32_t acc_words;  // NzGemv
   // dense output of a tensor whose last write is not known to have fitted its buffer: the words in that
   // write's scratch (null: all is known), its nonce, and the container to take if they say it is not whole
   const NzLbWords* late;
@@ -3099,7 +3125,7 @@ __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_ker
   }
   const NzBatchItem& it = b.item[t];
   const NzPart p(blockIdx.x, b.parts, it.g.spc);
-  const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features};
+  const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features, it.acc_words};
   nz_decode_chunk<S, MR, NORM, false, ONE, WHOLE>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
                                         at - first, gv, NzNorm{it.norm, b.log2n}, p.first, p.end);
 }
