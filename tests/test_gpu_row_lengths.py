@@ -212,3 +212,48 @@ def test_capture_without_a_product_before_it():
         torch.cuda.synchronize()
         assert torch.allclose(y, torch.nn.functional.linear(x, w), rtol=2e-2, atol=2e-3)
     mgr._be.check()
+
+
+def test_a_captured_linear_shares_nothing_with_other_calls():
+    """Rows that are not whole groups: the accumulators of the fused product belong to the manager, so a
+    captured call decodes and multiplies into memory of its own and can be replayed beside products on another stream."""
+    import neuzip_amd
+
+    mgr = neuzip_amd.Manager()
+    cols = 1000
+    ws = [(torch.randn(64, cols, device="cuda") * 0.02).to(torch.bfloat16) for _ in range(3)]
+    hs = [mgr.write(w) for w in ws]
+    x = torch.randn(2, cols, device="cuda").to(torch.bfloat16)
+    other = torch.randn(2, cols, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        for _ in range(3):  # the three share a launch from the second time on
+            eager = [mgr.linear(h, x) for h in hs]
+            mgr.linear(hs[0], other)
+        mgr.linear(hs[0], x)  # leaves results of the other two behind
+        for w in ws:
+            torch.nn.functional.linear(x, w)  # the GEMM library is ready
+        torch.cuda.synchronize()
+        made = []
+        real = mgr._be._product
+        mgr._be._product = lambda fn, names, *a: (real(fn, names, *a), made.append(names[0]))[0]
+        try:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                ys = [mgr.linear(h, x) for h in hs]
+            assert not made
+            side = torch.cuda.Stream()
+            for k in range(4):
+                x.copy_(torch.randn(2, cols, device="cuda"))
+                torch.cuda.synchronize()
+                with torch.cuda.stream(side):
+                    beside = [mgr.linear(hs[0], other) for _ in range(8)]
+                graph.replay()
+                torch.cuda.synchronize()
+                for y, w in zip(ys, ws):
+                    assert torch.allclose(y, torch.nn.functional.linear(x, w), rtol=2e-2, atol=2e-3), k
+                for y in beside:
+                    assert torch.allclose(y, torch.nn.functional.linear(other, ws[0]), rtol=2e-2, atol=2e-3), k
+            assert made
+        finally:
+            del mgr._be._product
+    mgr._be.check()
