@@ -1085,6 +1085,7 @@ int order_scratch_use(nz_manager* m, hipStream_t st, bool* captured = nullptr);
 bool late_reads(nz_manager* m, int k, hipStream_t st) {
   RewriteSlot& s = m->rw[k];
   if (!s.busy || s.stream != st || hipEventQuery(s.ev) == hipSuccess || capturing(st)) return false;
+  if (st == hipStreamPerThread) return false;  // one handle, and a stream of its own in every thread
   if (hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();  // (the query's)
   for (uint32_t j = 0; j < s.count; ++j)
     if (!s.b.item[j].direct) return false;  // (records that a second kernel places are not marked)
