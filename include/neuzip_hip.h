@@ -280,7 +280,12 @@ int nz_manager_write_batch(nz_manager* m, const char* const* names, const void* 
    headroom, is then given a larger one and re-compacted from scratch memory
    that is kept until then).  Counters for tests and tuning: batches written in
    place so far, entries that outgrew their buffer, entries whose records were
-   placed a second time (see nz_set_lookback_spins).  Settles what is pending. */
+   placed a second time (see nz_set_lookback_spins).  Settles what is pending.
+   (Scratch is allocated by the first such writes, and by a larger one: the
+   encode workspace, more than two bytes per element, and, once a read has come
+   while the write before it was still running, a byte per element and a little
+   more, up to 128 MiB, into which containers that have outgrown their buffers
+   are put for such reads.  Twice per manager; nz_manager_trim frees both.) */
 int nz_manager_rewrite_stats(nz_manager* m, uint64_t* in_place_batches, uint64_t* outgrown_entries,
                              uint64_t* placed_again);
 
@@ -411,8 +416,8 @@ int nz_manager_import(nz_manager* m, const char* name, const void* host_comp, ui
                       const void* host_packed, uint64_t packed_bytes, const void* host_norm,
                       uint64_t norm_bytes, void* stream);
 
-/* Release the manager's scratch (the workspace of the largest write so far, the
-   accumulators of the matrix-vector product, unless a captured product holds
+/* Release the manager's scratch (the workspace of the largest write so far, what
+   in-place writes keep, see nz_manager_rewrite_stats, the accumulators of the matrix-vector product, unless a captured product holds
    their address: they are needed when its graph is replayed and are then kept);
    it is allocated again on demand.
    The reference allocates its scratch per call (cuda/high_level.cu:81-108).

@@ -516,7 +516,7 @@ struct RewriteSlot {
   std::string names[NZ_ENC_BATCH_MAX];
   NzEncBatch b;
   // for reads that are enqueued before the outcome is known (late_reads): room for a container of any size
-  // for each tensor, at late_at[] of `late`, filled by nz_late_kernel if it is needed
+  // for each tensor, at late_at[] of `late` (null: none, reads wait), filled by nz_late_kernel if it is needed
   bool late_ready = false;
   void* late = nullptr;
   uint64_t late_bytes = 0;
@@ -1078,6 +1078,26 @@ int settle_all(nz_manager* m) {
 bool capturing(hipStream_t st);
 int order_scratch_use(nz_manager* m, hipStream_t st, bool* captured = nullptr);
 
+// Room for the containers of slot k's batch, for late_reads: found by the write, because a read allocates nothing.
+// At most 128 MiB, a batch of some 130 million elements: the 10 us and more that a wait costs are little beside
+// the encode of a larger one.
+constexpr uint64_t NZ_LATE_MAX_BYTES = 128ull << 20;
+void late_room(RewriteSlot& s) {
+  s.late_at[0] = 256;  // before the containers a place for a size and a status that nobody reads
+  for (uint32_t j = 0; j < s.count; ++j) s.late_at[j + 1] = align_up(s.late_at[j] + nz_geom_bound(&s.b.item[j].g), 256);
+  const uint64_t need = s.late_at[s.count];
+  if (s.late_bytes >= need || need > NZ_LATE_MAX_BYTES) return;
+  if (s.late && hipFree(s.late) != hipSuccess) return;
+  s.late = nullptr;
+  s.late_bytes = 0;
+  if (hipMalloc(&s.late, need) != hipSuccess) {  // short of memory: reads wait
+    (void)hipGetLastError();
+    s.late = nullptr;
+    return;
+  }
+  s.late_bytes = need;
+}
+
 // Can a read on `st` of an entry of slot k be enqueued without waiting for the write's outcome?
 // Where the write is still running on that very stream, it can: nz_late_kernel, launched once per
 // write, sees to the tensors whose container is not whole.  (Rewrite and read of the four weights of a
@@ -1091,23 +1111,8 @@ bool late_reads(nz_manager* m, int k, hipStream_t st) {
     if (!s.b.item[j].direct) return false;  // (records that a second kernel places are not marked)
   if (order_scratch_use(m, st) != NZ_OK) return false;  // the read uses the slot's scratch
   if (s.late_ready) return true;
-  if (!m->late_wanted) {  // the first time a read comes this soon it waits: the buffer's allocation would make it longer
-    m->late_wanted = true;
-    return false;
-  }
-  s.late_at[0] = 256;  // before the containers a place for a size and a status that nobody reads
-  for (uint32_t j = 0; j < s.count; ++j) s.late_at[j + 1] = align_up(s.late_at[j] + nz_geom_bound(&s.b.item[j].g), 256);
-  if (s.late_bytes < s.late_at[s.count]) {
-    if (s.late && hipFree(s.late) != hipSuccess) return false;
-    s.late = nullptr;
-    s.late_bytes = 0;
-    if (hipMalloc(&s.late, s.late_at[s.count]) != hipSuccess) {  // short of memory: reads wait
-      (void)hipGetLastError();
-      s.late = nullptr;
-      return false;
-    }
-    s.late_bytes = s.late_at[s.count];
-  }
+  m->late_wanted = true;  // (the write before the first read that comes this soon has found no room for it)
+  if (!s.late || s.late_bytes < s.late_at[s.count]) return false;
   NzEncBatch b = s.b;
   for (uint32_t j = 0; j < b.count; ++j) {
     NzEncItem& it = b.item[j];
@@ -1267,6 +1272,7 @@ int nz_manager_write_batch(nz_manager* m, const char* const* names, const void* 
                              (uint8_t*)ent.norm);
       s.b.item[i].d_gave_up = s.d_totals + 16 + i;
     }
+    if (m->late_wanted) late_room(s);
     if (int rc = encode_phase1(&s.b, m->precision, m->normalizer, st)) return rc;
     if (int rc = encode_phase2(&s.b, st)) return rc;
     NZ_HIP(hipEventRecord(s.ev, st));  // behind it the sizes and give-up marks are in the pinned block

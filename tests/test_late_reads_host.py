@@ -68,3 +68,27 @@ for k in range(4):
     rewrite(b"w", N, PER_THREAD)
     assert read(b"w", N, PER_THREAD)[0] == 1  # may be another thread's
 """)
+
+
+def test_reads_allocate_nothing(child):
+    """The room that a read behind a write may need is the write's to find, and has a bound."""
+    child("""
+store(h, b"v", 80)
+for name, n in ((b"w", N), (b"v", 2 * N), (b"w", N), (b"v", 2 * N)):
+    for k in range(3):
+        rewrite(name, n, 64)
+        assert read(name, n, 64)[1] == 0
+assert read(b"v", 2 * N, 64)[0] == 0 and read(b"w", N, 64)[1] == 0
+# 135 million elements: more room than is kept for this, the read waits
+big = 132000
+store(h, b"b", big)
+for k in range(3):
+    rewrite(b"b", big * CHUNK, 64)
+    assert read(b"b", big * CHUNK, 64)[:2] == (1, 0)
+rewrite(b"w", N, 64)
+assert read(b"w", N, 64)[:2] == (0, 0)
+L.nz_manager_trim(h)  # gives the room back; the next write finds it again
+rewrite(b"w", N, 64)
+assert read(b"w", N, 64)[:2] == (0, 0)
+L.nz_manager_destroy(h)
+""")
