@@ -346,13 +346,6 @@ int nz_manager_linear_rows_batch(nz_manager* m, const char* const* names, uint32
                                  const void* dev_x, uint32_t x_rows, uint32_t in_features,
                                  const void* const* dev_bias, void* const* dev_y, void* stream);
 
-/* Sums over the rows of a contiguous bf16 matrix (the gradient of a Linear's
-   bias, autograd's `grad.sum(0)`): formed in fp32, in an order of their own,
-   rounded once.  cols a multiple of 8; dev_bf16 and dev_scratch 16-byte
-   aligned, dev_scratch of nz_row_sums_bytes; dev_out: cols bf16. */
-uint64_t nz_row_sums_bytes(uint64_t rows, uint64_t cols);
-int nz_row_sums(const void* dev_bf16, uint64_t rows, uint64_t cols, void* dev_scratch, void* dev_out, void* stream);
-
 /* Embedding lookup on a stored table (neuzip/nn/embedding.py:30-39 decompresses
    the WHOLE table for every forward): row dev_indices[i] (int64) of the table
    `name`, read as rows of row_len elements, goes to dev_out[i * row_len ...];

@@ -26,7 +26,7 @@ DECODE_CHECK, DECODE_STREAM_OUT, DECODE_RESIDENT_OUT = 1, 2, 4  # nz_decode flag
 
 EXPORTS = [
     "nz_abi_version", "nz_last_error", "nz_packed_bytes", "nz_packed_stored_bytes", "nz_exp_bound_bytes",
-    "nz_encode_workspace_bytes", "nz_norm_bytes", "nz_row_sums_bytes", "nz_row_sums", "nz_split", "nz_encode", "nz_encode_static", "nz_decode",
+    "nz_encode_workspace_bytes", "nz_norm_bytes", "nz_split", "nz_encode", "nz_encode_static", "nz_decode",
     "nz_manager_create", "nz_manager_destroy", "nz_manager_set_size_budget", "nz_manager_size_budget", "nz_estimated_size_ratio", "nz_manager_in_budget", "nz_manager_write", "nz_manager_write_batch",
     "nz_manager_read", "nz_manager_read_batch", "nz_manager_gemv_batch", "nz_manager_gemv_rows_batch", "nz_manager_linear_rows_batch", "nz_manager_gather_rows",
     "nz_manager_meta", "nz_manager_geometry", "nz_manager_size", "nz_manager_size_reference", "nz_manager_exp_bytes", "nz_manager_packed_bytes",
@@ -61,10 +61,6 @@ def load() -> ctypes.CDLL:
     L.nz_exp_bound_bytes.argtypes = [u64, u32, u32]
     L.nz_encode_workspace_bytes.restype = u64
     L.nz_encode_workspace_bytes.argtypes = [u64, u32, u32]
-    L.nz_row_sums_bytes.restype = u64
-    L.nz_row_sums_bytes.argtypes = [u64, u64]
-    L.nz_row_sums.restype = i32
-    L.nz_row_sums.argtypes = [vp, u64, u64, vp, vp, vp]
     L.nz_split.restype = i32
     L.nz_norm_bytes.restype = u64
     L.nz_norm_bytes.argtypes = [u64, u32]

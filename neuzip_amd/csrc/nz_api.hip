@@ -610,36 +610,6 @@ int nz_split(const void* dev_bf16, uint64_t n, void* dev_exponents, void* dev_fr
   return NZ_OK;
 }
 
-// rows of the matrix that a workgroup of nz_row_sums adds: 512 workgroups or so, of at least 32 rows
-static uint64_t row_sums_per(uint64_t rows, uint64_t cols) {
-  const uint64_t across = (cols + NZ_SUM_COLS - 1) / NZ_SUM_COLS, down = 512 / across ? 512 / across : 1;
-  const uint64_t per = (rows + down - 1) / down;
-  return per < 32 ? 32 : (per + 31) / 32 * 32;
-}
-
-uint64_t nz_row_sums_bytes(uint64_t rows, uint64_t cols) {
-  const uint64_t per = row_sums_per(rows, cols);
-  return (rows + per - 1) / per * cols * 4;
-}
-
-int nz_row_sums(const void* dev_bf16, uint64_t rows, uint64_t cols, void* dev_scratch, void* dev_out, void* stream) {
-  if (rows == 0 || cols == 0 || cols % 8 || rows >= 1ull << 31 || cols >= 1ull << 31)
-    return fail(NZ_ERR_ARG, "rows and columns from 1 to 2^31, columns in eights");
-  if (!dev_bf16 || !dev_scratch || !dev_out) return fail(NZ_ERR_ARG, "null pointer");
-  if (((uintptr_t)dev_bf16 & 15) || ((uintptr_t)dev_scratch & 15) || ((uintptr_t)dev_out & 1))
-    return fail(NZ_ERR_ALIGN, "input and scratch must be 16-byte aligned");
-  const uint64_t per = row_sums_per(rows, cols), parts = (rows + per - 1) / per;  // at most 512 down
-  hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(nz_row_sums_kernel, dim3((uint32_t)((cols + NZ_SUM_COLS - 1) / NZ_SUM_COLS), (uint32_t)parts),
-                     dim3(256), 0, st, (const uint16_t*)dev_bf16, (uint32_t)rows, (uint32_t)cols, (uint32_t)per,
-                     (float*)dev_scratch);
-  NZ_HIP(hipGetLastError());
-  hipLaunchKernelGGL(nz_row_sums_end_kernel, dim3((uint32_t)((cols + 63) / 64)), dim3(1024), 0, st,
-                     (const float*)dev_scratch, (uint32_t)parts, (uint32_t)cols, (uint16_t*)dev_out);
-  NZ_HIP(hipGetLastError());
-  return NZ_OK;
-}
-
 int nz_encode(const void* dev_bf16, uint64_t n, int precision, uint32_t chunk_size,
               uint32_t lane_syms, void* dev_packed, void* dev_comp, uint64_t comp_cap,
               void* dev_workspace, uint64_t workspace_bytes, uint64_t* dev_total,

@@ -330,87 +330,6 @@ __global__ __launch_bounds__(256) void nz_split_unpacked_kernel(const uint16_t* 
 
 #endif  // NZ_TEMPLATES_ONLY
 
-#ifndef NZ_TEMPLATES_ONLY
-// ----------------------------------------------------------------------------
-// sums over the rows of a bf16 matrix (the gradient of a Linear's bias)
-// ----------------------------------------------------------------------------
-// Bound by the read of the matrix.  A workgroup adds `per` rows of 512 columns, a lane eight columns of
-// every fourth row with eight loads under way, and leaves fp32 sums; the second kernel adds
-// those of all workgroups, 64 columns to each of its own, in the order of the rows, and rounds.
-// 8192 x 1024: 4.8 + 4.3 us, 8192 x 4096: 12.4 + 4.7 (5.4 TB/s in the first); torch's reduction and the
-// fill before it 25.5 and 29.2.
-#define NZ_SUM_COLS 512u
-__global__ __launch_bounds__(256) void nz_row_sums_kernel(const uint16_t* __restrict__ in, uint32_t rows, uint32_t cols,
-                                                          uint32_t per, float* __restrict__ part) {
-  __shared__ float4 red[3][2][64];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t col = blockIdx.x * NZ_SUM_COLS + 8 * lane;
-  const uint32_t r1 = (blockIdx.y + 1) * per < rows ? (blockIdx.y + 1) * per : rows;
-  float s[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) s[j] = 0.f;
-  const auto add = [&](const uint4 v) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      s[2 * j] += __uint_as_float(w[j] << 16);
-      s[2 * j + 1] += __uint_as_float(w[j] & 0xFFFF0000u);
-    }
-  };
-  if (col < cols) {  // (columns in eights)
-    uint32_t r = blockIdx.y * per + wave;
-    const uint16_t* p = in + (uint64_t)r * cols + col;
-    for (; r + 28 < r1; r += 32, p += 32ull * cols) {
-      uint4 v[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const uint4*>(p + (uint64_t)(4 * q) * cols);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) add(v[q]);
-    }
-    for (; r < r1; r += 4, p += 4ull * cols) add(*reinterpret_cast<const uint4*>(p));
-  }
-  if (wave) {
-    red[wave - 1][0][lane] = make_float4(s[0], s[1], s[2], s[3]);
-    red[wave - 1][1][lane] = make_float4(s[4], s[5], s[6], s[7]);
-  }
-  __syncthreads();
-  if (wave == 0 && col < cols) {
-#pragma unroll
-    for (int w = 0; w < 3; ++w) {
-      const float4 a = red[w][0][lane], b = red[w][1][lane];
-      s[0] += a.x, s[1] += a.y, s[2] += a.z, s[3] += a.w, s[4] += b.x, s[5] += b.y, s[6] += b.z, s[7] += b.w;
-    }
-    float4* to = reinterpret_cast<float4*>(part + (uint64_t)blockIdx.y * cols + col);
-    to[0] = make_float4(s[0], s[1], s[2], s[3]);
-    to[1] = make_float4(s[4], s[5], s[6], s[7]);
-  }
-}
-__global__ __launch_bounds__(1024) void nz_row_sums_end_kernel(const float* __restrict__ part, uint32_t parts, uint32_t cols,
-                                                               uint16_t* __restrict__ out) {
-  __shared__ float red[16][64];
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63, col = blockIdx.x * 64 + lane;
-  float s = 0.f;
-  if (col < cols) {
-    uint32_t k = wave;
-    for (; k + 48 < parts; k += 64) {
-      float v[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = part[(uint64_t)(k + 16 * q) * cols + col];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) s += v[q];
-    }
-    for (; k < parts; k += 16) s += part[(uint64_t)k * cols + col];
-  }
-  red[wave][lane] = s;
-  __syncthreads();
-  if (wave == 0 && col < cols) {
-#pragma unroll
-    for (int w = 1; w < 16; ++w) s += red[w][lane];
-    out[col] = (uint16_t)nz_f32_to_bf16(s);
-  }
-}
-#endif  // NZ_TEMPLATES_ONLY
-
 // ----------------------------------------------------------------------------
 // encode: one workgroup per chunk
 // ----------------------------------------------------------------------------
