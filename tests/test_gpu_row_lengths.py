@@ -257,3 +257,24 @@ def test_a_captured_linear_shares_nothing_with_other_calls():
         finally:
             del mgr._be._product
     mgr._be.check()
+
+
+@pytest.mark.parametrize("cols", [1000, 1024])
+def test_an_error_of_the_product_is_raised(cols):
+    """... and not answered by another path: a library that fails would look like a slow one."""
+    import neuzip_amd
+
+    mgr = neuzip_amd.Manager()
+    h = mgr.write((torch.randn(48, cols, device="cuda") * 0.02).to(torch.bfloat16))
+    x = torch.randn(2, cols, device="cuda").to(torch.bfloat16)
+
+    def fails(*a):
+        raise RuntimeError("planted")
+
+    mgr._be._product = fails
+    with torch.no_grad(), pytest.raises(RuntimeError, match="planted"):
+        mgr.linear(h, x)
+    del mgr._be._product
+    with torch.no_grad():
+        assert torch.isfinite(mgr.linear(h, x)).all()
+    mgr._be.check()
