@@ -50,6 +50,33 @@ def test_held_updates_keep_their_values(ahead):
     mgr._be.check()
 
 
+@pytest.mark.parametrize("fill,copied", [(4, True), (64, False)])
+def test_held_updates_do_not_keep_large_buffers(fill, copied):
+    """A weight decoded together with its neighbours is a view of their common buffer: held as it is,
+    it would keep all of it.  (``fill`` in weights: how much may be held.)"""
+    import neuzip_amd
+
+    mgr = neuzip_amd.Manager()
+    pairs = [_param(mgr, 64, 512) for _ in range(24)]
+    mgr.flush()
+    be = mgr._be
+    be.ahead_fill = fill * 64 * 512
+    for step in range(4):
+        for p, w in pairs:
+            g = torch.randn(64, 512, device="cuda").to(torch.bfloat16)
+            p._gradient = g
+            neuzip_amd.compressed_lomo_hook(_Rate(), p)
+            w.add_(g, alpha=-0.5)
+            stores = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for _, t, _ in be._held}
+            assert sum(stores.values()) <= 2 * 2 * be.ahead_fill, step
+        if be._held and step:
+            shared = any(t.untyped_storage().nbytes() > 2 * t.numel() for _, t, _ in be._held)
+            assert shared != copied
+    for p, w in pairs:
+        assert torch.equal(p(), w)
+    mgr._be.check()
+
+
 def test_plans_and_sizes_follow_the_writes():
     import neuzip_amd
 
