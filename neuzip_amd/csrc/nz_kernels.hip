@@ -1735,13 +1735,45 @@ NZ_HD static inline bool nz_stream_output(uint64_t n) { return 2 * n > NZ_STREAM
 
 // S+1 packed bytes of one group from the stored stream in global memory,
 // which a decode reads exactly once: a streaming (non-temporal) load, so that
-// the bytes do not displace what the caches could keep.
-template <int S>
-__device__ __forceinline__ uint64_t nz_stream_sm(const uint8_t* p) {
+// the bytes do not displace what the caches could keep.  `off`: where the lane's
+// bytes are in the stream of its segment.  One and two bytes come with the 32-bit word
+// around them (which the lanes of the group share: stream and groups are multiples of 64 bytes) and
+// are shifted down where they are used.  Loaded by themselves, they are kept as a byte or half word until that use,
+// groups later, and the compiler masks them to 32 bits wherever it likes: in front of the steps that the load was
+// to be under way for, which then wait for memory (one-read step, 256 chunks, precision 1: 33.5 or 36.0 us with
+// what else was in the kernel, 31.0 with the word; two-read step, 512 chunks: 51.0 and 45.6).
+// ALONE: by themselves all the same.  The row gather, which is bound by one wavefront's steps, needs 16 vector
+// registers more with the words and normalizers, and then has room for three workgroups to a compute unit, not four.
+template <int S, bool ALONE>
+using NzPacked = std::conditional_t<S == 7 || ALONE, uint64_t, uint32_t>;
+template <int S, bool ALONE>
+__device__ __forceinline__ NzPacked<S, ALONE> nz_stream_sm(const uint8_t* stream, uint32_t off) {
+  const uint8_t* p = stream + (S < 3 && !ALONE ? off & ~3u : off);
   if constexpr (S == 7) return __builtin_nontemporal_load(reinterpret_cast<const uint64_t*>(p));
-  else if constexpr (S == 3) return __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
+  else if constexpr (S == 3 || !ALONE) return __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
   else if constexpr (S == 1) return __builtin_nontemporal_load(reinterpret_cast<const uint16_t*>(p));
   else return __builtin_nontemporal_load(p);
+}
+// bits that the lane's bytes lie above the word's lowest
+template <int S, bool ALONE>
+__device__ __forceinline__ uint32_t nz_packed_shift(uint32_t lane) {
+  return ALONE ? 0u : S == 1 ? 16 * (lane & 1) : S == 0 ? 8 * (lane & 3) : 0u;
+}
+// The same for the one normalizer byte of a group of eight elements: the four bytes at `at`, or at `last`, the last
+// place that has four, and how far up the byte is.  (256 chunks, precision 3, groups of 64: 35.5 or 38 us with the byte
+// alone, 33.0 with the word; two-read step, 512 chunks, precision 0, groups of 8: 53.3 and 49.9.)
+struct NzNormByte {
+  uint32_t word, up;
+  __device__ __forceinline__ uint32_t get() const { return __builtin_amdgcn_ubfe(word, 8 * up, 8); }
+};
+template <bool ALONE>
+__device__ __forceinline__ NzNormByte nz_stream_norm(const uint8_t* bytes, uint32_t at, uint32_t last) {
+  if constexpr (ALONE) return NzNormByte{bytes[at], 0u};
+  const uint32_t from = at < last ? at : last;
+  NzNormByte b;
+  __builtin_memcpy(&b.word, bytes + from, 4);
+  b.up = at - from;
+  return b;
 }
 
 // The exponent byte as the decoder's tables hold it: rotated right by one.  An exponent lies across
@@ -2504,7 +2536,17 @@ __device__ __forceinline__ void nz_decode_chunk(
   w.attach(comp, comp_bytes, bad_rec ? 0 : rec_pos, rings + ring * 2 * RING);
   w.nwords = rec_all / 2;
   w.lane = lane;
-  uint64_t sm_next = 0, nb_next = 0;
+  const uint64_t norm_bytes = NORM ? ((g.n - 1) >> nm.log2n) + 1 : 0;
+  const bool wide_norm = nm.log2n >= 3 && norm_bytes >= 4;
+  // Normalizer bytes, where a lane needs one for each of its groups: counted from the segment's first one, or
+  // from the last place that has four, in 32 bits.
+  const uint64_t norm_first = seg_base >> nm.log2n, norm_four = norm_bytes - 4;
+  const uint64_t norm_from = norm_first < norm_four ? norm_first : norm_four;
+  const uint8_t* const norm_at = nm.bytes + norm_from;
+  const uint32_t norm_off = (uint32_t)(seg_base - (norm_from << nm.log2n)) + lane * NZ_GROUP;
+  const uint32_t norm_last = (uint32_t)(norm_four - norm_from < seg_n ? norm_four - norm_from : seg_n);
+  NzPacked<S, ROWS> sm_next = 0;
+  NzNormByte nb_next{};
   constexpr int MR = GEMV ? GEMV : 1;  // activation rows a lane multiplies with (GEMV: 0 = plain decode)
   // The activation of the next group is fetched a group ahead.  Of several rows it is this
   // group's: the registers of the next ones' cost a workgroup per compute unit where there would
@@ -2521,8 +2563,8 @@ __device__ __forceinline__ void nz_decode_chunk(
       if constexpr (X_AHEAD) xq_next = walk.load(walk.col);
     }
     if (whole) {
-      sm_next = nz_stream_sm<S>(pk + lane_off);
-      if constexpr (NORM) nb_next = nz_norm_load8(nm, seg_base + lane * NZ_GROUP);
+      sm_next = nz_stream_sm<S, ROWS>(pk, lane_off);
+      if (NORM && wide_norm) nb_next = nz_stream_norm<ROWS>(norm_at, norm_off >> nm.log2n, norm_last);
     }
   }
   __syncthreads();
@@ -2818,19 +2860,23 @@ __device__ __forceinline__ void nz_decode_chunk(
   // store is waited for.
   const auto sm_at = [&](uint32_t gq) {
     const uint32_t off = gq * NZ_LANES * (S + 1) + lane_off;
-    return nz_stream_sm<S>(pk + (off < last_off ? off : last_off));
+    return nz_stream_sm<S, ROWS>(pk, off < last_off ? off : last_off);
   };
-  // `wide`: groups of 8 elements or more, one byte per lane and group.  The
+  // `wide`: groups of 8 elements or more, one byte per lane and group (where there are four in all).  The
   // walk over the full groups exists once per case, so that the common one has
   // no branch between the byte's load and its use two groups later (a load
   // behind a branch is waited for at the join, with every store before it).
-  const auto nb_at = [&](uint32_t gq, auto wide) -> uint64_t {
-    const uint64_t e0 = seg_base + ((gq < whole ? gq : whole - 1) * NZ_LANES + lane) * NZ_GROUP;
-    if constexpr (decltype(wide)::value) return nm.bytes[e0 >> nm.log2n];
-    else return nz_norm_load8(nm, e0);
+  const auto nb_at = [&](uint32_t gq, auto wide) {
+    const uint32_t e = (gq < whole ? gq : whole - 1) * NZ_GROUP_SYMS;
+    if constexpr (decltype(wide)::value) {
+      return nz_stream_norm<ROWS>(norm_at, (e + norm_off) >> nm.log2n, norm_last);
+    } else {
+      const uint64_t v = nz_norm_load8(nm, seg_base + e + lane * NZ_GROUP);
+      return nm.log2n >= 3 ? v * 0x0101010101010101ull : v;  // (fewer than four normalizers in all)
+    }
   };
   // (`xl`: the group's activations in LDS, or NzNoLds)
-  const auto full_group = [&](uint32_t gq, const uint64_t sm, const uint64_t nb, auto wide, auto fetch_ahead,
+  const auto full_group = [&](uint32_t gq, const NzPacked<S, ROWS> sm, const auto nb, auto wide, auto fetch_ahead,
                               auto xl) __attribute__((always_inline)) {
     constexpr bool X_LDS = !std::is_same_v<decltype(xl), NzNoLds>;
     if constexpr (ONE_READ) w.look();  // before the group's loads: a refill waits for all that are under way
@@ -2845,21 +2891,40 @@ __device__ __forceinline__ void nz_decode_chunk(
     if constexpr (!ONE_READ) w.look();  // (behind them here: 143 us for 8192 x 28672, before them 145)
     uint32_t ew[8];
     w.group(ew);
-    // the merge starts only here: its wait for the packed bytes must not be
+    // the merge starts only here: its wait for the packed bytes (and the normalizers' bytes) must not be
     // hoisted in front of the rANS steps
-    uint32_t sml = (uint32_t)sm, smh = (uint32_t)(sm >> 32);
-    asm volatile("" : "+v"(sml), "+v"(smh), "+v"(ew[7]));
+    constexpr bool WIDE = decltype(wide)::value;
+    uint32_t sml, smh = 0, nbl = 0, nbh = 0;
+    if constexpr (sizeof(sm) == 8) {
+      sml = (uint32_t)sm, smh = (uint32_t)(sm >> 32);
+      asm volatile("" : "+v"(sml), "+v"(smh), "+v"(ew[7]));
+    } else {
+      sml = sm;
+      asm volatile("" : "+v"(sml), "+v"(ew[7]));
+      sml >>= nz_packed_shift<S, ROWS>(lane);
+    }
+    if constexpr (NORM && WIDE) {
+      NzNormByte byte = nb;
+      asm volatile("" : "+v"(byte.word), "+v"(ew[7]));
+      nbl = byte.get();
+    } else if constexpr (NORM) {
+      nbl = (uint32_t)nb, nbh = (uint32_t)(nb >> 32);
+      asm volatile("" : "+v"(nbl), "+v"(nbh), "+v"(ew[7]));
+    }
     if constexpr (ROWS)
       if (!row.overlaps(seg_base + gq * NZ_GROUP_SYMS, NZ_GROUP_SYMS)) return;
     uint4 mv = nz_merge_group<S>(((uint64_t)smh << 32) | sml, ew);
-    if constexpr (NORM) mv = nz_scale8<true>(mv, nb, decltype(wide)::value);
+    if constexpr (NORM) mv = nz_scale8<true>(mv, ((uint64_t)nbh << 32) | nbl, WIDE);
     if constexpr (X_LDS) walk.add(mv, xl, lane);
     else if constexpr (GEMV) walk.add(mv, xq, lane);
     else if constexpr (STREAM) nz_stream_store(dst + (gq * NZ_LANES + lane) * NZ_GROUP, mv);
     else store8((gq * NZ_LANES + lane) * NZ_GROUP, mv);
   };
   const auto full_groups = [&](auto wide) __attribute__((always_inline)) {
-    uint64_t sm_a = sm_next, sm_b = 0, nb_a = nb_next, nb_b = 0;
+    NzPacked<S, ROWS> sm_a = sm_next, sm_b = 0;
+    std::conditional_t<decltype(wide)::value, NzNormByte, uint64_t> nb_a{}, nb_b{};
+    if constexpr (NORM && decltype(wide)::value) nb_a = nb_next;
+    else if constexpr (NORM) nb_a = whole ? nb_at(0, wide) : 0;
     uint32_t gq = 0;
     const auto fetch_a = [&] {
       sm_a = sm_at(gq + 2);
@@ -2898,8 +2963,13 @@ __device__ __forceinline__ void nz_decode_chunk(
     }
     if (gq < whole) full_group(gq, sm_a, nb_a, wide, [] {}, NzNoLds{});
   };
-  if (!NORM || nm.log2n >= 3) full_groups(NzConst<1>{});
-  else full_groups(NzConst<0>{});
+  if (!NORM || wide_norm) full_groups(NzConst<1>{});
+  else {
+    full_groups(NzConst<0>{});
+    // What was fetched for groups that are not there has to come, too: the compiler lets this path run into the other
+    // walk, and would have that wait in every turn for a register that such a load might still be under way to.
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  }
   if ((!GEMV || !WHOLE) && whole < body) {  // the ragged last group of the tensor
     const uint32_t idx0 = (whole * NZ_LANES + lane) * NZ_GROUP;
     uint32_t ew[8];

@@ -44,6 +44,43 @@ def test_encode_decode_match_oracle(oracle, norm, s):
         assert np.array_equal(out, oracle.reconstruct_normalized(bits, s, norm))
 
 
+@pytest.mark.parametrize("norm", [8, 64, 512, 1024])
+@pytest.mark.parametrize("s", [7, 3, 1, 0])
+def test_the_last_normalizers_of_a_tensor(oracle, norm, s):
+    """Tensors with one to six normalizers and segments that begin among the last three: the decoder fetches
+    four bytes at a time, and none behind the last."""
+    sizes = {k * norm - d for k in range(1, 7) for d in (0, 1, norm // 2)} | {k * 512 for k in range(1, 14)} | {8192 + 512, 7 * 1024 + 8}
+    for n in sorted(x for x in sizes if x > 0):
+        bits = _finite(stress_bits(1, n, seed=n))
+        print(f"case norm={norm} s={s} n={n}", flush=True)
+        comp, packed, nb = gpu_encode(bits, s, 2048, 16, norm_size=norm)
+        count = -(-n // norm)
+        # what is in memory behind the last one must not matter
+        for fill in (0, 255):
+            store = torch.full((count + 64,), fill, dtype=torch.uint8, device="cuda")
+            store[:count] = nb
+            rc, out = gpu_decode(comp, packed, n, s, 2048, 16, norm_size=norm, norm=store)
+            assert rc == 0
+            assert np.array_equal(out, oracle.reconstruct_normalized(bits, s, norm))
+
+
+@pytest.mark.parametrize("chunks", [3, 160, 257])
+@pytest.mark.parametrize("kind", ["wide", "bursts"])
+@pytest.mark.parametrize("s,norm", [(7, 64), (3, 8), (3, 4), (1, 512), (0, 64)])
+def test_records_that_refill_the_ring(oracle, s, norm, kind, chunks):
+    """Segments of 8192 symbols with more words than any ring holds, several per group or none for long: refills between
+    groups and inside them, in chunks that workgroups share, at most one workgroup per compute unit, and more."""
+    from test_gpu_decode_forms import _bits as values, _coded_chunks
+
+    n = chunks * 65536 - 1000
+    bits = values(kind, n)
+    print(f"case {kind} chunks={chunks} s={s} norm={norm}", flush=True)
+    comp, packed, nb = gpu_encode(bits, s, 65536, 128, norm_size=norm)
+    assert _coded_chunks(comp.cpu().numpy(), n, 65536, 128) >= chunks - 1
+    rc, out = gpu_decode(comp, packed, n, s, 65536, 128, norm_size=norm, norm=nb)
+    assert rc == 0 and np.array_equal(out, oracle.reconstruct_normalized(bits, s, norm))
+
+
 @pytest.mark.parametrize("e_big,e_x", [(1, 0), (1, 1), (2, 0), (8, 0), (9, 1), (127, 120), (254, 254), (254, 200)])
 def test_every_mantissa_pair_on_the_gpu(oracle, e_big, e_x):
     """Groups of two [maximum with mantissa mb, element with mantissa mx] around the
