@@ -1675,9 +1675,9 @@ static_assert(2 * (NZ_M - NZ_TMETA_SLOT) >= NZ_TMETA_DWORDS && NZ_TMETA_SLOT % 3
 //   gather   1 row 32.5 / 27.8, 256 rows 40.5 / 38.1, 320 rows 48.2 / 47.8, 512 rows 52.4 / 53.3
 // It counts workgroups and not wavefronts: chunks of four wavefronts (65536 / 256)
 // would still gain above it (320: 34.6 / 30.8, 512: 35.5 / 32.4, 768: 39.4 / 38.3)
-// and lose at 1024 (45.2 / 61.1); reads with normalizers (320, precision 3, groups of 64:
-// 50.3 / 47.2) would gain as well.
-// Those keep the two-read step.  Below the line it costs where a wavefront
+// and lose at 1024 (45.2 / 61.1).  Those keep the two-read step, and so do reads with normalizers (narrow
+// ring; precision 3, groups of 64: 320 chunks 45.0 / 45.3, 512: 49.7 / 51.3, precision 7: 45.5 / 44.7, 52.2 / 52.5).
+// Below the line it costs where a wavefront
 // takes many words (6 bits per exponent, 256 workgroups: 36.3 / 36.9; 8 workgroups:
 // 29.8 / 27.1) and where four streams launch 256 workgroups each at the same time
 // (342 / 370 for sixteen reads: two workgroups to a compute unit and not three;
@@ -2443,12 +2443,7 @@ __device__ __forceinline__ void nz_decode_chunk(
     uint16_t* __restrict__ out, const NzGeom& g, uint32_t* __restrict__ d_status, const uint64_t c,
     const NzGemv& gv, const NzNorm& nm, const uint32_t first_seg, const uint32_t end_seg,
     const NzRowOut& row = NzRowOut{}) {
-  // One read per step with the narrow ring for normalizers as well (precision 3 and 7; 264 to 512 chunks): precision 3, groups of
-  // 64: 320 chunks 45.8 -> 42.8 us, 512 48.1 -> 46.8, groups of 2: 59.9 -> 56.1, 66.9 -> 62.3, precision 7: 44.7 -> 41.5,
-  // 46.5 -> 44.4.  With the wide ring 320 chunks take 46.5; precision 0, groups of 8, loses (512: 51.5 -> 54.5).
-  constexpr bool NORM_ONE = NORM && !STREAM && !ONE && S >= 3;
-  constexpr bool ONE_READ = ONE || GEMV || ROWS || NORM_ONE;
-  constexpr bool PAIRS = GEMV || ROWS || NORM_ONE || (ONE && !NORM && S >= 3);  // how the slot table is filled
+  constexpr bool ONE_READ = ONE || GEMV || ROWS;
   // At LDS address 0: a kernel that decodes has no static LDS (pinned in tests/test_kernel_resources.py),
   // because NzWaveDecOne numbers table and rings through from there.
   extern __shared__ uint32_t lds[];
@@ -2571,8 +2566,7 @@ __device__ __forceinline__ void nz_decode_chunk(
   // the first 32 table bytes hold the mode and all run descriptors there can be
   const uint4 h0 = reinterpret_cast<const uint4*>(tb)[0], h1 = reinterpret_cast<const uint4*>(tb)[1];
   const uint32_t bm_byte = tb[1 + (lane >> 1)];  // bitmap mode: the byte with this lane's four symbols
-  uint32_t mode = h0.x & 0xFFu;
-  if constexpr (PAIRS) mode = (uint32_t)__builtin_amdgcn_readfirstlane(mode);
+  const uint32_t mode = (uint32_t)__builtin_amdgcn_readfirstlane(h0.x & 0xFFu);
   uint32_t tab_len = 4;
 
   if (mode != NZ_MODE_RAW) {
@@ -2600,47 +2594,27 @@ __device__ __forceinline__ void nz_decode_chunk(
       } else {
         head = 1 + 2 * mode;
         uint32_t acc = 0;
-        if constexpr (PAIRS) {
-          // the run descriptors, 16 bits each from the second byte on, move down through scalar registers
-          const auto pair = [](uint32_t lo, uint32_t hi) {
-            return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(lo) | ((uint64_t)__builtin_amdgcn_readfirstlane(hi) << 32);
-          };
-          uint64_t q0 = pair(h0.x, h0.y), q1 = pair(h0.z, h0.w), q2 = pair(h1.x, h1.y), q3 = pair(h1.z, h1.w);
+        // the run descriptors, 16 bits each from the second byte on, move down through scalar registers
+        const auto pair = [](uint32_t lo, uint32_t hi) {
+          return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(lo) | ((uint64_t)__builtin_amdgcn_readfirstlane(hi) << 32);
+        };
+        uint64_t q0 = pair(h0.x, h0.y), q1 = pair(h0.z, h0.w), q2 = pair(h1.x, h1.y), q3 = pair(h1.z, h1.w);
 #pragma nounroll
-          for (uint32_t r = 0; r < mode; ++r) {
-            const uint32_t st = (uint32_t)(q0 >> 8) & 0xFFu, ln = ((uint32_t)(q0 >> 16) & 0xFFu) + 1u;
-            q0 = q0 >> 16 | q1 << 48;
-            q1 = q1 >> 16 | q2 << 48;
-            q2 = q2 >> 16 | q3 << 48;
-            q3 >>= 16;
+        for (uint32_t r = 0; r < mode; ++r) {
+          const uint32_t st = (uint32_t)(q0 >> 8) & 0xFFu, ln = ((uint32_t)(q0 >> 16) & 0xFFu) + 1u;
+          q0 = q0 >> 16 | q1 << 48;
+          q1 = q1 >> 16 | q2 << 48;
+          q2 = q2 >> 16 | q3 << 48;
+          q3 >>= 16;
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
-              const uint32_t d = 4 * lane + j - st;
-              if (d < ln) {
-                live4 |= 1u << j;
-                rk[j] = acc + d;
-              }
-            }
-            acc += ln;
-          }
-        } else {
-          const uint32_t hw[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-#pragma unroll
-          for (uint32_t r = 0; r < NZ_MAX_RUNS; ++r) {
-            if (r < mode) {
-              const uint32_t st = (hw[(1 + 2 * r) >> 2] >> (8 * ((1 + 2 * r) & 3))) & 0xFFu;
-              const uint32_t ln = ((hw[(2 + 2 * r) >> 2] >> (8 * ((2 + 2 * r) & 3))) & 0xFFu) + 1u;
-#pragma unroll
-              for (uint32_t j = 0; j < 4; ++j) {
-                const uint32_t sym = 4 * lane + j;
-                if (sym >= st && sym < st + ln) {
-                  live4 |= 1u << j;
-                  rk[j] = acc + sym - st;
-                }
-              }
-              acc += ln;
+          for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t d = 4 * lane + j - st;
+            if (d < ln) {
+              live4 |= 1u << j;
+              rk[j] = acc + d;
             }
           }
+          acc += ln;
         }
         kk = acc;
       }
@@ -2694,69 +2668,39 @@ __device__ __forceinline__ void nz_decode_chunk(
     // write to different banks.  (One slot at a time, two LDS reads and a write of 8 bytes for each, the
     // fill took 2900 cycles, of some 50000 that a chunk of 256 symbols per lane takes.  With this, and the
     // run descriptors in scalar registers above: read of 1024 x 1024 22.2 -> 21.5 us, gather of a row 21.8 -> 21.2,
-    // one and eight rows through the Linears of a block of width 4096 160.6 -> 158.4, 237.4 -> 234.0.)
-    // Elsewhere consecutive threads fill consecutive slots one by one, and every thread keeps its part of the last:
-    // the compiler's code for the steps behind the fill in pairs was slower there.  With pairs and without, two-read
-    // step: 512 chunks, precision 1: 52.4 and 48.8 us; 1023 chunks, precision 0, normalizers of 8: 111.9 and 102.3;
-    // precision 7: 43.4 and 42.6.  One-read step, 128 chunks: precision 0: 28.5 and 26.7,
-    // precision 7 with normalizers of 64: 30.5 and 29.3.
+    // one and eight rows through the Linears of a block of width 4096 160.6 -> 158.4, 237.4 -> 234.0; reads of 128
+    // chunks, precision 0, 26.0 -> 25.1, precision 7 with normalizers of 64 27.6 -> 27.0, of 512 chunks, two-read
+    // step, precision 1, 46.4 -> 45.9.)
     {
-      uint32_t table_ok, table_len;
-      if constexpr (PAIRS) {
-        const auto slot_at = [&](uint32_t at, uint32_t i) { return at + 2u * ((i + (lane >> 2)) & 3u); };
-        const auto entries = [&](uint32_t at, uint4 (&en)[4]) {
-          const uint2 wn = wins[at >> 5];
+      const auto slot_at = [&](uint32_t at, uint32_t i) { return at + 2u * ((i + (lane >> 2)) & 3u); };
+      const auto entries = [&](uint32_t at, uint4 (&en)[4]) {
+        const uint2 wn = wins[at >> 5];
 #pragma unroll
-          for (uint32_t i = 0; i < 4; ++i) {
-            const uint32_t slot = slot_at(at, i), bit = slot & 31;
-            const uint32_t k = wn.y + (uint32_t)__popc(wn.x & ((2u << bit) - 1u)) - 1u;
-            const uint2 a = runs[k & 255u];
-            uint2 b = a;
-            if ((wn.x >> (bit + 1)) & 1u) b = runs[(k + 1u) & 255u];
-            en[i] = make_uint4(a.x, slot - a.y, b.x, slot + 1u - b.y);
-          }
-        };
-        const auto put = [&](uint32_t at, const uint4 (&en)[4]) {
-#pragma unroll
-          for (uint32_t i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(lut + slot_at(at, i)) = en[i];
-        };
-        uint4 en[4];
-        // (whole rounds end at slot 3584 at the latest, with 64, 128, ... 512 threads)
-        static_assert(NZ_M - 8 * NZ_LANES <= NZ_TMETA_SLOT, "");
-        uint32_t at = 8 * tid;
-        for (uint32_t done = 8 * blockDim.x; done < NZ_M; done += 8 * blockDim.x, at += 8 * blockDim.x) {
-          entries(at, en);
-          put(at, en);
+        for (uint32_t i = 0; i < 4; ++i) {
+          const uint32_t slot = slot_at(at, i), bit = slot & 31;
+          const uint32_t k = wn.y + (uint32_t)__popc(wn.x & ((2u << bit) - 1u)) - 1u;
+          const uint2 a = runs[k & 255u];
+          uint2 b = a;
+          if ((wn.x >> (bit + 1)) & 1u) b = runs[(k + 1u) & 255u];
+          en[i] = make_uint4(a.x, slot - a.y, b.x, slot + 1u - b.y);
         }
-        if (at < NZ_M) entries(at, en);
-        table_ok = tflag[0], table_len = tflag[1];
-        __syncthreads();
-        if (at < NZ_M) put(at, en);
-      } else {
-        const uint32_t below = (2u << (tid & 31)) - 1u;  // bits of a window up to this thread's slot
-        const auto entry_of = [&](uint32_t slot) {
-          const uint2 wn = wins[slot >> 5];
-          const uint32_t k = wn.y + (uint32_t)__popc(wn.x & below) - 1u;
-          const uint2 rn = runs[k & 255u];
-          return make_uint2(rn.x, slot - rn.y);
-        };
-        for (uint32_t slot = tid; slot < NZ_TMETA_SLOT; slot += blockDim.x) lut[slot] = entry_of(slot);
-        // (NZ_TMETA_SLOT is a multiple of 32, so `below` fits these slots as well)
-        constexpr uint32_t LAST = (NZ_M - NZ_TMETA_SLOT + 63) / 64;  // per thread, for the smallest workgroup
-        uint2 last[LAST];
+      };
+      const auto put = [&](uint32_t at, const uint4 (&en)[4]) {
 #pragma unroll
-        for (uint32_t i = 0; i < LAST; ++i) {
-          const uint32_t slot = NZ_TMETA_SLOT + tid + i * blockDim.x;
-          last[i] = slot < NZ_M ? entry_of(slot) : make_uint2(0u, 0u);
-        }
-        table_ok = tflag[0], table_len = tflag[1];
-        __syncthreads();
-#pragma unroll
-        for (uint32_t i = 0; i < LAST; ++i) {
-          const uint32_t slot = NZ_TMETA_SLOT + tid + i * blockDim.x;
-          if (slot < NZ_M) lut[slot] = last[i];
-        }
+        for (uint32_t i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(lut + slot_at(at, i)) = en[i];
+      };
+      uint4 en[4];
+      // (whole rounds end at slot 3584 at the latest, with 64, 128, ... 512 threads)
+      static_assert(NZ_M - 8 * NZ_LANES <= NZ_TMETA_SLOT, "");
+      uint32_t at = 8 * tid;
+      for (uint32_t done = 8 * blockDim.x; done < NZ_M; done += 8 * blockDim.x, at += 8 * blockDim.x) {
+        entries(at, en);
+        put(at, en);
       }
+      if (at < NZ_M) entries(at, en);
+      const uint32_t table_ok = tflag[0], table_len = tflag[1];
+      __syncthreads();
+      if (at < NZ_M) put(at, en);
       if (!table_ok) {
         if (tid == 0) atomicOr(d_status, 2u);
         return;
