@@ -2484,8 +2484,12 @@ __device__ __forceinline__ void nz_decode_chunk(
     if (tid == 0) atomicOr(d_status, 2u);
     return;
   }
-  bool has_seg = wave < nseg && wave >= first_seg && wave < end_seg;
-  uint32_t ring = wave - first_seg + (first_seg ? 1u : 0u);  // the first segment's record, with the table, has the first one
+  bool has_seg = wave < nseg;
+  uint32_t ring = wave;  // the first segment's record, with the table, has the first one
+  if constexpr (ONE && !ROWS) {
+    has_seg = has_seg && wave >= first_seg && wave < end_seg;
+    ring = wave - first_seg + (first_seg ? 1u : 0u);
+  }
   if constexpr (ROWS) {
     const uint32_t from = row.first > chunk_base ? (uint32_t)((row.first - chunk_base) / g.seg_syms) : 0u;
     has_seg = has_seg && row.overlaps(chunk_base + (uint64_t)wave * g.seg_syms, g.seg_syms);
@@ -2550,7 +2554,8 @@ __device__ __forceinline__ void nz_decode_chunk(
   constexpr bool X_AHEAD = MR == 1;
   NzXq<X_AHEAD ? MR : 1> xq_next{};
   NzGemvWalk<MR, WHOLE> walk;
-  if (wave == 0 && !has_seg && !bad_rec) w.stage();  // the table
+  if constexpr (ONE || ROWS)
+    if (wave == 0 && !has_seg && !bad_rec) w.stage();  // the table
   if (has_seg && !bad_rec) {
     w.stage();
     if constexpr (GEMV) {
@@ -2991,7 +2996,7 @@ template <int S, bool NORM, bool STREAM, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_kernel(
     const uint8_t* __restrict__ comp, uint64_t comp_bytes, const uint8_t* __restrict__ packed,
     uint16_t* __restrict__ out, NzGeom g, uint32_t* __restrict__ d_status, const NzNorm nm, const uint32_t parts) {
-  const NzPart p(blockIdx.x, parts, g.spc);
+  const NzPart p(blockIdx.x, ONE ? parts : 1u, g.spc);
   nz_decode_chunk<S, 0, NORM, STREAM, ONE>(comp, comp_bytes, packed, out, g, d_status, p.chunk, NzGemv{}, nm, p.first, p.end);
 }
 
@@ -3032,13 +3037,13 @@ template <int S, bool NORM, bool STREAM, bool ONE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_batch_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
   uint32_t t = 0, first = 0;
-  const uint32_t at = blockIdx.x >> (31u - (uint32_t)__builtin_clz(b.parts));
+  const uint32_t parts = ONE ? b.parts : 1u, at = blockIdx.x >> (31u - (uint32_t)__builtin_clz(parts));
   while (t + 1 < b.count && at >= b.item[t].chunk_end) {
     first = b.item[t].chunk_end;
     ++t;
   }
   const NzBatchItem& it = b.item[t];
-  const NzPart p(blockIdx.x, b.parts, it.g.spc);
+  const NzPart p(blockIdx.x, parts, it.g.spc);
   const bool other = it.late && nz_lb_not_whole(it.late, it.late_nonce);
   nz_decode_chunk<S, 0, NORM, STREAM, ONE>(other ? it.late_comp : it.comp, other ? it.late_bytes : it.comp_bytes,
                                           it.packed, it.out, it.g, d_status, at - first, NzGemv{},
@@ -3051,13 +3056,13 @@ template <int S, bool NORM, int MR, bool ONE, bool WHOLE>
 __global__ __launch_bounds__(64 * NZ_MAX_SEGS_PER_CHUNK) void nz_decode_gemv_kernel(
     const NzBatch b, uint32_t* __restrict__ d_status) {
   uint32_t t = 0, first = 0;
-  const uint32_t at = blockIdx.x >> (31u - (uint32_t)__builtin_clz(b.parts));
+  const uint32_t parts = ONE ? b.parts : 1u, at = blockIdx.x >> (31u - (uint32_t)__builtin_clz(parts));
   while (t + 1 < b.count && at >= b.item[t].chunk_end) {
     first = b.item[t].chunk_end;
     ++t;
   }
   const NzBatchItem& it = b.item[t];
-  const NzPart p(blockIdx.x, b.parts, it.g.spc);
+  const NzPart p(blockIdx.x, parts, it.g.spc);
   const NzGemv gv{b.x, it.acc, it.y, it.bias, b.in_features, it.acc_words};
   nz_decode_chunk<S, MR, NORM, false, ONE, WHOLE>(it.comp, it.comp_bytes, it.packed, nullptr, it.g, d_status,
                                         at - first, gv, NzNorm{it.norm, b.log2n}, p.first, p.end);
