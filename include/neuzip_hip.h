@@ -245,10 +245,10 @@ int nz_manager_in_budget(const nz_manager* m, uint64_t n, uint32_t chunk_size, u
    stream order, or after an event / synchronisation; memory from a
    stream-ordered allocator that belongs to another stream has to be told, as
    torch's record_stream does).
-   Streams and graphs: writes, products and row gathers of one manager share
-   its scratch memory; a call that arrives on another stream than the one
-   before it is ordered behind that one on the device (an event, no host
-   wait).  A call that may allocate or wait on the host - every write, a read
+   Streams and graphs: writes and products of one manager share its scratch
+   memory; such a call, or a row gather, that arrives on another stream than
+   the one before it is ordered behind that one on the device (an event, no
+   host wait).  A call that may allocate or wait on the host - every write, a read
    or product of an entry whose in-place rewrite has not been looked at yet, a
    product that needs larger accumulators, a row gather - is refused with
    NZ_ERR_ARG while its stream is being captured into a graph, before it

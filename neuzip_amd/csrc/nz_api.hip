@@ -533,7 +533,7 @@ struct nz_manager {
   bool own_lanes = false;   // lane_syms 0 or AUTO was given: the segment length follows the size budget
   bool auto_lanes = false;  // pick the geometry per tensor so that small tensors still fill the GPU
   double budget = NZ_DEFAULT_SIZE_BUDGET;  // stored exponent bytes over their order-0 entropy the manager's own choices stay within
-  hipStream_t last_stream = nullptr;  // stream of the last call that used the shared scratch (write, product, row gather)
+  hipStream_t last_stream = nullptr;  // stream of the last call that is ordered with the others (order_scratch_use)
   bool has_stream = false;
   hipEvent_t order_ev = nullptr;      // orders such a call on another stream behind it
   uint32_t given_chunk = 0;  // the caller's chunk_size (0: the library's own)
@@ -1132,8 +1132,10 @@ int refuse_under_capture(hipStream_t st, bool may_block, const char* what) {
   return NZ_OK;
 }
 
-// Writes, products and row gathers of one manager share its scratch memory
-// (encode workspace, row accumulators): they are ordered on the device.  When
+// Writes and products of one manager share its scratch memory
+// (encode workspace, row accumulators): they are ordered on the device.  So are row gathers, which need none
+// (a write that follows on another stream may go into the very buffers a gather reads), and reads behind
+// a write that is still running.  When
 // such a call arrives on another stream than the one before it, the new stream
 // is made to wait (an event, no host synchronisation) for what the other has
 // been given so far.  Streams under capture are left alone: what a graph holds
