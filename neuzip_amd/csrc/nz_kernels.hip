@@ -1610,7 +1610,7 @@ __global__ __launch_bounds__(256) void nz_compact_kernel(const NzEncBatch b) {
 // the tensors of which the write has left a record out of the container (it outgrew its buffer, or
 // a chunk gave up waiting) are put together again in a buffer that holds any container, and the read
 // goes by the same mark (NzBatchItem::late).  There is next to never anything to do, so the grid
-// is small, and the marks of all tensors are looked at together: 1.5 to 3 us (64 workgroups that look at one
+// is small, and the marks of all tensors are looked at together: 1.5 to 4 us (64 workgroups that look at one
 // tensor after the other: 4.3).
 __global__ __launch_bounds__(256) void nz_late_kernel(const NzEncBatch b) {
   __shared__ uint64_t red4[4];
