@@ -49,3 +49,29 @@ def test_rows_of_every_length_and_place(rows, dim, chunk, lane, kind, norm, s):
     with pytest.raises(RuntimeError, match="outside the table"):
         be.check()
     be.check()
+
+
+@pytest.mark.parametrize("precision,norm", [(7, 0), (3, 64)])
+def test_captured_lookups_read_the_table(precision, norm):
+    """A lookup of as many rows as the table has chunks can be captured: it reads the table and indexes."""
+    import neuzip_amd
+
+    rows, cols = 4000, 512
+    mgr = neuzip_amd.Manager(precision=precision, normalizer_size=norm)
+    w = (torch.randn(rows, cols, device="cuda") * 0.02).to(torch.bfloat16)
+    h = mgr.write(w)
+    mgr.flush()
+    table = mgr.read(h).clone()
+    assert rows * cols // mgr._be.geometry(h)[0] < 40
+    idx = torch.randint(0, rows, (40,), device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = mgr.gather_rows(h, idx)
+    for k in range(4):
+        idx.copy_(torch.randint(0, rows, (40,), device="cuda"))
+        graph.replay()
+        eager = mgr.gather_rows(h, idx)
+        torch.cuda.synchronize()
+        assert torch.equal(got, table[idx]) and torch.equal(eager, table[idx]), k
+    mgr._be.check()
