@@ -173,7 +173,7 @@ class FusedGemv:
             self._recording.append((handle, inputs if single_row else None))
             return self._plain(handle, inputs, bias)
         hit = self._where.get(handle)
-        if (hit is None or not single_row or inputs.dtype != torch.bfloat16 or not inputs.is_cuda
+        if (hit is None or not single_row or inputs.dtype != torch.bfloat16 or not inputs.is_cuda or inputs.is_inference()
                 or inputs.shape[-1] != hit[0].in_features or torch.is_grad_enabled() and inputs.requires_grad):
             return self._plain(handle, inputs, bias)
         g, k = hit

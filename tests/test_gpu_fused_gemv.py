@@ -685,3 +685,53 @@ def test_damaged_records_leave_the_other_segments_right(m_rows):
         mgr._be.check()
     good = good.cuda()
     assert torch.equal(got[:, good].view(torch.int16), want[:, good].view(torch.int16))
+
+
+@pytest.mark.parametrize("cols", [1024, 1000])
+def test_linears_in_inference_mode(cols):
+    """Tensors made there have no version: their Linears are served one by one, whatever was learned outside."""
+    import neuzip_amd
+
+    mgr = neuzip_amd.Manager()
+    ws = [(torch.randn(64, cols, device="cuda") * 0.02).to(torch.bfloat16) for _ in range(3)]
+    hs = [mgr.write(w) for w in ws]
+    with torch.no_grad():
+        outside = torch.randn(4, cols, device="cuda").to(torch.bfloat16)
+        for _ in range(3):
+            want = [mgr.linear(h, outside) for h in hs]
+        mgr.linear(hs[0], outside)  # leaves results of the others behind
+    with torch.inference_mode():
+        for rows in (4, 1, 16):
+            x = torch.randn(rows, cols, device="cuda").to(torch.bfloat16)
+            for k in range(3):
+                for h, w in zip(hs, ws):
+                    ref, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+                    # rounding to bf16, and fp32 partial sums relative to the sum of magnitudes
+                    assert bool(((mgr.linear(h, x).double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * mag).all())
+                x.add_(1.0)  # nobody can tell
+        assert all(torch.equal(mgr.linear(h, outside), y) for h, y in zip(hs, want))
+    with torch.no_grad():
+        assert all(torch.equal(mgr.linear(h, outside), y) for h, y in zip(hs, want))
+    mgr._be.check()
+
+
+def test_fused_gemv_in_inference_mode():
+    import neuzip_amd
+
+    torch.manual_seed(12)
+    model = torch.nn.Sequential(_Attn(512), _Attn(512)).to(torch.bfloat16)
+    for p in model.parameters():
+        p.data.normal_(0, 0.05)
+    mgr = neuzip_amd.Manager()
+    mgr.convert(model)
+    model = model.cuda()
+    x = torch.randn(1, 1, 512, device="cuda").to(torch.bfloat16)
+    fused = neuzip_amd.FusedGemv(mgr, model)
+    with torch.no_grad():
+        fused.trace(lambda: model(x))
+        with fused:
+            want = model(x)
+    with torch.inference_mode(), fused:
+        assert torch.equal(model(x), want)  # sums in fixed point: the same one by one as in groups
+        assert torch.equal(model(x.clone()), want)
+    mgr._be.check()
